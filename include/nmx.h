@@ -98,10 +98,12 @@ int nmx_synchronize(nmx_ctx *ctx);
  * plus library knobs
  * prefixed nmx_ (nmx_path:
  * plain|batched|perelement, nmx_graph: yes|no, nmx_graph_steps, nmx_geometry:
- * stored|analytic, nmx_block: full|half|quarter, nmx_xcd: yes|no,
- * nmx_autotune: yes|no, nmx_batch: legacy|buckets|persistent (the batched
- * path's launch shape; the autotuner times the three unless it is set),
- * nmx_stream_hints: 0..7 (streaming cache hints of the stage epilogue)). */
+ * stored|analytic, nmx_xcd: yes|no,
+ * nmx_autotune: yes|no, nmx_batch: buckets|persistent (the batched path's DG
+ * launches per stage: one per order, side by side, or one over all orders;
+ * the autotuner times both unless it is set; legacy is another name of
+ * buckets); accepted without effect: nmx_block (full|half|quarter) and
+ * nmx_stream_hints (0..7)). */
 int nmx_set_param(nmx_ctx *ctx, const char *name, const char *value);
 int nmx_get_param(nmx_ctx *ctx, const char *name, char *buf, int buflen);
 

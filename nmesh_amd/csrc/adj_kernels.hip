@@ -60,6 +60,7 @@ __global__ __launch_bounds__(NT, 2) void dg_adjoint_kernel(AdjArgs a) {
   __shared__ double s_D[NP2];
 
   const int tid = threadIdx.x;
+  const StageRegs o = {a.lam, a.U, a.Wa, a.Wb, a.cA, a.cW, a.wmode};
   for (int q = tid; q < NP2; q += NT) s_D[q] = a.D[q];
 
   int e_hi, e_step, e_first;
@@ -222,24 +223,22 @@ __global__ __launch_bounds__(NT, 2) void dg_adjoint_kernel(AdjArgs a) {
           for (int v = 0; v < 4; ++v) y[c][v] += s_f[v][f][q] - scale * F[v];
         }
       }
-      const double yv[5] = {y[c][0] + a.lam[gi + 4 * NP3], y[c][1], y[c][2], y[c][3], 0.0};
+      const double yv[5] = {y[c][0] + a.phi[gi + 4 * NP3], y[c][1], y[c][2], y[c][3], 0.0};
       if (a.R) {
 #pragma unroll
         for (int v = 0; v < 5; ++v) a.R[gi + v * NP3] = yv[v];
       }
-      if (a.Aout) {
-        double Ab[5];
+      if (a.wmode >= 3) {
+        StageIn q;
+        double out[5];
+        stage_in(o, gi, NP3, q);
+        stage_out<false>(o, q, lam[c], yv, out);
 #pragma unroll
-        for (int v = 0; v < 5; ++v) Ab[v] = a.Abase[gi + v * NP3];
+        for (int v = 0; v < 4; ++v) a.Wout[gi + v * NP3] = out[v];
+      } else if (a.wmode == 1) {
+        const double Ub[5] = {a.U[gi], a.U[gi + NP3], a.U[gi + 2 * NP3], a.U[gi + 3 * NP3], a.U[gi + 4 * NP3]};
 #pragma unroll
-        for (int v = 0; v < 5; ++v) a.Aout[gi + v * NP3] = Ab[v] + a.cA * yv[v];
-      }
-      if (a.Wout) {
-        double Wb[5];
-#pragma unroll
-        for (int v = 0; v < 5; ++v) Wb[v] = a.Wbase[gi + v * NP3];
-#pragma unroll
-        for (int v = 0; v < 5; ++v) a.Wout[gi + v * NP3] = a.cU * Wb[v] + a.cW * yv[v];
+        for (int v = 0; v < 5; ++v) a.Wout[gi + v * NP3] = Ub[v] + a.cW * yv[v];
       }
     }
   }

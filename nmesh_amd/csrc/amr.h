@@ -38,72 +38,17 @@ struct SlotRec {
   int fs1[6], fs2[6];   // kind 1: neighbour node = base + a*fs1 + b*fs2
   int dom;              // CubedShell patch direction and sign
   int n;                // points per direction
-  int jfirst, jcount;   // batched DG path: the element's interpolation jobs
-  int pad[6];
+  int pad[8];
 };
 static_assert(sizeof(SlotRec) == 256, "SlotRec is 256 bytes");
 
-// One (interpolated face, neighbour) job of the batched DG path, done by the
-// receiving element's workgroup in its load phase.  An element's jobs are
-// grouped in rounds; a round holds whole faces, its lines (4 m per job, one
-// thread each) fit the workgroup and its first-pass results and rows fit the
-// stage buffer of the own fields, which is free until those are written.
-struct RJob {
-  long nbase;           // the neighbour's first state double + the plane's base node
-  int t1, t2;           // neighbour plane node = base + q1*t1 + q2*t2
-  int pk;               // m | f << 4 | sw << 7 | a0 << 8 | a1 << 12 | b0 << 16 | b1 << 20
-                        // | (first job of its face) << 24
-  int offA, offB;       // rows (m doubles each) for my a and my b points in Btab
-  int line0;            // first of this job's 4 m lines in its round
-  int toff, r1off, r2off;   // first-pass results, pass-1 and pass-2 rows in the buffer
-  int nround;           // jobs in the round that starts here (0 inside a round)
-};
-static_assert(sizeof(RJob) == 48, "RJob is 48 bytes");
-constexpr int kBatchLines = 256;      // lines per round
-constexpr int kBatchRows = 1024;      // row values (both passes) per round
-constexpr int kBatchScratch = 4000;   // the own-field buffer at n = 10, in doubles
 constexpr int kBatchMaxN = 10;
-// doubles a round of an element of order n may use: the own-field buffer,
-// at least enough for one face of 4 neighbours of up to 10 points
-__host__ __device__ constexpr int batch_scratch(int n) {
-  return 4 * n * n * n > 240 * n ? (4 * n * n * n < kBatchScratch ? 4 * n * n * n : kBatchScratch) : 240 * n;
-}
-
-// One launch per RK stage for every DG element of a batched mesh: items are
-// elements in 8 lists (one per XCD, contiguous in element order, by
-// decreasing n inside); workgroup q of XCD x takes items lo[x] + q, + g8, ...
-struct BatchArgs {
-  const double *win = nullptr, *U = nullptr, *Ain = nullptr;
-  double *Aout = nullptr, *Wout = nullptr, *R = nullptr;
-  const SlotRec *rec = nullptr;
-  const RJob *jobs = nullptr;
-  const double *Btab = nullptr;
-  const double *dXdx = nullptr;   // element blocks of 9*np
-  const double *xyz = nullptr;    // element blocks of 3*np
-  const double *Dall = nullptr;   // D of order n at batch_doff(n)
-  const double *xball = nullptr;  // LGL nodes of order n at batch_xoff(n)
-  const double *wend_inv = nullptr;   // [n]: 1 / (end weight of the LGL quadrature)
-  const int *xlo = nullptr;       // [9]: items of XCD x in [xlo[x], xlo[x + 1])
-  const double *tdev = nullptr;
-  int tidx = 0;
-  double cA = 0, cW = 0;
-  double k[3] = {0, 0, 0};
-  double om = 0;
-  int wmode = 0, numflux = 0, profile = 0;
-  int nt = 0;                     // streaming hints of the epilogue (NodeOut::nt)
-};
 // offsets of order n (2 <= n <= 10) in the concatenated D and node tables
 __host__ __device__ constexpr int batch_doff(int n) { return (n - 1) * n * (2 * n - 1) / 6 - 1; }
 __host__ __device__ constexpr int batch_xoff(int n) { return n * (n - 1) / 2 - 1; }
-// grid: a multiple of 8 (XCD lists)
-hipError_t launch_dg_batch(int geom, const BatchArgs &a, int grid, hipStream_t s);
-// one order: items [a.xlo[0], a.xlo[1]); tile 1 or 2: nodes per thread, 3
-// or 4: 1 or 2 nodes per thread with the epilogue's operands requested at
-// each element's start; grid a multiple of 8
-hipError_t launch_dg_bucket(int np, int geom, const BatchArgs &a, int grid, int tile, hipStream_t s);
 
 struct AmrArgs {
-  const double *win = nullptr, *U = nullptr, *Ain = nullptr;
+  const double *win = nullptr, *U = nullptr, *Wa = nullptr, *Wb = nullptr, *Ain = nullptr;
   double *Aout = nullptr, *Wout = nullptr, *R = nullptr;
   const SlotRec *rec = nullptr;   // this bucket's elements
   int nlist = 0;
@@ -113,13 +58,15 @@ struct AmrArgs {
   const double *xyz = nullptr;    // element blocks of 3*np
   const double *D = nullptr;      // this bucket's D[i*n + l]
   const double *xb = nullptr;     // this bucket's LGL nodes
+  // launches over several orders: D and nodes of order n at batch_doff(n) and
+  // batch_xoff(n), 1 / (end weight) at [n]
+  const double *Dall = nullptr, *xball = nullptr, *wall = nullptr;
   const double *tdev = nullptr;
   int tidx = 0;
   double cA = 0, cW = 0, wend_inv = 0;
   double k[3] = {0, 0, 0};
   double om = 0;
   int wmode = 0, numflux = 0, profile = 0, xcd_map = 0;
-  int nt = 0;                     // streaming hints of the epilogue (NodeOut::nt)
   int fv_mid = 0;                 // FV buckets: metric and normal at the midpoints
   // FV buckets: fv_divf_extrap_s1, _s2, _opt (ex_on: s1 > 0 or s2 < DBL_MAX)
   double ex_s1 = 0, ex_s2 = 1.7976931348623157e308;
@@ -188,10 +135,11 @@ struct AdjJob {
 static_assert(sizeof(AdjJob) == 80, "AdjJob is 80 bytes");
 
 struct AdjAmrArgs {
-  const double *lam = nullptr;
-  const double *Abase = nullptr, *Wbase = nullptr;
-  double *Aout = nullptr, *Wout = nullptr, *R = nullptr;
-  double cA = 0, cU = 0, cW = 0;
+  const double *lam = nullptr, *phi = nullptr;   // as AdjArgs
+  const double *U = nullptr, *Wa = nullptr, *Wb = nullptr;
+  double *Wout = nullptr, *R = nullptr;
+  double cA = 0, cW = 0;
+  int wmode = 0;
   const int *list = nullptr;      // this launch's elements
   int nlist = 0;
   const long *eoff = nullptr;     // [e]: first node
@@ -222,8 +170,17 @@ hipError_t launch_adj_jobs(const AdjAmrArgs &a, hipStream_t s);
 // the transposed RHS and adjoint stage combination of one order bucket
 hipError_t launch_dg_adjoint_amr(int np, int geom, const AdjAmrArgs &a, int grid, hipStream_t s);
 
-// div: nodes per thread (1, 2 or 4)
-hipError_t launch_dg_amr(int np, int geom, const AmrArgs &a, int grid, int div, hipStream_t s);
+// the DG stage kernels (dg_stage.h) over a.nlist elements of order np, or of
+// any order up to nmax (np = 0); geom 0 Cartesian, 1 stored dX/dx, 2
+// CubedShell recomputed
+hipError_t launch_dg_box(int np, int nmax, const AmrArgs &a, hipStream_t s);
+hipError_t launch_dg_stored(int np, int nmax, const AmrArgs &a, hipStream_t s);
+hipError_t launch_dg_shell(int np, int nmax, const AmrArgs &a, hipStream_t s);
+inline hipError_t launch_dg(int np, int nmax, int geom, const AmrArgs &a, hipStream_t s) {
+  return geom == 0   ? launch_dg_box(np, nmax, a, s)
+         : geom == 1 ? launch_dg_stored(np, nmax, a, s)
+                     : launch_dg_shell(np, nmax, a, s);
+}
 hipError_t launch_face_interp(const FaceArgs &a, hipStream_t s);
 hipError_t launch_filter(int np, int geom, const FilterArgs &a, hipStream_t s);
 // an FV order bucket (fv_divf on uniform points): rec 5 = WENOm5_2, 7 =

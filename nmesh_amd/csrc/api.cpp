@@ -79,19 +79,12 @@ struct nmx_ctx {
   int filt_jpow = 0;
   bool filt_on = false;
   double *dBtab = nullptr, *dDall = nullptr, *dxball = nullptr, *daj = nullptr;
-  // persistent batched DG path: every DG element as an item in 8 XCD lists,
-  // the items' interpolation jobs, D and nodes of every order
+  // every DG element by decreasing order, for launches over all orders; D,
+  // nodes and 1 / (end weight) of every order
   SlotRec *dbrec = nullptr;
-  RJob *drjobs = nullptr;
   double *dbD = nullptr, *dbxb = nullptr, *dbW = nullptr;
-  int *dbxlo = nullptr;
-  // the order-per-launch shape: records by decreasing n, each order's range,
-  // element count and tuned tile (nodes per thread, 0: the nmx_block parameter)
-  SlotRec *dbrec2 = nullptr;
-  int *dbnr = nullptr;
-  std::vector<int> bcount, bdiv;
+  int ndg = 0, nmaxdg = 0;   // DG elements, their largest order
   int ncu = 0;
-  int bgrid = 0;          // workgroups of the persistent launch
   bool anydg = false;     // the batched mesh has DG elements
   // troubled elements: TROUBLE values, scores, the mesh score (device),
   // the scores kept across a re-mirror, the per-element FV flags, a
@@ -102,17 +95,14 @@ struct nmx_ctx {
   void *trouble_user = nullptr;
   long trouble_redos = 0, trouble_switches = 0;
   bool batch_fixed = false;   // nmx_batch set by the caller (the autotuner leaves it)
-  // div: nodes per thread of this bucket's tile (0: the nmx_block parameter)
-  // f1first/f1count: the face interpolation jobs of its elements in djobs1
   struct Bucket {
-    int n; int count; SlotRec *drec; long doff; long xoff; int div;
-    int f1first, f1count;
-    float ms;   // tuned stage time alone (0: not tuned) of the shape in use
-    float ms_legacy, ms_order;   // ... with the face kernel, and in the order's own launch
+    int n; int count; SlotRec *drec; long doff; long xoff;
+    float ms;   // tuned stage time alone (0: not tuned)
     int fv;     // 1: FV elements on uniform points (fv_divf)
     long woff;  // FV: the bucket's midpoint distances in dwcall
   };
   std::vector<Bucket> buckets;
+  int nfacejobs = 0;                   // interpolation jobs in djobs1
   std::vector<long> eoff;   // node offset per element
   // graph cache
   hipGraph_t graph = nullptr;
@@ -376,8 +366,7 @@ static void free_mesh_dev(nmx_ctx *c) {
   {
     void **ptrs[] = {(void **)&c->djobs1, (void **)&c->dmdesc, (void **)&c->dFilt, (void **)&c->dfrec,
                      (void **)&c->dBtab, (void **)&c->dDall, (void **)&c->dxball, (void **)&c->daj,
-                     (void **)&c->dbrec, (void **)&c->drjobs, (void **)&c->dbD, (void **)&c->dbxb,
-                     (void **)&c->dbW, (void **)&c->dbxlo, (void **)&c->dbrec2, (void **)&c->dbnr,
+                     (void **)&c->dbrec, (void **)&c->dbD, (void **)&c->dbxb, (void **)&c->dbW,
                      (void **)&c->dtr, (void **)&c->dscore, (void **)&c->dtrout, (void **)&c->defv};
     for (auto q : ptrs)
       if (*q) { (void)hipFree(*q); *q = nullptr; }
@@ -531,8 +520,6 @@ extern "C" int nmx_set_param(nmx_ctx *c, const char *name, const char *value) {
   c->par[k] = v;
   if (k == "nmx_block" || k == "nmx_xcd") c->tuned = true;   // explicit choice wins
   if (k == "nmx_batch") c->batch_fixed = true;
-  if (k == "nmx_block")
-    for (auto &b : c->buckets) b.div = 0;
   drop_stage_graphs(c);
   if (c->gexec) { (void)hipGraphExecDestroy(c->gexec); c->gexec = nullptr; }
   if (c->graph) { (void)hipGraphDestroy(c->graph); c->graph = nullptr; }
@@ -651,104 +638,17 @@ static std::vector<double> fv_cell_widths(int n) {
   return wc;
 }
 
-// Tables of the persistent batched DG launch.  Items: the DG elements in 8
-// lists, one per XCD, each a contiguous range of the element order holding
-// about an eighth of the work, with decreasing n inside (stable), so a
-// workgroup walks its elements order by order.  Each item's interpolation
-// jobs are split into rounds of whole faces whose lines fit the workgroup and
-// whose rows and first-pass results fit the own-field buffer.
-static int upload_batch_tables(nmx_ctx *c, const std::vector<int> &fd,
-                               std::vector<std::vector<RJob>> &erj) {
-  const Mesh &M = c->mesh;
-  const size_t ne = M.e.size();
-  std::vector<int> dg;
-  for (size_t i = 0; i < ne; ++i)
-    if (!M.e[i].fv) dg.push_back((int)i);
-  c->anydg = !dg.empty();
-  if (dg.empty()) return NMX_OK;
-  auto cost = [&](int e) {
-    const double n = M.e[e].n;
-    return n * n * n + 0.25 * (double)erj[e].size() * n * n * n / 2.;
-  };
-  double total = 0;
-  for (int e : dg) total += cost(e);
-  std::vector<int> items, xlo(9, 0);
-  items.reserve(dg.size());
-  size_t k = 0;
-  double acc = 0;
-  for (int x = 0; x < 8; ++x) {
-    xlo[x] = (int)items.size();
-    const size_t k0 = k;
-    while (k < dg.size() && (x == 7 || acc + 0.5 * cost(dg[k]) <= total * (x + 1) / 8.)) acc += cost(dg[k++]);
-    std::vector<int> part(dg.begin() + k0, dg.begin() + k);
-    std::stable_sort(part.begin(), part.end(), [&](int a, int b) { return M.e[a].n > M.e[b].n; });
-    items.insert(items.end(), part.begin(), part.end());
-  }
-  xlo[8] = (int)items.size();
-  std::vector<SlotRec> recs(items.size());
-  std::vector<RJob> jobs;
-  for (size_t it = 0; it < items.size(); ++it) {
-    const int e = items[it];
-    const int n = M.e[e].n;
-    if (n < 2 || n > kBatchMaxN) return fail(NMX_EUNSUP, "batched DG elements need 2 to 10 points per direction");
-    SlotRec &R = recs[it];
-    slot_geometry(M, e, R);
-    for (int f = 0; f < 6; ++f) {
-      const int *d = &fd[48 * e + 8 * f];
-      R.fkind[f] = d[0];
-      if (d[0] == 1) {
-        R.foff[f] = 5 * M.e[d[1]].off + d[2];
-        R.fs1[f] = d[3];
-        R.fs2[f] = d[4];
-      }
-    }
-    R.jfirst = (int)jobs.size();
-    R.jcount = (int)erj[e].size();
-    // rounds of whole faces
-    std::vector<RJob> &J = erj[e];
-    const int cap = batch_scratch(n);
-    size_t j = 0;
-    while (j < J.size()) {
-      const size_t r0 = j;
-      int lines = 0, scr = 0, rows = 0;
-      while (j < J.size()) {
-        size_t je = j + 1;
-        while (je < J.size() && !((J[je].pk >> 24) & 1)) ++je;
-        int fl = 0, fs = 0, fr = 0;
-        for (size_t q = j; q < je; ++q) {
-          const int m = J[q].pk & 15, sw = (J[q].pk >> 7) & 1;
-          const int a0 = (J[q].pk >> 8) & 15, a1 = (J[q].pk >> 12) & 15;
-          const int b0 = (J[q].pk >> 16) & 15, b1 = (J[q].pk >> 20) & 15;
-          const int nx1 = (sw ? b1 - b0 : a1 - a0) + 1, nx2 = (sw ? a1 - a0 : b1 - b0) + 1;
-          fl += 4 * m;
-          fs += 4 * nx1 * m + nx1 * m + nx2 * m;
-          fr += nx1 * m + nx2 * m;
-        }
-        if (fl > kBatchLines || fs > cap || fr > kBatchRows)
-          return fail(NMX_EUNSUP, "face too large for one round");
-        if (j > r0 && (lines + fl > kBatchLines || scr + fs > cap || rows + fr > kBatchRows)) break;
-        rows += fr;
-        for (size_t q = j; q < je; ++q) {
-          const int m = J[q].pk & 15, sw = (J[q].pk >> 7) & 1;
-          const int a0 = (J[q].pk >> 8) & 15, a1 = (J[q].pk >> 12) & 15;
-          const int b0 = (J[q].pk >> 16) & 15, b1 = (J[q].pk >> 20) & 15;
-          const int nx1 = (sw ? b1 - b0 : a1 - a0) + 1, nx2 = (sw ? a1 - a0 : b1 - b0) + 1;
-          if (a1 >= n || b1 >= n) return fail(NMX_EINVAL, "interpolation coverage out of range");
-          J[q].line0 = lines;
-          J[q].toff = scr;
-          J[q].r1off = scr + 4 * nx1 * m;
-          J[q].r2off = J[q].r1off + nx1 * m;
-          J[q].nround = 0;
-          lines += 4 * m;
-          scr += 4 * nx1 * m + nx1 * m + nx2 * m;
-        }
-        j = je;
-      }
-      J[r0].nround = (int)(j - r0);
-    }
-    jobs.insert(jobs.end(), J.begin(), J.end());
-  }
-  if (jobs.empty()) jobs.resize(1);
+// The DG elements' records (in recs, element order) for launches over all
+// orders, by decreasing order, and D, nodes and end weights of every order.
+static int upload_order_tables(nmx_ctx *c, std::vector<SlotRec> &recs) {
+  c->ndg = (int)recs.size();
+  c->anydg = !recs.empty();
+  c->nmaxdg = 0;
+  if (recs.empty()) return NMX_OK;
+  std::stable_sort(recs.begin(), recs.end(), [](const SlotRec &x, const SlotRec &y) { return x.n > y.n; });
+  if (recs.back().n < 2 || recs[0].n > kBatchMaxN)
+    return fail(NMX_EUNSUP, "batched DG elements need 2 to 10 points per direction");
+  c->nmaxdg = recs[0].n;
   std::vector<double> D, xb, wi(kBatchMaxN + 1, 0.0);
   for (int n = 2; n <= kBatchMaxN; ++n) {
     const Basis &b = lgl_basis(n);
@@ -758,41 +658,18 @@ static int upload_batch_tables(nmx_ctx *c, const std::vector<int> &fd,
     xb.insert(xb.end(), b.x, b.x + n);
     wi[n] = 1.0 / b.w[0];
   }
-  // the order-per-launch shape: the same records by decreasing n, element
-  // order inside; order n holds [nrange[2n], nrange[2n + 1])
-  std::vector<int> perm(items.size());
-  for (size_t i = 0; i < perm.size(); ++i) perm[i] = (int)i;
-  std::stable_sort(perm.begin(), perm.end(), [&](int x, int y) {
-    if (recs[x].n != recs[y].n) return recs[x].n > recs[y].n;
-    return items[x] < items[y];
-  });
-  std::vector<SlotRec> recs2(perm.size());
-  std::vector<int> nrange(2 * (kBatchMaxN + 1), 0);
-  for (size_t i = 0; i < perm.size(); ++i) recs2[i] = recs[perm[i]];
-  for (size_t i = 0; i < recs2.size(); ++i) {
-    const int n = recs2[i].n;
-    if (i == 0 || recs2[i - 1].n != n) nrange[2 * n] = (int)i;
-    nrange[2 * n + 1] = (int)i + 1;
-  }
-  c->bcount.assign(kBatchMaxN + 1, 0);
-  for (int n = 2; n <= kBatchMaxN; ++n) c->bcount[n] = nrange[2 * n + 1] - nrange[2 * n];
-  c->bdiv.assign(kBatchMaxN + 1, 0);
   hipDeviceProp_t prop;
   HIPCHK(hipGetDeviceProperties(&prop, c->device));
   c->ncu = prop.multiProcessorCount;
-  c->bgrid = 8 * ((3 * prop.multiProcessorCount + 7) / 8);
   int r;
-  if ((r = dev_upload(&c->dbrec, recs)) || (r = dev_upload(&c->drjobs, jobs)) || (r = dev_upload(&c->dbD, D)) ||
-      (r = dev_upload(&c->dbxb, xb)) || (r = dev_upload(&c->dbW, wi)) || (r = dev_upload(&c->dbxlo, xlo)) ||
-      (r = dev_upload(&c->dbrec2, recs2)) || (r = dev_upload(&c->dbnr, nrange)))
+  if ((r = dev_upload(&c->dbrec, recs)) || (r = dev_upload(&c->dbD, D)) || (r = dev_upload(&c->dbxb, xb)) ||
+      (r = dev_upload(&c->dbW, wi)))
     return r;
   return NMX_OK;
 }
 
 // Tables of the batched path: face descriptors, face interpolation jobs
-// (single-neighbour faces and faces with several neighbours in separate
-// lists, each grouped by the receiving element's order bucket) with
-// deduplicated 1D Lagrange rows, order buckets with one SlotRec per element.
+// (grouped by the element whose plane they read) with deduplicated 1D Lagrange rows, order buckets with one SlotRec per element.
 // Every gather a kernel will make is bounds-checked here.
 static int upload_amr_tables(nmx_ctx *c) {
   Mesh &M = c->mesh;
@@ -800,10 +677,10 @@ static int upload_amr_tables(nmx_ctx *c) {
   std::vector<long> soff(ne);
   for (size_t i = 0; i < ne; ++i) soff[i] = 5 * M.e[i].off;
   std::vector<int> fd(48 * ne, 0);
-  // jobs of each element's interpolated faces, one per (face, neighbour),
-  // in the face kernel's form (ej1) and the persistent DG kernel's (erj)
+  // the jobs that read each element's face planes, one per (interpolated
+  // face, neighbour): side by side, they find the plane's lines in L2 (a
+  // plane normal to x touches every line of the element)
   std::vector<std::vector<int>> ej1(ne);
-  std::vector<std::vector<RJob>> erj(ne);
   std::vector<int> mdesc;
   std::vector<double> btab;
   std::map<std::vector<double>, int> bdedup;
@@ -880,15 +757,7 @@ static int upload_amr_tables(nmx_ctx *c) {
                              q.a0, q.a1, q.b0, q.b1, oa, ob, 0, 0};
         const long so = soff[q.nb];
         std::memcpy(rec + 14, &so, sizeof(long));
-        ej1[i].insert(ej1[i].end(), rec, rec + kJobInts);
-        RJob rj;
-        std::memset(&rj, 0, sizeof rj);
-        rj.nbase = so + base;
-        rj.t1 = q.t1; rj.t2 = q.t2;
-        rj.pk = m | (f << 4) | (q.swap << 7) | (q.a0 << 8) | (q.a1 << 12) | (q.b0 << 16) | (q.b1 << 20) |
-                ((si == 0 ? 1 : 0) << 24);
-        rj.offA = oa; rj.offB = ob;
-        erj[i].push_back(rj);
+        ej1[q.nb].insert(ej1[q.nb].end(), rec, rec + kJobInts);
         if (ns > 1) {
           const int md[5] = {(int)region, q.a0, q.a1, q.b0, q.b1};
           mdesc.insert(mdesc.end(), md, md + 5);
@@ -940,7 +809,7 @@ static int upload_amr_tables(nmx_ctx *c) {
   if ((r = dev_upload(&c->dBtab, btab)) || (r = dev_alloc(&c->daj, ajlen)) ||
       (r = dev_upload(&c->dmdesc, mdesc)))
     return r;
-  std::vector<int> jobs1;
+  std::vector<SlotRec> dgrecs;
   // order buckets with their D matrices and nodes
   std::vector<double> dall, xball, wcall;
   for (int n = 2; n <= 10; ++n)
@@ -953,8 +822,7 @@ static int upload_amr_tables(nmx_ctx *c) {
     b.n = n;
     b.count = (int)list.size();
     b.drec = nullptr;
-    b.div = fv ? 1 : 0;
-    b.ms = b.ms_legacy = b.ms_order = 0.f;
+    b.ms = 0.f;
     b.fv = fv;
     b.woff = 0;
     if (fv) {
@@ -979,10 +847,7 @@ static int upload_amr_tables(nmx_ctx *c) {
         }
       }
     }
-    // the face jobs of this bucket's elements, in element order
-    b.f1first = (int)(jobs1.size() / kJobInts);
-    for (int e : list) jobs1.insert(jobs1.end(), ej1[e].begin(), ej1[e].end());
-    b.f1count = (int)(jobs1.size() / kJobInts) - b.f1first;
+    if (!fv) dgrecs.insert(dgrecs.end(), recs.begin(), recs.end());
     c->buckets.push_back(b);
     if ((r = dev_upload(&c->buckets.back().drec, recs))) return r;
     const Basis &bs = lgl_basis(n);
@@ -997,9 +862,12 @@ static int upload_amr_tables(nmx_ctx *c) {
       (r = dev_upload(&c->dwcall, wcall)))
     return r;
   assign_lanes(c);
+  std::vector<int> jobs1;
+  for (const auto &ej : ej1) jobs1.insert(jobs1.end(), ej.begin(), ej.end());
+  c->nfacejobs = (int)(jobs1.size() / kJobInts);
   if (jobs1.empty()) jobs1.assign(kJobInts, 0);
   if ((r = dev_upload(&c->djobs1, jobs1))) return r;
-  return upload_batch_tables(c, fd, erj);
+  return upload_order_tables(c, dgrecs);
 }
 
 // host -> device mirror of the mesh (element-block layout)
@@ -1097,12 +965,6 @@ static int upload_mesh(nmx_ctx *c) {
     if ((r = dev_upload(&c->dwc, fv_cell_widths(c->np1)))) return r;
   }
   if (c->amr) return upload_amr_tables(c);
-  {
-    // every element, for the filter
-    std::vector<SlotRec> fr(ne);
-    for (size_t i = 0; i < ne; ++i) slot_geometry(M, (int)i, fr[i]);
-    if ((r = dev_upload(&c->dfrec, fr))) return r;
-  }
   // face gather descriptors {nb, local base, s1, s2}
   std::vector<int4> hf(6 * ne);
   for (size_t i = 0; i < ne; ++i)
@@ -1128,6 +990,23 @@ static int upload_mesh(nmx_ctx *c) {
       }
       hf[6 * i + f] = d;
     }
+  {
+    // every element, for the stage kernel and the filter
+    std::vector<SlotRec> fr(ne);
+    const long np3 = (long)c->np1 * c->np1 * c->np1;
+    for (size_t i = 0; i < ne; ++i) {
+      slot_geometry(M, (int)i, fr[i]);
+      for (int f = 0; f < 6; ++f) {
+        const int4 &d = hf[6 * i + f];
+        fr[i].fkind[f] = d.x >= 0 ? 1 : 0;
+        if (d.x < 0) continue;
+        fr[i].foff[f] = 5 * np3 * d.x + d.y;
+        fr[i].fs1[f] = d.z;
+        fr[i].fs2[f] = d.w;
+      }
+    }
+    if ((r = dev_upload(&c->dfrec, fr))) return r;
+  }
   if ((r = dev_alloc(&c->dface, hf.size()))) return r;
   HIPCHK(hipMemcpy(c->dface, hf.data(), hf.size() * sizeof(int4), hipMemcpyHostToDevice));
   // the neighbour's face on each conforming face (adjoint gathers)
@@ -1774,7 +1653,6 @@ static StageArgs base_args(nmx_ctx *c) {
   a.om = std::sqrt(a.k[0] * a.k[0] + a.k[1] * a.k[1] + a.k[2] * a.k[2]);
   a.profile = (a.k[0] != 0 || a.k[1] != 0 || a.k[2] != 0);
   a.numflux = (P(c, "scalarwave1_numflux") == "LLF") ? 1 : 0;
-  a.nt = Pi(c, "nmx_stream_hints") & 7;
   a.e0 = 0;
   a.e1 = (int)c->mesh.e.size();
   return a;
@@ -1782,173 +1660,101 @@ static StageArgs base_args(nmx_ctx *c) {
 
 static AmrArgs amr_args(nmx_ctx *c, const StageArgs &sa) {
   AmrArgs a;
-  a.win = sa.win; a.U = sa.U; a.Ain = sa.Ain; a.Aout = sa.Aout; a.Wout = sa.Wout; a.R = sa.R;
+  a.win = sa.win; a.U = sa.U; a.Wa = sa.Wa; a.Wb = sa.Wb; a.Ain = sa.Ain; a.Aout = sa.Aout; a.Wout = sa.Wout; a.R = sa.R;
   a.aj = c->daj;
   a.mdesc = c->dmdesc;
   a.dXdx = c->dXdx; a.xyz = c->dxyz; a.tdev = sa.tdev; a.tidx = sa.tidx;
   a.cA = sa.cA; a.cW = sa.cW;
   for (int d = 0; d < 3; ++d) a.k[d] = sa.k[d];
-  a.om = sa.om; a.wmode = sa.wmode; a.numflux = sa.numflux; a.profile = sa.profile; a.nt = sa.nt;
+  a.om = sa.om; a.wmode = sa.wmode; a.numflux = sa.numflux; a.profile = sa.profile;
   return a;
 }
 
-// one order bucket's stage kernel with tile div (1, 2 or 4 nodes per thread)
-static int launch_bucket(nmx_ctx *c, AmrArgs a, const nmx_ctx::Bucket &b, int div, int xcd_map,
-                         hipStream_t st) {
+// one order bucket's stage kernel
+static int launch_bucket(nmx_ctx *c, AmrArgs a, const nmx_ctx::Bucket &b, int xcd_map, hipStream_t st) {
   a.D = c->dDall + b.doff;
   a.xb = c->dxball + b.xoff;
   a.wend_inv = 1.0 / lgl_basis(b.n).w[0];
   a.rec = b.drec;
   a.nlist = b.count;
   a.xcd_map = xcd_map;
-  int grid = a.xcd_map ? 8 * ((b.count + 7) / 8) : b.count;
   hipError_t err;
   if (b.fv) {
+    const int grid = a.xcd_map ? 8 * ((b.count + 7) / 8) : b.count;
     const int rec = fv_rec_pars(c, a.recend, a.rec_s1, a.rec_s2, a.rec_opt, a.rec_on);
     a.rec_first = P(c, "fv_rec") == "1";
     a.fv_mid = P(c, "coordinates_midpoint_data") != "no";
     fv_extrap_pars(c, a.ex_s1, a.ex_s2, a.ex_opt, a.ex_on);
     err = launch_fvelm_amr(b.n, rec, c->geom == 0 ? 0 : 2, a, c->dwcall + b.woff, grid, st);
   } else {
-    err = launch_dg_amr(b.n, c->geom, a, grid, div, st);
+    err = launch_dg(b.n, b.n, c->geom, a, st);
   }
   if (err != hipSuccess) return fail(NMX_EHIP, std::string("stage launch: ") + hipGetErrorString(err));
   return NMX_OK;
 }
 
-static BatchArgs batch_args(nmx_ctx *c, const StageArgs &sa) {
-  BatchArgs b;
-  b.win = sa.win; b.U = sa.U; b.Ain = sa.Ain; b.Aout = sa.Aout; b.Wout = sa.Wout; b.R = sa.R;
-  b.rec = c->dbrec; b.jobs = c->drjobs; b.Btab = c->dBtab;
-  b.dXdx = c->dXdx; b.xyz = c->dxyz; b.Dall = c->dbD; b.xball = c->dbxb;
-  b.tdev = sa.tdev; b.tidx = sa.tidx;
-  b.wend_inv = c->dbW; b.xlo = c->dbxlo;
-  b.cA = sa.cA; b.cW = sa.cW;
-  for (int d = 0; d < 3; ++d) b.k[d] = sa.k[d];
-  b.om = sa.om; b.wmode = sa.wmode; b.numflux = sa.numflux; b.profile = sa.profile; b.nt = sa.nt;
-  return b;
-}
-
-// the persistent launch of every DG element of a batched mesh (one per stage)
-static int launch_batch(nmx_ctx *c, const StageArgs &sa) {
-  hipError_t err = launch_dg_batch(c->geom, batch_args(c, sa), c->bgrid, c->stream);
-  if (err != hipSuccess) return fail(NMX_EHIP, std::string("batch launch: ") + hipGetErrorString(err));
+// every DG element in one launch
+static int launch_mixed(nmx_ctx *c, AmrArgs a, int xcd_map, hipStream_t st) {
+  a.rec = c->dbrec;
+  a.nlist = c->ndg;
+  a.xcd_map = xcd_map;
+  a.Dall = c->dbD;
+  a.xball = c->dbxb;
+  a.wall = c->dbW;
+  hipError_t err = launch_dg(0, c->nmaxdg, c->geom, a, st);
+  if (err != hipSuccess) return fail(NMX_EHIP, std::string("stage launch: ") + hipGetErrorString(err));
   return NMX_OK;
 }
 
-// the DG elements of order n in one launch of the order's own kernel, with
-// tile (launch_dg_bucket)
-static int launch_order(nmx_ctx *c, const StageArgs &sa, int n, int div, hipStream_t st) {
-  BatchArgs b = batch_args(c, sa);
-  b.rec = c->dbrec2;
-  b.xlo = c->dbnr + 2 * n;
-  const int count = c->bcount[n];
-  const int grid = 8 * ((std::min(count, 8 * c->ncu) + 7) / 8);
-  hipError_t err = launch_dg_bucket(n, c->geom, b, grid, div, st);
-  if (err != hipSuccess) return fail(NMX_EHIP, std::string("bucket launch: ") + hipGetErrorString(err));
-  return NMX_OK;
-}
-
+// One stage of the batched path: every interpolated face, then the order
+// buckets side by side on kLanes stream lanes: lane 0 is the context's stream,
+// the others helpers forked from it (parallel branches when captured into a
+// graph); the longest buckets start first, one per lane, the rest queue on the
+// least loaded lane.  With nmx_batch = persistent the DG elements go in one
+// launch on lane 0 and FV buckets beside it.
 static int launch_amr(nmx_ctx *c, const StageArgs &sa) {
   const bool perelm = (P(c, "nmx_path") == "perelement");
+  const bool one = !perelm && P(c, "nmx_batch") == "persistent";
   AmrArgs a = amr_args(c, sa);
-  if (!perelm && P(c, "nmx_batch") == "buckets") {
-    // one launch per order, side by side on the stream lanes (FV buckets
-    // with their face kernel)
-    std::string blk = P(c, "nmx_block");
-    const int div0 = blk == "half" ? 2 : blk == "quarter" ? 4 : 1;
-    const bool fork = c->buckets.size() > 1 && P(c, "nmx_concurrent") == "yes";
-    auto lane_stream = [c](int lane) { return lane == 0 ? c->stream : c->helper[lane - 1]; };
-    if (fork) {
-      HIPCHK(hipEventRecord(c->evfork, c->stream));
-      for (int l = 1; l < nmx_ctx::kLanes; ++l) HIPCHK(hipStreamWaitEvent(lane_stream(l), c->evfork, 0));
-    }
-    for (size_t k = 0; k < c->buckets.size(); ++k) {
-      const int bi = c->border[k];
-      const auto &b = c->buckets[bi];
-      hipStream_t st = fork ? lane_stream(c->blane[bi]) : c->stream;
-      if (b.fv) {
-        FaceArgs fa;
-        fa.win = sa.win; fa.Btab = c->dBtab; fa.aj = c->daj;
-        fa.jobs = c->djobs1 + (long)kJobInts * b.f1first; fa.nfaces = b.f1count;
-        hipError_t err = launch_face_interp(fa, st);
-        if (err != hipSuccess) return fail(NMX_EHIP, std::string("face launch: ") + hipGetErrorString(err));
-        if (int r = launch_bucket(c, a, b, 1, sa.xcd_map, st)) return r;
-      } else {
-        const int tile = c->bdiv[b.n] ? c->bdiv[b.n] : (div0 >= 2 ? 2 : 1);
-        if (int r = launch_order(c, sa, b.n, tile, st)) return r;
-      }
-    }
-    if (fork)
-      for (int l = 1; l < nmx_ctx::kLanes; ++l) {
-        HIPCHK(hipEventRecord(c->evjoin[l - 1], lane_stream(l)));
-        HIPCHK(hipStreamWaitEvent(c->stream, c->evjoin[l - 1], 0));
-      }
-    return NMX_OK;
-  }
-  if (!perelm && P(c, "nmx_batch") == "persistent") {
-    // FV buckets (faces from the face kernel), then every DG element at once
-    std::string blk = P(c, "nmx_block");
-    for (size_t k = 0; k < c->buckets.size(); ++k) {
-      const auto &b = c->buckets[c->border[k]];
-      if (!b.fv) continue;
-      FaceArgs fa;
-      fa.win = sa.win; fa.Btab = c->dBtab; fa.aj = c->daj;
-      fa.jobs = c->djobs1 + (long)kJobInts * b.f1first; fa.nfaces = b.f1count;
-      hipError_t err = launch_face_interp(fa, c->stream);
-      if (err != hipSuccess) return fail(NMX_EHIP, std::string("face launch: ") + hipGetErrorString(err));
-      if (int r = launch_bucket(c, a, b, 1, sa.xcd_map, c->stream)) return r;
-    }
-    return c->anydg ? launch_batch(c, sa) : NMX_OK;
-  }
-  std::string blk = P(c, "nmx_block");
-  const int div0 = blk == "half" ? 2 : blk == "quarter" ? 4 : 1;
-  // interpolated faces of one bucket's elements, just before its stage kernel
-  auto faces = [&](const nmx_ctx::Bucket &b, hipStream_t st) -> int {
-    FaceArgs fa;
-    fa.win = sa.win; fa.Btab = c->dBtab; fa.aj = c->daj;
-    fa.jobs = c->djobs1 + (long)kJobInts * b.f1first; fa.nfaces = b.f1count;
-    hipError_t err = launch_face_interp(fa, st);
-    if (err != hipSuccess) return fail(NMX_EHIP, std::string("face launch: ") + hipGetErrorString(err));
-    return NMX_OK;
-  };
-  // buckets run concurrently on kLanes stream lanes: lane 0 is the context's
-  // stream, the others helpers forked from it (parallel branches when
-  // captured into a graph); the longest buckets start first, one per lane,
-  // the rest queue on the least loaded lane.  A bucket's faces read only the
-  // stage input, so each lane computes its own buckets' faces and the face
-  // work overlaps other lanes' buckets.
-  const bool fork = !perelm && c->buckets.size() > 1 && P(c, "nmx_concurrent") == "yes";
-  auto lane_stream = [c](int lane) { return lane == 0 ? c->stream : c->helper[lane - 1]; };
-  if (fork) {
-    HIPCHK(hipEventRecord(c->evfork, c->stream));
-    for (int l = 1; l < nmx_ctx::kLanes; ++l) HIPCHK(hipStreamWaitEvent(lane_stream(l), c->evfork, 0));
-  }
-  for (size_t k = 0; k < c->buckets.size(); ++k) {
-    const int bi = perelm ? (int)k : c->border[k];
-    const auto &b = c->buckets[bi];
-    hipStream_t st = fork ? lane_stream(c->blane[bi]) : c->stream;
-    a.D = c->dDall + b.doff;
-    a.xb = c->dxball + b.xoff;
-    a.wend_inv = 1.0 / lgl_basis(b.n).w[0];
-    const int div = b.div ? b.div : div0;
-    if (int r = faces(b, st)) return r;
-    if (perelm) {
+  FaceArgs fa;
+  fa.win = sa.win; fa.Btab = c->dBtab; fa.aj = c->daj;
+  fa.jobs = c->djobs1; fa.nfaces = c->nfacejobs;
+  hipError_t err = launch_face_interp(fa, c->stream);
+  if (err != hipSuccess) return fail(NMX_EHIP, std::string("face launch: ") + hipGetErrorString(err));
+  if (perelm) {
+    for (const auto &b : c->buckets) {
       if (b.fv) return fail(NMX_EUNSUP, "FV elements run on the plain or batched path");
-      a.xcd_map = 0;
-      a.nlist = 1;
       for (int q = 0; q < b.count; ++q) {
-        a.rec = b.drec + q;
-        hipError_t err = launch_dg_amr(b.n, c->geom, a, 1, div, c->stream);
-        if (err != hipSuccess) return fail(NMX_EHIP, std::string("stage launch: ") + hipGetErrorString(err));
+        nmx_ctx::Bucket b1 = b;
+        b1.drec = b.drec + q;
+        b1.count = 1;
+        if (int r = launch_bucket(c, a, b1, 0, c->stream)) return r;
       }
-      continue;
     }
-    int r = launch_bucket(c, a, b, div, sa.xcd_map, st);
-    if (r) return r;
+    return NMX_OK;
   }
-  if (fork)
-    for (int l = 1; l < nmx_ctx::kLanes; ++l) {
+  // the buckets launched on their own, by decreasing work, and their lanes
+  std::vector<std::pair<int, int>> own;
+  for (size_t k = 0; k < c->buckets.size(); ++k) {
+    const int bi = c->border[k];
+    if (!one) own.push_back({bi, c->blane[bi]});
+    else if (c->buckets[bi].fv)
+      own.push_back({bi, c->anydg ? 1 + (int)own.size() % (nmx_ctx::kLanes - 1) : (int)own.size() % nmx_ctx::kLanes});
+  }
+  if (P(c, "nmx_concurrent") != "yes")
+    for (auto &b : own) b.second = 0;
+  unsigned used = 0;
+  for (const auto &b : own) used |= 1u << b.second;
+  auto lane_stream = [c](int lane) { return lane == 0 ? c->stream : c->helper[lane - 1]; };
+  if (used >> 1) HIPCHK(hipEventRecord(c->evfork, c->stream));
+  for (int l = 1; l < nmx_ctx::kLanes; ++l)
+    if (used >> l & 1) HIPCHK(hipStreamWaitEvent(lane_stream(l), c->evfork, 0));
+  for (const auto &b : own)
+    if (int r = launch_bucket(c, a, c->buckets[b.first], sa.xcd_map, lane_stream(b.second))) return r;
+  if (one && c->anydg)
+    if (int r = launch_mixed(c, a, sa.xcd_map, c->stream)) return r;
+  for (int l = 1; l < nmx_ctx::kLanes; ++l)
+    if (used >> l & 1) {
       HIPCHK(hipEventRecord(c->evjoin[l - 1], lane_stream(l)));
       HIPCHK(hipStreamWaitEvent(c->stream, c->evjoin[l - 1], 0));
     }
@@ -1968,23 +1774,24 @@ static int launch(nmx_ctx *c, StageArgs a) {
     if (err != hipSuccess) return fail(NMX_EHIP, std::string("fv stage launch: ") + hipGetErrorString(err));
     return NMX_OK;
   }
-  bool perelm = (P(c, "nmx_path") == "perelement");
-  std::string blk = P(c, "nmx_block");
-  int nt = dg_stage_threads(c->np1, blk == "half" ? 2 : blk == "quarter" ? 4 : 1);
-  if (perelm) {
-    int ne = a.e1;
-    a.xcd_map = 0;
-    for (int e = 0; e < ne; ++e) {
-      a.e0 = e; a.e1 = e + 1;
-      hipError_t err = launch_dg_stage(c->np1, c->geom, a, 1, nt, c->stream);
-      if (err != hipSuccess) return fail(NMX_EHIP, std::string("stage launch: ") + hipGetErrorString(err));
-    }
-    return NMX_OK;
+  AmrArgs ca = amr_args(c, a);
+  ca.D = c->dD;
+  ca.xb = c->dxb;
+  ca.wend_inv = a.wend_inv;
+  ca.rec = c->dfrec;
+  ca.nlist = (int)c->mesh.e.size();
+  ca.xcd_map = a.xcd_map;
+  int launches = 1;
+  if (P(c, "nmx_path") == "perelement") {
+    launches = ca.nlist;
+    ca.xcd_map = 0;
+    ca.nlist = 1;
   }
-  int nel = a.e1 - a.e0;
-  int grid = a.xcd_map ? 8 * ((nel + 7) / 8) : nel;
-  hipError_t err = launch_dg_stage(c->np1, c->geom, a, grid, nt, c->stream);
-  if (err != hipSuccess) return fail(NMX_EHIP, std::string("stage launch: ") + hipGetErrorString(err));
+  for (int e = 0; e < launches; ++e) {
+    ca.rec = c->dfrec + e;
+    hipError_t err = launch_dg(c->np1, c->np1, c->geom, ca, c->stream);
+    if (err != hipSuccess) return fail(NMX_EHIP, std::string("stage launch: ") + hipGetErrorString(err));
+  }
   return NMX_OK;
 }
 
@@ -2609,40 +2416,60 @@ static int launch_limiter_on(nmx_ctx *c, double *reg) {
   return NMX_OK;
 }
 
+// Whether a step ends in the other of the registers U and A: Euler steps do
+// (the stage's neighbours read U while it writes), and steps with a limiter,
+// which changes the stage inputs, so that the right-hand sides cannot be
+// recovered from them and are accumulated.  The others end in U.
+static bool step_swaps(nmx_ctx *c, int method) { return c->lim_on || method == 2; }
+
 // issue the stage launches of one step; stage times at dT[tbase + s]
 static int issue_step(nmx_ctx *c, int method, double dt, int tbase, bool swap_parity) {
-  double *U = swap_parity ? c->dA : c->dU;
-  double *A = swap_parity ? c->dU : c->dA;
+  const bool swaps = step_swaps(c, method);
+  double *U = swaps && swap_parity ? c->dA : c->dU;
+  double *A = swaps && swap_parity ? c->dU : c->dA;
+  double *end = swaps ? A : U;
   StageArgs a = base_args(c);
   int r;
+  a.U = U;
+  auto stage = [&](int s, double *win, double *wout, int wmode, double cW) {
+    a.win = win; a.Wout = wout; a.wmode = wmode; a.cW = cW; a.tidx = tbase + s;
+    return launch(c, a);
+  };
   // the MRS limiter acts on every later stage's input w (RungeKutta.c:45,
   // 56, 67, 161, 173) and on the final u (evolve.c:143-144)
-  auto lim = [&](double *reg) { return c->lim_on ? launch_limiter_on(c, reg) : NMX_OK; };
-  if (method == 0) {   // evolve_RK4_mesh (RungeKutta.c:19-82)
-    a.win = U; a.U = U; a.Ain = nullptr; a.Aout = A; a.cA = dt / 6.; a.Wout = c->dW0; a.wmode = 1;
-    a.cW = dt / 2.; a.tidx = tbase + 0;
-    if ((r = launch(c, a)) || (r = lim(c->dW0))) return r;
-    a.win = c->dW0; a.Ain = A; a.cA = dt / 3.; a.Wout = c->dW1; a.cW = dt / 2.; a.tidx = tbase + 1;
-    if ((r = launch(c, a)) || (r = lim(c->dW1))) return r;
-    a.win = c->dW1; a.cA = dt / 3.; a.Wout = c->dW0; a.cW = dt; a.tidx = tbase + 2;
-    if ((r = launch(c, a)) || (r = lim(c->dW0))) return r;
-    a.win = c->dW0; a.cA = dt / 6.; a.Wout = nullptr; a.wmode = 0; a.tidx = tbase + 3;
-    if ((r = launch(c, a))) return r;
-  } else if (method == 1) {   // evolve_sspRK3_mesh (RungeKutta.c:130-188)
-    a.win = U; a.U = U; a.Aout = A; a.cA = dt / 6.; a.Wout = c->dW0; a.wmode = 1; a.cW = dt;
-    a.tidx = tbase + 0;
-    if ((r = launch(c, a)) || (r = lim(c->dW0))) return r;
-    a.win = c->dW0; a.Ain = A; a.cA = dt / 6.; a.Wout = c->dW1; a.wmode = 2; a.cW = dt; a.tidx = tbase + 1;
-    if ((r = launch(c, a)) || (r = lim(c->dW1))) return r;
-    a.win = c->dW1; a.cA = dt * 2. / 3.; a.Wout = nullptr; a.wmode = 0; a.tidx = tbase + 2;
-    if ((r = launch(c, a))) return r;
-  } else {   // evolve_Euler_mesh (RungeKutta.c:85-115)
-    a.win = U; a.U = U; a.Aout = A; a.cA = dt; a.wmode = 0; a.tidx = tbase;
-    if ((r = launch(c, a))) return r;
+  auto lim = [&](double *reg) { return launch_limiter_on(c, reg); };
+  if (method == 2) {   // evolve_Euler_mesh (RungeKutta.c:85-115)
+    a.Aout = A; a.cA = dt;
+    if ((r = stage(0, U, nullptr, 0, 0.))) return r;
+    if (c->lim_on && (r = lim(A))) return r;
+  } else if (!c->lim_on && method == 0) {   // evolve_RK4_mesh (RungeKutta.c:19-82)
+    if ((r = stage(0, U, c->dW0, 3, dt / 2.)) || (r = stage(1, c->dW0, c->dW1, 3, dt / 2.)) ||
+        (r = stage(2, c->dW1, A, 3, dt)))
+      return r;
+    a.Wa = c->dW0; a.Wb = c->dW1; a.cA = dt / 6.;
+    if ((r = stage(3, A, U, 5, 0.))) return r;
+  } else if (!c->lim_on) {                  // evolve_sspRK3_mesh (RungeKutta.c:130-188)
+    if ((r = stage(0, U, c->dW0, 3, dt)) || (r = stage(1, c->dW0, c->dW1, 4, dt))) return r;
+    a.Wa = c->dW0; a.cA = dt / 6.;
+    if ((r = stage(2, c->dW1, U, 6, dt))) return r;
+  } else if (method == 0) {
+    a.Aout = A; a.cA = dt / 6.;
+    if ((r = stage(0, U, c->dW0, 1, dt / 2.)) || (r = lim(c->dW0))) return r;
+    a.Ain = A; a.cA = dt / 3.;
+    if ((r = stage(1, c->dW0, c->dW1, 1, dt / 2.)) || (r = lim(c->dW1))) return r;
+    if ((r = stage(2, c->dW1, c->dW0, 1, dt)) || (r = lim(c->dW0))) return r;
+    a.cA = dt / 6.;
+    if ((r = stage(3, c->dW0, nullptr, 0, 0.)) || (r = lim(A))) return r;
+  } else {
+    a.Aout = A; a.cA = dt / 6.;
+    if ((r = stage(0, U, c->dW0, 1, dt)) || (r = lim(c->dW0))) return r;
+    a.Ain = A;
+    if ((r = stage(1, c->dW0, c->dW1, 2, dt)) || (r = lim(c->dW1))) return r;
+    a.cA = dt * 2. / 3.;
+    if ((r = stage(2, c->dW1, nullptr, 0, 0.)) || (r = lim(A))) return r;
   }
-  if ((r = lim(A))) return r;
   // FILTER bin after the full step (main.c:628-630)
-  if (c->filt_on && (r = launch_filters(c, A))) return r;
+  if (c->filt_on && (r = launch_filters(c, end))) return r;
   return NMX_OK;
 }
 
@@ -2686,133 +2513,59 @@ extern "C" int nmx_autotune(nmx_ctx *c) {
   const int method = method_id(c);
   stage_times(method, c->time, c->dt, c->hT);
   HIPCHK(hipMemcpyAsync(c->dT, c->hT, 4 * sizeof(double), hipMemcpyHostToDevice, c->stream));
-  const char *blocks[] = {"full", "half", "quarter"};
-  const char *xcds[] = {"yes", "no"};
-  std::string best_b = P(c, "nmx_block"), best_x = P(c, "nmx_xcd");
-  float best = 1e30f;
   hipEvent_t t0, t1;
   HIPCHK(hipEventCreate(&t0));
   HIPCHK(hipEventCreate(&t1));
-  for (const char *b : blocks)
-    for (const char *x : xcds) {
-      c->par["nmx_block"] = b;
-      c->par["nmx_xcd"] = x;
-      if ((r = issue_step(c, method, c->dt, 0, false))) return r;   // warm-up
+  // 4 steps after one to warm up
+  auto steps_ms = [&](float &ms) -> int {
+    if (int rr = issue_step(c, method, c->dt, 0, false)) return rr;
+    HIPCHK(hipEventRecord(t0, c->stream));
+    for (int s = 0; s < 4; ++s)
+      if (int rr = issue_step(c, method, c->dt, 0, (s & 1) != 0)) return rr;
+    HIPCHK(hipEventRecord(t1, c->stream));
+    HIPCHK(hipEventSynchronize(t1));
+    HIPCHK(hipEventElapsedTime(&ms, t0, t1));
+    return NMX_OK;
+  };
+  std::string best_x = P(c, "nmx_xcd");
+  float best = 1e30f;
+  for (const char *x : {"yes", "no"}) {
+    c->par["nmx_xcd"] = x;
+    float ms = 0;
+    if ((r = steps_ms(ms))) return r;
+    if (ms < best) { best = ms; best_x = x; }
+  }
+  c->par["nmx_xcd"] = best_x;
+  if (c->amr) {
+    // the buckets' stages timed alone, on an RK4 second-stage launch (reads w
+    // and u, writes the next w), order them for the lanes
+    StageArgs sa = base_args(c);
+    sa.win = c->dW0; sa.U = c->dU; sa.Wout = c->dW1; sa.wmode = 3; sa.cW = c->dt / 2.; sa.tidx = 0;
+    HIPCHK(hipMemcpyAsync(c->dW0, c->dU, c->nstate * 8, hipMemcpyDeviceToDevice, c->stream));
+    if ((r = launch_amr(c, sa))) return r;   // fills the face buffer
+    const AmrArgs a = amr_args(c, sa);
+    for (auto &b : c->buckets) {
+      if ((r = launch_bucket(c, a, b, sa.xcd_map, c->stream))) return r;   // warm-up
       HIPCHK(hipEventRecord(t0, c->stream));
-      for (int s = 0; s < 4 && !r; ++s) r = issue_step(c, method, c->dt, 0, (s & 1) != 0);
-      if (r) return r;
+      for (int s = 0; s < 5; ++s)
+        if ((r = launch_bucket(c, a, b, sa.xcd_map, c->stream))) return r;
       HIPCHK(hipEventRecord(t1, c->stream));
       HIPCHK(hipEventSynchronize(t1));
-      float ms = 0;
-      HIPCHK(hipEventElapsedTime(&ms, t0, t1));
-      if (ms < best) { best = ms; best_b = b; best_x = x; }
+      HIPCHK(hipEventElapsedTime(&b.ms, t0, t1));
     }
-  c->par["nmx_block"] = best_b;
-  c->par["nmx_xcd"] = best_x;
-  // batched path: each order bucket gets its own tile, timed alone on an
-  // RK4 second-stage launch (reads w, u_p, u_acc; writes u_acc, w)
-  if (c->amr) {
-    StageArgs sa = base_args(c);
-    sa.win = c->dW0; sa.U = c->dU; sa.Ain = c->dA; sa.Aout = c->dA; sa.Wout = c->dW1;
-    sa.wmode = 1; sa.cA = c->dt / 3.; sa.cW = c->dt / 2.; sa.tidx = 0;
-    HIPCHK(hipMemcpyAsync(c->dW0, c->dU, c->nstate * 8, hipMemcpyDeviceToDevice, c->stream));
-    HIPCHK(hipMemcpyAsync(c->dA, c->dU, c->nstate * 8, hipMemcpyDeviceToDevice, c->stream));
-    {   // the face buffer of every bucket, for the face-kernel shape
-      const std::string shape = P(c, "nmx_batch");
-      c->par["nmx_batch"] = "legacy";
-      r = launch_amr(c, sa);
-      c->par["nmx_batch"] = shape;
-      if (r) return r;
-    }
-    const int xcd = best_x == "yes" ? 1 : 0;
-    AmrArgs a = amr_args(c, sa);
-    for (auto &b : c->buckets) {
-      // each order's tile, timed alone: with the face kernel's buffer
-      // (FV buckets and the legacy shape) and in the order's own launch of
-      // the receiver-gathering kernel (DG buckets)
-      for (int variant = 0; variant < (b.fv ? 1 : 2); ++variant) {
-        int best_div = 0;
-        float bms = 1e30f;
-        const std::vector<int> divs = b.fv ? std::vector<int>{1}
-                                      : variant == 0 ? std::vector<int>{1, 2, 4} : std::vector<int>{1, 2, 3, 4};
-        auto one = [&](int div) {
-          return variant == 0 ? launch_bucket(c, a, b, div, xcd, c->stream)
-                              : launch_order(c, sa, b.n, div, c->stream);
-        };
-        for (int div : divs) {
-          if ((r = one(div))) return r;   // warm-up
-          HIPCHK(hipEventRecord(t0, c->stream));
-          for (int s = 0; s < 5 && !r; ++s) r = one(div);
-          if (r) return r;
-          HIPCHK(hipEventRecord(t1, c->stream));
-          HIPCHK(hipEventSynchronize(t1));
-          float ms = 0;
-          HIPCHK(hipEventElapsedTime(&ms, t0, t1));
-          if (ms < bms) { bms = ms; best_div = div; }
-        }
-        if (variant == 0) { b.div = best_div; b.ms_legacy = bms; }
-        else { c->bdiv[b.n] = best_div; b.ms_order = bms; }
-      }
-      if (b.fv) b.ms_order = b.ms_legacy;
-    }
-    auto lanes_for = [c](const std::string &shape) {
-      for (auto &b : c->buckets) b.ms = shape == "legacy" ? b.ms_legacy : b.ms_order;
-      assign_lanes(c);
-    };
-    lanes_for(P(c, "nmx_batch"));
-    // launch shape: one persistent launch per stage, one launch per order on
-    // the stream lanes, or per order with the face kernel first, whichever
-    // takes the steps fastest (unless set)
+    assign_lanes(c);
+    // one launch for the DG elements of all orders, or one per order, by
+    // whole steps (unless set)
     if (!c->batch_fixed && c->anydg) {
-      std::string best_shape = P(c, "nmx_batch");
+      std::string best_shape;
       float bt = 1e30f;
-      for (const char *shape : {"persistent", "buckets", "legacy"}) {
+      for (const char *shape : {"persistent", "buckets"}) {
         c->par["nmx_batch"] = shape;
-        lanes_for(shape);
-        if ((r = issue_step(c, method, c->dt, 0, false))) return r;   // warm-up
-        HIPCHK(hipEventRecord(t0, c->stream));
-        for (int s = 0; s < 4 && !r; ++s) r = issue_step(c, method, c->dt, 0, (s & 1) != 0);
-        if (r) return r;
-        HIPCHK(hipEventRecord(t1, c->stream));
-        HIPCHK(hipEventSynchronize(t1));
         float ms = 0;
-        HIPCHK(hipEventElapsedTime(&ms, t0, t1));
+        if ((r = steps_ms(ms))) return r;
         if (ms < bt) { bt = ms; best_shape = shape; }
       }
       c->par["nmx_batch"] = best_shape;
-      lanes_for(best_shape);
-    }
-    // with the face kernel's shape, the order buckets' tiles refined on whole
-    // steps, where the buckets run beside one another as they will: each DG
-    // bucket, longest first, keeps the tile that makes the steps fastest with
-    // the others fixed (the tile that is fastest alone need not be)
-    if (P(c, "nmx_batch") == "legacy" && c->anydg && c->buckets.size() > 1) {
-      auto steps_ms = [&](float &ms) -> int {
-        if (int rr = issue_step(c, method, c->dt, 0, false)) return rr;   // warm-up
-        HIPCHK(hipEventRecord(t0, c->stream));
-        for (int s = 0; s < 6; ++s)
-          if (int rr = issue_step(c, method, c->dt, 0, (s & 1) != 0)) return rr;
-        HIPCHK(hipEventRecord(t1, c->stream));
-        HIPCHK(hipEventSynchronize(t1));
-        HIPCHK(hipEventElapsedTime(&ms, t0, t1));
-        return NMX_OK;
-      };
-      float cur = 0.f;
-      if ((r = steps_ms(cur))) return r;
-      for (size_t k = 0; k < c->buckets.size(); ++k) {
-        auto &b = c->buckets[c->border[k]];
-        if (b.fv) continue;
-        const int keep = b.div;
-        for (int div : {1, 2, 4}) {
-          if (div == keep) continue;
-          const int prev = b.div;
-          b.div = div;
-          float ms = 0.f;
-          if ((r = steps_ms(ms))) return r;
-          if (ms < cur) cur = ms;
-          else b.div = prev;
-        }
-      }
     }
   }
   (void)hipEventDestroy(t0);
@@ -2923,7 +2676,7 @@ extern "C" int nmx_evolve(nmx_ctx *c, int nsteps) {
     HIPCHK(hipMemcpyAsync(c->dT, c->hT, 4 * sizeof(double), hipMemcpyHostToDevice, c->stream));
     int r = issue_step(c, method, dt, 0, parity);
     if (r) return r;
-    parity = !parity;
+    parity = parity != step_swaps(c, method);
     advance_time(c, dt);
   }
   // keep register pointers fixed (captured graphs refer to them)
@@ -3117,8 +2870,8 @@ static int adj_amr_prepare(nmx_ctx *c) {
 // launch per order, all on the context's stream
 static int launch_adj_amr(nmx_ctx *c, const AdjArgs &s) {
   AdjAmrArgs a;
-  a.lam = s.lam; a.Abase = s.Abase; a.Wbase = s.Wbase; a.Aout = s.Aout; a.Wout = s.Wout; a.R = s.R;
-  a.cA = s.cA; a.cU = s.cU; a.cW = s.cW;
+  a.lam = s.lam; a.phi = s.phi; a.U = s.U; a.Wa = s.Wa; a.Wb = s.Wb; a.Wout = s.Wout; a.R = s.R;
+  a.cA = s.cA; a.cW = s.cW; a.wmode = s.wmode;
   a.eoff = c->deoff; a.en = c->den; a.dXbdX = c->dXbdX; a.egeo = c->degeo; a.edom = c->dedom;
   a.dXdx = c->dXdx; a.Dall = c->dbD; a.xball = c->dbxb; a.wend_inv = c->dbW;
   a.af = c->dadjf; a.goff = c->dadjg; a.G = c->dadjG; a.jobs = c->dadjj; a.njobs = c->adjnjobs;
@@ -3153,46 +2906,39 @@ extern "C" int nmx_adjoint_setrhs(nmx_ctx *c, int reg_out, int reg_in) {
   if (!out || !in || out == in) return fail(NMX_EINVAL, "bad registers");
   AdjArgs a = adj_base_args(c);
   a.lam = in;
+  a.phi = in;
   a.R = out;
   return launch_adj(c, a);
 }
 
-// One adjoint RK step lam <- (du_{n+1}/du_n)^T lam: the forward stages of
-// issue_step taken in reverse.  With y_s = L^T x_s:
-//   RK4:    x4 = lam; acc = lam + dt/6 y4; x3 = dt/3 lam + dt^2/6 y4;
-//           acc += y3; x2 = dt/3 lam + dt/2 y3; acc += y2; x1 = dt/6 lam + dt/2 y2;
-//           acc += y1
-//   sspRK3: x3 = lam; acc = lam + 2dt/3 y3; x2 = dt/6 lam + dt^2/6 y3;
-//           acc += y2; x1 = x2 + dt y2; acc += y1
-//   Euler:  acc = lam + dt y1
+// One adjoint RK step lam <- (du_{n+1}/du_n)^T lam.  L is the same at every
+// stage, so du_{n+1}/du_n is a polynomial in dt L and its transpose the same
+// polynomial in dt L^T: the forward's stages with the transposed RHS.
+// phi's component stays (y_phi = 0), so only Euler steps, whose state is
+// read by neighbours while it is written, end in the other register.
 static int issue_adj_step(nmx_ctx *c, int method, double dt, bool swap_parity) {
-  double *L = swap_parity ? c->dA : c->dL;
-  double *Acc = swap_parity ? c->dL : c->dA;
   AdjArgs a = adj_base_args(c);
   int r;
+  double *L = method == 2 && swap_parity ? c->dA : c->dL;
+  a.phi = L;
+  a.U = L;
+  auto stage = [&](double *lam, double *wout, int wmode, double cW) {
+    a.lam = lam; a.Wout = wout; a.wmode = wmode; a.cW = cW;
+    return launch_adj(c, a);
+  };
   if (method == 0) {
-    a.lam = L; a.Abase = L; a.Aout = Acc; a.cA = dt / 6.;
-    a.Wbase = L; a.Wout = c->dW0; a.cU = dt / 3.; a.cW = dt * dt / 6.;
-    if ((r = launch_adj(c, a))) return r;
-    a.lam = c->dW0; a.Abase = Acc; a.cA = 1.0; a.Wbase = L; a.Wout = c->dW1; a.cU = dt / 3.; a.cW = dt / 2.;
-    if ((r = launch_adj(c, a))) return r;
-    a.lam = c->dW1; a.Wout = c->dW0; a.cU = dt / 6.; a.cW = dt / 2.;
-    if ((r = launch_adj(c, a))) return r;
-    a.lam = c->dW0; a.Wout = nullptr; a.Wbase = nullptr;
-    if ((r = launch_adj(c, a))) return r;
-  } else if (method == 1) {
-    a.lam = L; a.Abase = L; a.Aout = Acc; a.cA = 2. * dt / 3.;
-    a.Wbase = L; a.Wout = c->dW0; a.cU = dt / 6.; a.cW = dt * dt / 6.;
-    if ((r = launch_adj(c, a))) return r;
-    a.lam = c->dW0; a.Abase = Acc; a.cA = 1.0; a.Wbase = c->dW0; a.Wout = c->dW1; a.cU = 1.0; a.cW = dt;
-    if ((r = launch_adj(c, a))) return r;
-    a.lam = c->dW1; a.Wout = nullptr; a.Wbase = nullptr;
-    if ((r = launch_adj(c, a))) return r;
-  } else {
-    a.lam = L; a.Abase = L; a.Aout = Acc; a.cA = dt;
-    if ((r = launch_adj(c, a))) return r;
+    if ((r = stage(L, c->dW0, 3, dt / 2.)) || (r = stage(c->dW0, c->dW1, 3, dt / 2.)) ||
+        (r = stage(c->dW1, c->dA, 3, dt)))
+      return r;
+    a.Wa = c->dW0; a.Wb = c->dW1; a.cA = dt / 6.;
+    return stage(c->dA, L, 5, 0.);
   }
-  return NMX_OK;
+  if (method == 1) {
+    if ((r = stage(L, c->dW0, 3, dt)) || (r = stage(c->dW0, c->dW1, 4, dt))) return r;
+    a.Wa = c->dW0; a.cA = dt / 6.;
+    return stage(c->dW1, L, 6, dt);
+  }
+  return stage(L, swap_parity ? c->dL : c->dA, 1, dt);
 }
 
 extern "C" int nmx_adjoint_evolve(nmx_ctx *c, int nsteps) {
@@ -3232,7 +2978,7 @@ extern "C" int nmx_adjoint_evolve(nmx_ctx *c, int nsteps) {
   for (; done < nsteps; ++done) {
     int r = issue_adj_step(c, method, dt, parity);
     if (r) return r;
-    parity = !parity;
+    parity = parity != (method == 2);
   }
   if (parity) HIPCHK(hipMemcpyAsync(c->dL, c->dA, c->nstate * 8, hipMemcpyDeviceToDevice, c->stream));
   HIPCHK(hipEventRecord(c->ev1, c->stream));

@@ -1,6 +1,5 @@
-// dg_common.h -- device code shared by the plain and the batched DG stage
-// kernels: numerical flux, boundary profile, cubed-shell Jacobian, and the
-// per-node RHS + RK stage update from LDS-staged element data.
+// dg_common.h -- device code shared by the DG, adjoint and FV stage kernels:
+// numerical flux, boundary profile, cubed-shell Jacobian and the RK stages.
 #pragma once
 #include <hip/hip_runtime.h>
 
@@ -81,27 +80,97 @@ __device__ __forceinline__ double det3(const double M[3][3]) {
          M[0][2] * (M[1][0] * M[2][1] - M[1][1] * M[2][0]);
 }
 
-// Everything the per-node update needs besides LDS.
-struct NodeOut {
-  const double *win, *U, *Ain;
-  double *Aout, *Wout, *R;
-  double cA, cW, wend_inv;
-  int wmode, numflux;
-  // streaming hints for the registers each node touches once per stage:
-  // bit 0 loads of u_p and the accumulator base, bit 1 stores of the
-  // accumulator and the RHS, bit 2 stores of the next stage input
-  int nt = 0;
+// What stage_in and stage_out take of a stage's arguments (kernels.h).
+struct StageRegs {
+  const double *win, *U, *Wa, *Wb;
+  double cA, cW;
+  int wmode;
 };
 
-__device__ __forceinline__ double ld_stream(const double *p, bool nt) {
-  return nt ? __builtin_nontemporal_load(p) : *p;
+// The operands of stage_out at one node.
+struct StageIn {
+  double U[5], a[4], b[4];
+};
+
+// Stages without an accumulator (wmodes 3 to 6), for right-hand sides in
+// which phi does not appear.  An RK step keeps its stage inputs W1, W2, ..
+// instead of accumulating u + sum_s b_s dt r_s, and the last stage recovers
+// the earlier r_s from them:
+//   RK4     W1 = U + dt/2 r1, W2 = U + dt/2 r2, W3 = U + dt r3, so the step
+//           ends at U + ((W1 - U) + 2 (W2 - U) + (W3 - U))/3 + dt/6 r4;
+//   sspRK3  W1 = U + dt r1, W2 = 0.75 U + 0.25 (W1 + dt r2), so it ends at
+//           U + 2/3 ((W2 - U) + dt r3).
+// phi is in no right-hand side and r_phi = pi, so its stage values are not
+// kept: the last stage sums the stages' pi.  Per RK4 step and node that is
+// 8 + 12 + 12 + 22 doubles moved instead of 15 + 25 + 25 + 15 (sspRK3: 8 +
+// 12 + 15 instead of 15 + 25 + 15), and the state is stepped in place: the
+// last stage reads U at its own nodes only.  W - U is exact where W is near
+// U, so a step has the rounding of the stage inputs, thirds of ulps, and of
+// one sum, where the accumulator had one rounding per stage.
+// gi: the node's first state double; vo: the offsets of pi and c, in the
+// order they are handed over; po: phi's.
+template <class O>
+__device__ __forceinline__ void stage_in(const O &o, long gi, const int (&vo)[4], int po, StageIn &q) {
+  if (o.wmode <= 4) {
+    if (o.U != o.win) {
+#pragma unroll
+      for (int v = 0; v < 4; ++v) q.U[v] = o.U[gi + vo[v]];
+    }
+  } else {
+#pragma unroll
+    for (int v = 0; v < 4; ++v) q.U[v] = o.U[gi + vo[v]];
+    q.U[4] = o.U[gi + po];
+    q.a[0] = o.Wa[gi + vo[0]];
+    if (o.wmode == 5) {
+#pragma unroll
+      for (int v = 1; v < 4; ++v) q.a[v] = o.Wa[gi + vo[v]];
+#pragma unroll
+      for (int v = 0; v < 4; ++v) q.b[v] = o.Wb[gi + vo[v]];
+    }
+  }
 }
-__device__ __forceinline__ void st_stream(double *p, double v, bool nt) {
-  if (nt) __builtin_nontemporal_store(v, p);
-  else *p = v;
+template <class O>
+__device__ __forceinline__ void stage_in(const O &o, long gi, int np3, StageIn &q) {
+  const int vo[4] = {0, np3, 2 * np3, 3 * np3};
+  stage_in(o, gi, vo, 4 * np3, q);
 }
 
-// Geometry of one element.
+// own: the stage input's pi and c at the node; r: their RHS.  PHI: the
+// system has r_phi = pi (else phi is left as it is).  Outputs in out[0..3],
+// and phi in out[4] when the step ends (returns true then).
+template <bool PHI, class O>
+__device__ __forceinline__ bool stage_out(const O &o, const StageIn &q, const double own[4], const double r[4],
+                                          double out[5]) {
+  if (o.wmode == 3) {
+    if (o.U == o.win) {
+#pragma unroll
+      for (int v = 0; v < 4; ++v) out[v] = own[v] + o.cW * r[v];
+    } else {
+#pragma unroll
+      for (int v = 0; v < 4; ++v) out[v] = q.U[v] + o.cW * r[v];
+    }
+    return false;
+  }
+  if (o.wmode == 4) {
+#pragma unroll
+    for (int v = 0; v < 4; ++v) out[v] = 0.75 * q.U[v] + 0.25 * (own[v] + o.cW * r[v]);
+    return false;
+  }
+  if (o.wmode == 5) {
+#pragma unroll
+    for (int v = 0; v < 4; ++v) {
+      const double s = (q.a[v] - q.U[v]) + 2. * (q.b[v] - q.U[v]) + (own[v] - q.U[v]);
+      out[v] = q.U[v] + (s * (1. / 3.) + o.cA * r[v]);
+    }
+    if (PHI) out[4] = q.U[4] + o.cA * (q.U[0] + 2. * (q.a[0] + q.b[0]) + own[0]);
+    return PHI;
+  }
+#pragma unroll
+  for (int v = 0; v < 4; ++v) out[v] = q.U[v] + (2. / 3.) * ((own[v] - q.U[v]) + o.cW * r[v]);
+  if (PHI) out[4] = q.U[4] + o.cA * (q.U[0] + q.a[0] + 4. * own[0]);
+  return PHI;
+}
+
 // outward unit normal and lift scale sqrtgdiag / w_end of face f at a node
 // with metric M (dX/dx; unused on Cartesian elements, GEOM 0), as the
 // stage kernels compute them (dg.c:90-146, utilities.c:48-81)
@@ -123,155 +192,6 @@ __device__ __forceinline__ void face_normal(const double M[3][3], const double *
     const double ism = 1.0 / (sig * s);
     nrm[0] = r0 * ism; nrm[1] = r1 * ism; nrm[2] = r2 * ism;
     scale = dXbdX[dir] * s * wend_inv;
-  }
-}
-
-struct ElmGeo {
-  double dXbdX[3];
-  const double *dXdx;   // GEOM 1: element's 9*np block
-  double bb[6];         // GEOM 2: element box in patch coordinates
-  double s0, s1;
-  int dom;
-};
-
-// RHS of scalarwave1 at one node and the RK stage combination.
-// s_u[v][np3]: own pi,cx,cy,cz; s_f[v][f][np2]: adjacent values on face f;
-// gbase: element's first state double; node: ijk.
-// Upre/Apre: the epilogue's u_p and accumulator base at this node, loaded
-// earlier by the caller (nullptr: loaded here)
-template <int NP, int GEOM>
-__device__ __forceinline__ void node_update(const NodeOut &o, const ElmGeo &g,
-                                            const double (*s_u)[NP * NP * NP],
-                                            const double (*s_f)[6][NP * NP],
-                                            const double *s_D, const double *s_xb, long gbase,
-                                            int node, const double *Upre = nullptr,
-                                            const double *Apre = nullptr) {
-  constexpr int NP2 = NP * NP;
-  constexpr int NP3 = NP * NP * NP;
-  constexpr bool CURV = (GEOM != 0);
-  const int k = node / NP2;
-  const int j = (node / NP) % NP;
-  const int i = node % NP;
-  const long gi = gbase + node;
-
-  double M[3][3];
-  if (GEOM == 1) {
-#pragma unroll
-    for (int m = 0; m < 3; ++m)
-#pragma unroll
-      for (int q = 0; q < 3; ++q) M[m][q] = g.dXdx[(3 * m + q) * NP3 + node];
-  } else if (GEOM == 2) {
-    const int I[3] = {i, j, k};
-    double X[3];
-#pragma unroll
-    for (int d = 0; d < 3; ++d)
-      X[d] = 0.5 * ((g.bb[2 * d + 1] - g.bb[2 * d]) * s_xb[I[d]] + (g.bb[2 * d + 1] + g.bb[2 * d]));
-    shell_dXdx(g.dom, g.s0, g.s1, X, M);
-  }
-
-  // tensor-product derivative along one direction m at a time
-  // (mm_array_indir, array.c:100-300), folded at once into the Cartesian
-  // partials d_q f = sum_m dXdx[m][q] dXbdX[m] D_m f (derivs.c:102-181):
-  // r_pi = d_q c_q, r_cq = d_q pi
-  double rpi = 0.0, rc[3] = {0.0, 0.0, 0.0};
-#pragma unroll
-  for (int m = 0; m < 3; ++m) {
-    const int im = (m == 0) ? i : (m == 1) ? j : k;
-    const int stride = (m == 0) ? 1 : (m == 1) ? NP : NP2;
-    const int base = node - im * stride;
-    double dp = 0.0, d0 = 0.0, d1 = 0.0, d2 = 0.0;
-#pragma unroll
-    for (int l = 0; l < NP; ++l) {
-      const double Dl = s_D[im * NP + l];
-      const int src = base + l * stride;
-      dp += Dl * s_u[0][src];
-      if (CURV) {
-        d0 += Dl * s_u[1][src];
-        d1 += Dl * s_u[2][src];
-        d2 += Dl * s_u[3][src];
-      } else {
-        d0 += Dl * s_u[1 + m][src];
-      }
-    }
-    if (CURV) {
-      const double sp = g.dXbdX[m] * dp;
-      rpi += M[m][0] * (g.dXbdX[m] * d0) + M[m][1] * (g.dXbdX[m] * d1) + M[m][2] * (g.dXbdX[m] * d2);
-      rc[0] += M[m][0] * sp;
-      rc[1] += M[m][1] * sp;
-      rc[2] += M[m][2] * sp;
-    } else {
-      rpi += g.dXbdX[m] * d0;
-      rc[m] = g.dXbdX[m] * dp;
-    }
-  }
-
-  // numerical flux and strong-form lift on the faces this node lies on
-  // (dg_add_surface_fluxes_sign_fvflag, dg.c:90-146; normal dg.c:470-481 via
-  // node_normal_from_idXdx_at_ijk, utilities.c:48-81)
-  const int I[3] = {i, j, k};
-#pragma unroll
-  for (int dir = 0; dir < 3; ++dir) {
-#pragma unroll
-    for (int side = 0; side < 2; ++side) {
-      if (I[dir] != side * (NP - 1)) continue;
-      const int f = 2 * dir + side;
-      const double sig = side ? 1.0 : -1.0;
-      double nrm[3], scale;
-      if (CURV) {
-        double s2 = M[dir][0] * M[dir][0] + M[dir][1] * M[dir][1] + M[dir][2] * M[dir][2];
-        double s = sqrt(s2);
-        const double ism = 1.0 / (sig * s);
-        nrm[0] = M[dir][0] * ism; nrm[1] = M[dir][1] * ism; nrm[2] = M[dir][2] * ism;
-        scale = g.dXbdX[dir] * s * o.wend_inv;
-      } else {
-        nrm[0] = nrm[1] = nrm[2] = 0.0;
-        nrm[dir] = sig;
-        scale = g.dXbdX[dir] * o.wend_inv;
-      }
-      const int ia = (dir == 0) ? j : i;          // index along Dir1_norm(dir)
-      const int ib = (dir == 2) ? j : k;          // index along Dir2_norm(dir)
-      const int q = ia + NP * ib;
-      const double dcv[3] = {s_u[1][node] - s_f[1][f][q], s_u[2][node] - s_f[2][f][q],
-                             s_u[3][node] - s_f[3][f][q]};
-      double F[4];
-      face_flux(o.numflux, nrm, s_u[0][node] - s_f[0][f][q], dcv, F);
-      rpi -= F[0] * scale;
-      rc[0] -= F[1] * scale;
-      rc[1] -= F[2] * scale;
-      rc[2] -= F[3] * scale;
-    }
-  }
-
-  // r = -(div f + lift), r_phi = pi (scalarwave1.c:242-321) and the stage
-  // combination (RungeKutta.c:19-188, variables.c:932-1041)
-  const double r[5] = {rpi, rc[0], rc[1], rc[2], s_u[0][node]};
-  const bool ntl = o.nt & 1, nta = o.nt & 2, ntw = o.nt & 4;
-  double Ubuf[5], Abuf[5];
-  if (o.wmode) {
-#pragma unroll
-    for (int v = 0; v < 5; ++v) Ubuf[v] = Upre ? Upre[v] : ld_stream(o.U + gi + v * NP3, ntl);
-  }
-  if (o.Aout) {
-    const double *bas = o.Ain ? o.Ain : o.win;
-#pragma unroll
-    for (int v = 0; v < 5; ++v) Abuf[v] = Apre ? Apre[v] : ld_stream(bas + gi + v * NP3, ntl);
-  }
-  if (o.R) {
-#pragma unroll
-    for (int v = 0; v < 5; ++v) st_stream(o.R + gi + v * NP3, r[v], nta);
-  }
-  if (o.Aout) {
-#pragma unroll
-    for (int v = 0; v < 5; ++v) st_stream(o.Aout + gi + v * NP3, Abuf[v] + o.cA * r[v], nta);
-  }
-  if (o.wmode == 1) {
-#pragma unroll
-    for (int v = 0; v < 5; ++v) st_stream(o.Wout + gi + v * NP3, Ubuf[v] + o.cW * r[v], ntw);
-  } else if (o.wmode == 2) {
-    const double wv[5] = {s_u[0][node], s_u[1][node], s_u[2][node], s_u[3][node],
-                          o.win[gi + 4 * NP3]};
-#pragma unroll
-    for (int v = 0; v < 5; ++v) st_stream(o.Wout + gi + v * NP3, 0.75 * Ubuf[v] + 0.25 * (wv[v] + o.cW * r[v]), ntw);
   }
 }
 

@@ -483,7 +483,7 @@ __device__ __forceinline__ void fv_line(const double *eu, const Face &face, int 
 
 // Outputs of the RK stage (as StageArgs / AmrArgs name them).
 struct FvOut {
-  const double *win, *U, *Ain;
+  const double *win, *U, *Wa, *Wb, *Ain;
   double *Aout, *Wout, *R;
   double cA, cW;
   int wmode;
@@ -518,6 +518,18 @@ __device__ __forceinline__ void fv_element(const FvOut &o, long gbase, const Fac
     double r[5];
 #pragma unroll
     for (int v = 0; v < 4; ++v) r[v] = -acc[v][node];
+    if (o.wmode >= 3) {
+      double own[4], out[5];
+      StageIn q;
+#pragma unroll
+      for (int v = 0; v < 4; ++v) own[v] = o.win[gi + v * NP3];
+      stage_in(o, gi, NP3, q);
+      const bool end = stage_out<true>(o, q, own, r, out);
+#pragma unroll
+      for (int v = 0; v < 4; ++v) o.Wout[gi + v * NP3] = out[v];
+      if (end) o.Wout[gi + 4 * NP3] = out[4];
+      continue;
+    }
     r[4] = o.win[gi];
     double Ubuf[5], Abuf[5];
     if (o.wmode) {
@@ -576,7 +588,7 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(2))) void fv
     e_first = a.e0 + blockIdx.x;
     e_step = gridDim.x;
   }
-  const FvOut o = {a.win, a.U, a.Ain, a.Aout, a.Wout, a.R, a.cA, a.cW, a.wmode};
+  const FvOut o = {a.win, a.U, a.Wa, a.Wb, a.Ain, a.Aout, a.Wout, a.R, a.cA, a.cW, a.wmode};
 
   for (int e = e_first; e < e_hi; e += e_step) {
     FvGeo G;
@@ -628,7 +640,7 @@ __global__ __launch_bounds__(NT) void fvelm_amr_kernel(AmrArgs a, const double *
     i_first = blockIdx.x;
     i_step = gridDim.x;
   }
-  const FvOut o = {a.win, a.U, a.Ain, a.Aout, a.Wout, a.R, a.cA, a.cW, a.wmode};
+  const FvOut o = {a.win, a.U, a.Wa, a.Wb, a.Ain, a.Aout, a.Wout, a.R, a.cA, a.cW, a.wmode};
 
   for (int it = i_first; it < i_hi; it += i_step) {
     const NMX_CONST SlotRec &R = *(const NMX_CONST SlotRec *)(a.rec + it);

@@ -11,9 +11,16 @@ namespace nmx {
 //   Aout = (Ain ? Ain : win) + cA * r              (RK accumulator "u")
 //   Wout = U + cW * r                   (wmode 1)  (next stage input "w")
 //   Wout = 0.75 U + 0.25 (win + cW r)   (wmode 2)  (sspRK3 third stage input)
+// and, without an accumulator (stage_out, dg_common.h):
+//   Wout = U + cW r                     (wmode 3)  pi and c only
+//   Wout = 0.75 U + 0.25 (win + cW r)   (wmode 4)  pi and c only
+//   Wout = the end of an RK4 step       (wmode 5)  from U, Wa, Wb, win and r
+//   Wout = the end of an sspRK3 step    (wmode 6)  from U, Wa, win and r
+// (Wout may be U in modes 5 and 6).
 struct StageArgs {
   const double *win = nullptr;   // stage input state
   const double *U = nullptr;     // state at the start of the step (u_p)
+  const double *Wa = nullptr, *Wb = nullptr;   // the step's first and second stage inputs after U
   const double *Ain = nullptr;
   double *Aout = nullptr;
   double *Wout = nullptr;
@@ -34,7 +41,6 @@ struct StageArgs {
   double om = 0;
   int e0 = 0, e1 = 0;
   int wmode = 0, numflux = 0, profile = 0;
-  int nt = 0;                    // streaming hints of the epilogue (NodeOut::nt)
   int fv_mid = 0;                // FV elements: metric and normal at the midpoints
   // FV elements: fv_divf_extrap_s1, _s2, _opt (ex_on: s1 > 0 or s2 < DBL_MAX)
   double ex_s1 = 0, ex_s2 = 1.7976931348623157e308;
@@ -46,17 +52,19 @@ struct StageArgs {
   double rec_s1 = 0, rec_s2 = 1.7976931348623157e308;
 };
 
-// Arguments of one fused adjoint RHS + adjoint RK stage launch: y = L^T lam
-// (L the Jacobian of the scalarwave1 DG RHS with respect to u), then
-//   R    = y
-//   Aout = Abase + cA * y
-//   Wout = cU * Wbase + cW * y
-// (each optional).  Wout must not alias lam: neighbours read lam.
+// Arguments of one fused adjoint RHS + RK stage launch: y = L^T lam (L the
+// Jacobian of the scalarwave1 DG RHS with respect to u), then R = y or Wout
+// as StageArgs' wmodes 1 and 3 to 6 with r = y and win = lam.  The RHS is
+// linear and the same at every stage, so the transpose of an RK step is that
+// RK step with L^T.  y_phi = 0 and y_pi has + lam_phi, which stays what it is
+// through a step: it is read from phi.  Wout must not alias lam: neighbours
+// read lam.
 struct AdjArgs {
-  const double *lam = nullptr;
-  const double *Abase = nullptr, *Wbase = nullptr;
-  double *Aout = nullptr, *Wout = nullptr, *R = nullptr;
-  double cA = 0, cU = 0, cW = 0;
+  const double *lam = nullptr, *phi = nullptr;
+  const double *U = nullptr, *Wa = nullptr, *Wb = nullptr;
+  double *Wout = nullptr, *R = nullptr;
+  double cA = 0, cW = 0;
+  int wmode = 0;
   const double *dXdx = nullptr, *dXbdX = nullptr, *egeo = nullptr, *xb = nullptr, *D = nullptr;
   const int *edom = nullptr;
   const int4 *face = nullptr;    // as StageArgs::face
@@ -79,9 +87,7 @@ struct DtArgs {
 int dt_grid(int nelem);
 hipError_t launch_dt(const DtArgs &a, int grid, hipStream_t s);
 
-// geom: 0 Cartesian, 1 stored dXdx, 2 CubedShell recomputed; nt from dg_stage_threads
-hipError_t launch_dg_stage(int np, int geom, const StageArgs &a, int grid, int nt, hipStream_t s);
-int dg_stage_threads(int np, int div);   // div: nodes per thread 1, 2 or 4
+// geom: 0 Cartesian, 1 stored dXdx, 2 CubedShell recomputed
 hipError_t launch_dg_adjoint(int np, int geom, const AdjArgs &a, int grid, hipStream_t s);
 // scalarwave1 on FV elements (fv_divf); rec: the interior scheme, 5 WENO5,
 // 7 WENO-Z, 9 WENOT, 3 WENOm3 (the end midpoints by StageArgs::recend);
