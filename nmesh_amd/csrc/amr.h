@@ -6,7 +6,8 @@ namespace nmx {
 
 // face interpolation job, kJobInts ints per (face, neighbour):
 //   [0] n (my points per direction), [1] m (neighbour's), [2] offset of the
-//   job's region in the face buffer ([v][n*n]), [3] 1, [4] base, [5] t1,
+//   job's region in the face buffer ([v][n*n]), [3] 16-bit reciprocals of n*n
+//   (low) and n (high), rounded up, [4] base, [5] t1,
 //   [6] t2 (neighbour plane node = base + q1*t1 + q2*t2 inside the
 //   neighbour), [7] swap, [8..11] a0,a1,b0,b1 covered point ranges, [12]
 //   offset of the rows for my a, [13] for my b, in Btab (rows of m doubles),

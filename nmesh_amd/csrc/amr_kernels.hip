@@ -24,15 +24,25 @@ namespace nmx {
 // one region per neighbour, averaged by the stage kernel.
 // The jobs are in the order of the elements whose planes they read, so the
 // lines of a plane normal to x (every line of the element's block) come from
-// HBM once.  19,200 elements of 4 to 10 points (100,318 jobs): 118 us.
+// HBM once, and four jobs, of which a CU mostly finds the plane in its L1, make
+// a workgroup (one wave per workgroup: the 100,318 jobs of 19,200 elements of 4
+// to 10 points take 118 us instead of 106, 276 MB fetched and 167 written).
 // ---------------------------------------------------------------------------
-constexpr int kFaceThreads = 64;
+constexpr int kFaceWaves = 4;   // jobs per workgroup
+
+// LDS written by some lanes of a wave, read by others of the same wave: the
+// wave's LDS instructions are done in order, so only the compiler has to keep
+// them so
+__device__ __forceinline__ void wave_lds_fence() {
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+}
 
 struct JobView {
-  int n, m, ajoff, nslot, base, t1, t2, sw, a0, a1, b0, b1, offA, offB;
+  int n, m, ajoff, inn, in, base, t1, t2, sw, a0, a1, b0, b1, offA, offB;
   long soff;
   __device__ JobView(const NMX_CONST int *j) {
-    n = j[0]; m = j[1]; ajoff = j[2]; nslot = j[3]; base = j[4]; t1 = j[5]; t2 = j[6];
+    n = j[0]; m = j[1]; ajoff = j[2]; inn = (unsigned)j[3] & 0xffff; in = (unsigned)j[3] >> 16; base = j[4]; t1 = j[5]; t2 = j[6];
     sw = j[7]; a0 = j[8]; a1 = j[9]; b0 = j[10]; b1 = j[11]; offA = j[12]; offB = j[13];
     soff = (long)(unsigned)j[14] | ((long)j[15] << 32);
   }
@@ -44,7 +54,12 @@ struct JobView {
 
 // One job with the neighbour's order M known at compile time: the loops
 // over its points are unrolled without branches, so the LDS reads of a row
-// are issued together instead of one round trip per term.
+// are issued together instead of one round trip per term.  The lanes of pass 2
+// take the face's points in order, whole lines of the face buffer at a time,
+// with their places from multiplications (divisions by n took a third of the
+// kernel's instructions; a lane per line of points instead of per point has
+// none, but writes every line in pieces: 138 us for the faces of 19,200
+// elements).
 template <int M>
 __device__ __forceinline__ void face_job(const FaceArgs &a, const JobView &J, int tid, double *s_T, double *s_R1,
                                          double *s_R2) {
@@ -62,12 +77,11 @@ __device__ __forceinline__ void face_job(const FaceArgs &a, const JobView &J, in
   double p[M];
 #pragma unroll
   for (int q1 = 0; q1 < M; ++q1) p[q1] = act ? P[q1 * J.t1] : 0.0;
-  __syncthreads();   // the previous face is done with LDS
   if (tid < n1) s_R1[tid] = r1a;
   if (tid + 64 < n1) s_R1[tid + 64] = r1b;
   if (tid < n2) s_R2[tid] = r2a;
   if (tid + 64 < n2) s_R2[tid + 64] = r2b;
-  __syncthreads();
+  wave_lds_fence();
   if (act) {
     double *T = s_T + v * nx1 * M + q2;
     for (int x = 0; x < nx1; ++x) {
@@ -78,60 +92,60 @@ __device__ __forceinline__ void face_job(const FaceArgs &a, const JobView &J, in
       T[x * M] = t;
     }
   }
-  __syncthreads();
+  wave_lds_fence();
   const int nn = n * n;
-  for (int idx = tid; idx < 4 * nn; idx += kFaceThreads) {
-    const int vv = idx / nn, q = idx % nn;
-    const int fa = q % n, fb = q / n;
-    double sum = 0.0;
+  double *out = a.aj + J.ajoff;
+  for (int idx = tid; idx < 4 * nn; idx += 64) {
+    // idx < 400 and n <= 10: exact quotients from 16-bit reciprocals
+    const int vv = (idx * J.inn) >> 16, q = idx - vv * nn;
+    const int fb = (q * J.in) >> 16, fa = q - fb * n;
+    double t = 0.0;
     if (fa >= J.a0 && fa <= J.a1 && fb >= J.b0 && fb <= J.b1) {
       const int x1 = (J.sw ? fb : fa) - J.x1lo(), x2 = (J.sw ? fa : fb) - J.x2lo();
       const double *T = s_T + (vv * nx1 + x1) * M;
       const double *row = s_R2 + x2 * M;
-      double sv = 0.0;
 #pragma unroll
-      for (int k = 0; k < M; ++k) sv += T[k] * row[k];
-      sum += sv;
+      for (int k = 0; k < M; ++k) t += T[k] * row[k];
     }
-    a.aj[J.ajoff + idx] = sum;
+    out[idx] = t;
   }
 }
 
-__global__ __launch_bounds__(kFaceThreads) void face_interp_kernel(FaceArgs a) {
-  __shared__ double s_T[kFaceT1];    // [v][x1][m]
-  __shared__ double s_R1[kFaceR1];   // [x1][m]
-  __shared__ double s_R2[kFaceR1];   // [x2][m]
-  const int tid = threadIdx.x;
-  const int xcd = blockIdx.x & 7, g8 = gridDim.x >> 3;
-  const int chunk = (a.nfaces + 7) >> 3;
-  const int f_hi = min((xcd + 1) * chunk, a.nfaces);
-  for (int fi = xcd * chunk + (blockIdx.x >> 3); fi < f_hi; fi += g8) {
-    const JobView J(as_const(a.jobs) + kJobInts * fi);
-    switch (J.m) {
-#define NMX_CASE(M_)                                   \
-  case M_:                                             \
-    face_job<M_>(a, J, tid, s_T, s_R1, s_R2);          \
+__global__ __launch_bounds__(64 * kFaceWaves) void face_interp_kernel(FaceArgs a) {
+  __shared__ double s_T[kFaceWaves][kFaceT1];    // [v][x1][m]
+  __shared__ double s_R1[kFaceWaves][kFaceR1];   // [x1][m]
+  __shared__ double s_R2[kFaceWaves][kFaceR1];   // [x2][m]
+  const int tid = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  // contiguous ranges of jobs per XCD, kFaceWaves of them per workgroup
+  const int chunk = (a.nfaces + 7) >> 3, q = kFaceWaves * (blockIdx.x >> 3) + wv;
+  const int fi = (blockIdx.x & 7) * chunk + q;
+  if (q >= chunk || fi >= a.nfaces) return;   // waves do not wait for one another
+  const JobView J(as_const(a.jobs) + kJobInts * fi);
+  switch (J.m) {
+#define NMX_CASE(M_)                                       \
+  case M_:                                                 \
+    face_job<M_>(a, J, tid, s_T[wv], s_R1[wv], s_R2[wv]);  \
     break;
-      NMX_CASE(2)
-      NMX_CASE(3)
-      NMX_CASE(4)
-      NMX_CASE(5)
-      NMX_CASE(6)
-      NMX_CASE(7)
-      NMX_CASE(8)
-      NMX_CASE(9)
-      NMX_CASE(10)
+    NMX_CASE(2)
+    NMX_CASE(3)
+    NMX_CASE(4)
+    NMX_CASE(5)
+    NMX_CASE(6)
+    NMX_CASE(7)
+    NMX_CASE(8)
+    NMX_CASE(9)
+    NMX_CASE(10)
 #undef NMX_CASE
-      default:
-        break;   // orders outside 2..10 are refused on the host
-    }
+    default:
+      break;   // orders outside 2..10 are refused on the host
   }
 }
 
 hipError_t launch_face_interp(const FaceArgs &a, hipStream_t s) {
   if (a.nfaces == 0) return hipSuccess;
-  const int grid = 8 * ((a.nfaces + 7) / 8);   // a multiple of 8 (XCD mapping)
-  hipLaunchKernelGGL(face_interp_kernel, dim3(grid), dim3(kFaceThreads), 0, s, a);
+  const int chunk = (a.nfaces + 7) / 8;
+  const int grid = 8 * ((chunk + kFaceWaves - 1) / kFaceWaves);
+  hipLaunchKernelGGL(face_interp_kernel, dim3(grid), dim3(64 * kFaceWaves), 0, s, a);
   return hipGetLastError();
 }
 

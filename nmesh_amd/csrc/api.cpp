@@ -753,7 +753,8 @@ static int upload_amr_tables(nmx_ctx *c) {
         if ((int)q.Ba.size() != n * m || (int)q.Bb.size() != n * m)
           return fail(NMX_EINVAL, "interpolation rows have the wrong size");
         int oa = brow(q.Ba), ob = brow(q.Bb);
-        int rec[kJobInts] = {n, m, (int)region, 1, (int)base, q.t1, q.t2, q.swap,
+        const int inv = (65535 / (n * n) + 1) | ((65535 / n + 1) << 16);
+        int rec[kJobInts] = {n, m, (int)region, inv, (int)base, q.t1, q.t2, q.swap,
                              q.a0, q.a1, q.b0, q.b1, oa, ob, 0, 0};
         const long so = soff[q.nb];
         std::memcpy(rec + 14, &so, sizeof(long));

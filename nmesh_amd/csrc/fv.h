@@ -15,11 +15,11 @@ struct FvGrid {
   double gam = 2.0;  // ideal-gas Gamma
 };
 
-// c2p of every cell: P = primitives of U, P's pressure as the Newton guess;
-// blocks whose solve fails get bad[b] = 1 (never cleared here)
+// c2p of every cell: P = primitives of U, guess's pressure as the Newton guess
+// (guess may be P); blocks whose solve fails get bad[b] = 1 (never cleared here)
 struct FvC2pArgs {
   FvGrid g;
-  const double *U = nullptr;
+  const double *U = nullptr, *guess = nullptr;
   double *P = nullptr;
   int *bad = nullptr;
   double tol = 1e-12;
@@ -27,14 +27,21 @@ struct FvC2pArgs {
 
 // fused RHS + RK stage on 8^3-cell tiles:
 //   r = -sum_d (F_{i+1/2} - F_{i-1/2}) from the primitives P (WENO5 + LLF)
-//   R = r; Aout = (Ain ? Ain : win) + cA r;
-//   Wout = U + cW r (wmode 1) or 0.75 U + 0.25 (win + cW r) (wmode 2)
+//   R = r and, by wmode,
+//   1: Wout = U + cW r
+//   2: Wout = 0.75 U + 0.25 (win + cW r)
+//   3: Wout = U + ((Wa - U) + 2 (Wb - U) + (win - U))/3 + cW r, the end of an
+//      RK4 step with the stage inputs Wa, Wb, win
+//   4: Wout = U + 2/3 ((win - U) + cW r), the end of an sspRK3 step
+// (the sum of the earlier stages' r recovered from their inputs; Wout may be
+// U), then Pout = the primitives of Wout, solved as c2p does from P's pressure
 struct FvStageArgs {
   FvGrid g;
   const double *P = nullptr;
-  const double *win = nullptr, *U = nullptr, *Ain = nullptr;
-  double *Aout = nullptr, *Wout = nullptr, *R = nullptr;
-  double cA = 0, cW = 0;
+  const double *win = nullptr, *U = nullptr, *Wa = nullptr, *Wb = nullptr;
+  double *Wout = nullptr, *R = nullptr, *Pout = nullptr;
+  int *bad = nullptr;
+  double cW = 0, tol = 1e-12;
   int wmode = 0;
   int xcd_map = 1;
 };

@@ -1,6 +1,6 @@
 // fv_api.cpp -- C ABI of the FV WENO5 + LLF path (include/nmx.h, nmx_fv_*):
 // a periodic grid of 16^3-cell blocks evolved with special-relativistic
-// Euler (ideal gas), c2p + fused RHS/stage kernels per RK stage, RK steps
+// Euler (ideal gas), one fused RHS/stage/c2p kernel per RK stage, RK steps
 // captured in hipGraphs.
 #include <hip/hip_runtime.h>
 
@@ -34,6 +34,7 @@ struct nmx_fv {
   hipGraphExec_t gexec = nullptr;
   int graph_steps = 0, graph_method = -1;
   double graph_dt = 0;
+  const double *graph_prim = nullptr;   // the captured steps' first primitives
   hipEvent_t ev0 = nullptr, ev1 = nullptr;
   double last_ms = 0;
 };
@@ -232,20 +233,27 @@ extern "C" int nmx_fv_download(nmx_fv *f, int which, double *h) {
   return NMX_OK;
 }
 
-// c2p of win into P, then the fused stage
-static int fv_launch(nmx_fv *f, FvStageArgs a) {
+// primitives of the conserved state U into P, the pressure guessed from dP
+static int fv_c2p(nmx_fv *f, const double *U, double *P_) {
   FvC2pArgs c;
   c.g = f->g;
-  c.U = a.win;
-  c.P = f->dP;
+  c.U = U;
+  c.guess = f->dP;
+  c.P = P_;
   c.bad = f->dbad;
   c.tol = std::atof(P(f, "fv_c2p_tol").c_str());
   hipError_t e = launch_fv_c2p(c, f->stream);
   if (e != hipSuccess) return fail(NMX_EHIP, std::string("c2p: ") + hipGetErrorString(e));
+  return NMX_OK;
+}
+
+// the fused stage from the primitives a.P
+static int fv_launch(nmx_fv *f, FvStageArgs a) {
   a.g = f->g;
-  a.P = f->dP;
+  a.bad = f->dbad;
+  a.tol = std::atof(P(f, "fv_c2p_tol").c_str());
   a.xcd_map = P(f, "nmx_xcd") == "yes" ? 1 : 0;
-  e = launch_fv_stage(a, f->stream);
+  hipError_t e = launch_fv_stage(a, f->stream);
   if (e != hipSuccess) return fail(NMX_EHIP, std::string("fv stage: ") + hipGetErrorString(e));
   return NMX_OK;
 }
@@ -253,14 +261,8 @@ static int fv_launch(nmx_fv *f, FvStageArgs a) {
 extern "C" int nmx_fv_max_speed(nmx_fv *f, double *amax) {
   NEED_GRID(f);
   if (!amax) return fail(NMX_EINVAL, "NULL argument");
-  FvC2pArgs c;
-  c.g = f->g;
-  c.U = f->dU;
-  c.P = f->dP;
-  c.bad = f->dbad;
-  c.tol = std::atof(P(f, "fv_c2p_tol").c_str());
-  hipError_t e = launch_fv_c2p(c, f->stream);
-  if (e != hipSuccess) return fail(NMX_EHIP, std::string("c2p: ") + hipGetErrorString(e));
+  if (int r = fv_c2p(f, f->dU, f->dP)) return r;
+  hipError_t e;
   const int grid = fv_speed_grid(f->g);
   double *part = nullptr;
   if (int r = dalloc(&part, (size_t)grid + 1)) return r;
@@ -274,7 +276,9 @@ extern "C" int nmx_fv_max_speed(nmx_fv *f, double *amax) {
 
 extern "C" int nmx_fv_setrhs(nmx_fv *f) {
   NEED_GRID(f);
+  if (int r = fv_c2p(f, f->dU, f->dP)) return r;
   FvStageArgs a;
+  a.P = f->dP;
   a.win = f->dU;
   a.R = f->dR;
   return fv_launch(f, a);
@@ -285,34 +289,37 @@ static int method_id(nmx_fv *f) {
   return m == "RK4" ? 0 : m == "sspRK3" ? 1 : 2;
 }
 
-// the stage sequences of evolve_RK4_mesh / evolve_sspRK3_mesh /
-// evolve_Euler_mesh (RungeKutta.c:19-188), as in the DG driver
-static int fv_issue_step(nmx_fv *f, int method, double dt, bool swap) {
-  double *U = swap ? f->dA : f->dU;
-  double *A = swap ? f->dU : f->dA;
+// The stage sequences of evolve_RK4_mesh / evolve_sspRK3_mesh /
+// evolve_Euler_mesh (RungeKutta.c:19-188), as in the DG driver: the stage
+// inputs are kept instead of an accumulator, RK4 and sspRK3 end in U, Euler
+// in the other register (swap).  The stages read their primitives from dP and
+// the scratch register dT in turn, first from *prim, and write the next
+// stage's into the other one; the last stage of the last step writes none, so
+// that the primitives stay those of the last stage's input.
+static int fv_issue_step(nmx_fv *f, int method, double dt, bool swap, bool last, double **prim) {
+  double *U = swap && method == 2 ? f->dA : f->dU;
   FvStageArgs a;
+  a.U = U;
+  auto stage = [&](const double *win, double *wout, int wmode, double cW, bool end) -> int {
+    a.win = win; a.Wout = wout; a.wmode = wmode; a.cW = cW;
+    a.P = *prim;
+    a.Pout = end && last ? nullptr : *prim == f->dP ? f->dT : f->dP;
+    if (a.Pout) *prim = a.Pout;
+    return fv_launch(f, a);
+  };
   int r;
   if (method == 0) {
-    a.win = U; a.U = U; a.Aout = A; a.cA = dt / 6.; a.Wout = f->dW0; a.wmode = 1; a.cW = dt / 2.;
-    if ((r = fv_launch(f, a))) return r;
-    a.win = f->dW0; a.Ain = A; a.cA = dt / 3.; a.Wout = f->dW1; a.cW = dt / 2.;
-    if ((r = fv_launch(f, a))) return r;
-    a.win = f->dW1; a.cA = dt / 3.; a.Wout = f->dW0; a.cW = dt;
-    if ((r = fv_launch(f, a))) return r;
-    a.win = f->dW0; a.cA = dt / 6.; a.Wout = nullptr; a.wmode = 0;
-    if ((r = fv_launch(f, a))) return r;
-  } else if (method == 1) {
-    a.win = U; a.U = U; a.Aout = A; a.cA = dt / 6.; a.Wout = f->dW0; a.wmode = 1; a.cW = dt;
-    if ((r = fv_launch(f, a))) return r;
-    a.win = f->dW0; a.Ain = A; a.cA = dt / 6.; a.Wout = f->dW1; a.wmode = 2; a.cW = dt;
-    if ((r = fv_launch(f, a))) return r;
-    a.win = f->dW1; a.cA = dt * 2. / 3.; a.Wout = nullptr; a.wmode = 0;
-    if ((r = fv_launch(f, a))) return r;
-  } else {
-    a.win = U; a.U = U; a.Aout = A; a.cA = dt; a.wmode = 0;
-    if ((r = fv_launch(f, a))) return r;
+    if ((r = stage(U, f->dW0, 1, dt / 2., false)) || (r = stage(f->dW0, f->dW1, 1, dt / 2., false)) ||
+        (r = stage(f->dW1, f->dA, 1, dt, false)))
+      return r;
+    a.Wa = f->dW0; a.Wb = f->dW1;
+    return stage(f->dA, U, 3, dt / 6., true);
   }
-  return NMX_OK;
+  if (method == 1) {
+    if ((r = stage(U, f->dW0, 1, dt, false)) || (r = stage(f->dW0, f->dW1, 2, dt, false))) return r;
+    return stage(f->dW1, U, 4, dt, true);
+  }
+  return stage(U, swap ? f->dU : f->dA, 1, dt, true);
 }
 
 extern "C" int nmx_fv_evolve(nmx_fv *f, int nsteps) {
@@ -328,13 +335,21 @@ extern "C" int nmx_fv_evolve(nmx_fv *f, int nsteps) {
   HIPCHK(hipEventRecord(f->ev0, f->stream));
   int done = 0;
   bool parity = false;
-  if (P(f, "nmx_graph") == "yes" && nsteps >= G) {
-    if (!f->gexec || f->graph_steps != G || f->graph_dt != dt || f->graph_method != method) {
+  // the first stage's primitives, into the register that leaves the last
+  // stage's in dP
+  const long stages = (long)nsteps * (method == 0 ? 4 : method == 1 ? 3 : 1);
+  double *prim = stages % 2 ? f->dP : f->dT;
+  if (nsteps > 0)
+    if (int r = fv_c2p(f, f->dU, prim)) return r;
+  // graphs hold G steps (an even number of stages), never the last one
+  if (P(f, "nmx_graph") == "yes" && nsteps > G) {
+    if (!f->gexec || f->graph_steps != G || f->graph_dt != dt || f->graph_method != method || f->graph_prim != prim) {
       if (f->gexec) { (void)hipGraphExecDestroy(f->gexec); f->gexec = nullptr; }
       if (f->graph) { (void)hipGraphDestroy(f->graph); f->graph = nullptr; }
       HIPCHK(hipStreamBeginCapture(f->stream, hipStreamCaptureModeThreadLocal));
       int r = NMX_OK;
-      for (int s = 0; s < G && !r; ++s) r = fv_issue_step(f, method, dt, (s & 1) != 0);
+      double *pr = prim;
+      for (int s = 0; s < G && !r; ++s) r = fv_issue_step(f, method, dt, (s & 1) != 0, false, &pr);
       hipGraph_t g = nullptr;
       hipError_t ec = hipStreamEndCapture(f->stream, &g);
       if (r || ec != hipSuccess) {
@@ -344,14 +359,14 @@ extern "C" int nmx_fv_evolve(nmx_fv *f, int nsteps) {
       }
       f->graph = g;
       HIPCHK(hipGraphInstantiate(&f->gexec, f->graph, nullptr, nullptr, 0));
-      f->graph_steps = G; f->graph_dt = dt; f->graph_method = method;
+      f->graph_steps = G; f->graph_dt = dt; f->graph_method = method; f->graph_prim = prim;
     }
-    for (; nsteps - done >= G; done += G) HIPCHK(hipGraphLaunch(f->gexec, f->stream));
+    for (; nsteps - done > G; done += G) HIPCHK(hipGraphLaunch(f->gexec, f->stream));
   }
   for (; done < nsteps; ++done) {
-    int r = fv_issue_step(f, method, dt, parity);
+    int r = fv_issue_step(f, method, dt, parity, done + 1 == nsteps, &prim);
     if (r) return r;
-    parity = !parity;
+    parity = parity != (method == 2);
   }
   if (parity) HIPCHK(hipMemcpyAsync(f->dU, f->dA, f->nstate * 8, hipMemcpyDeviceToDevice, f->stream));
   HIPCHK(hipEventRecord(f->ev1, f->stream));

@@ -1,22 +1,17 @@
 // fv_kernels.hip -- FV WENO5 + LLF for special-relativistic Euler (ideal
 // gas) on a periodic grid of 16^3-cell blocks, gfx950, FP64.
 //
-// Per RK stage:
-//   fv_c2p_kernel    primitives (rho, v, p) of every cell: Newton on the
-//                    pressure, guessed from the previous stage's value;
-//   fv_stage_kernel  one 64-lane workgroup per 8^3-cell tile: for each
-//                    direction a lane walks one line of the tile with a
-//                    six-cell register window of primitives, reconstructs
-//                    both face states with WENO5 (rec1d_p_WENO5 /
-//                    rec1d_m_WENO5 with uniform weights, rec1d.c:1190-1352,
-//                    u_scale = 1 as in fv.c:141), takes the LLF flux
-//                    (numflux1d.c:85-112) and accumulates the flux
-//                    difference of each cell in LDS; the epilogue applies the
-//                    RK stage combination (RungeKutta.c:19-188).
-// The WENO5 formulas are the reference's; two rearrangements save work: the
-// nonlinear weights are normalised with one division instead of four, and
-// the right-side smoothness indicators of a face are kept for the left side
-// of the next face, where the same stencils appear in the same roles.
+// fv_stage_kernel, once per RK stage: one 64-lane wave per 8^3-cell tile and
+// direction.  A lane walks one line of the tile along the direction with a
+// window of primitives in registers, reconstructs both face states with WENO5
+// (rec1d_p_WENO5 / rec1d_m_WENO5 with uniform weights, rec1d.c:1190-1352,
+// u_scale = 1 as in fv.c:141), takes the LLF flux (numflux1d.c:85-112) and
+// accumulates the flux difference of each cell in LDS; the epilogue applies
+// the RK stage combination (RungeKutta.c:19-188) and solves for the next
+// stage's primitives (rho, v, p): Newton on the pressure, guessed from this
+// stage's value.  fv_c2p_kernel does that solve alone, before the first stage.
+// The WENO5 formulas are the reference's in differences of neighbouring cells
+// (weno5_*, below).
 // The SR-Euler flux, eigenvalues and c2p are textbook (Marti & Mueller,
 // Living Rev. Relativ. 6 (2003) 7); the reference has no SR-Euler system.
 #include <hip/hip_runtime.h>
@@ -30,59 +25,57 @@ constexpr int kFvB = 16;                     // cells per block edge
 constexpr int kFvB3 = kFvB * kFvB * kFvB;
 constexpr int kFvT = 8;                      // cells per tile edge
 constexpr int kFvT3 = kFvT * kFvT * kFvT;
-constexpr double kWeno5Eps = 1e-40;
 constexpr int kC2pMaxIt = 100;
+// up to this many tiles a tile gets three waves (fv_stage_kernel): sspRK3 and
+// RK4 steps of 48^3 cells (216 tiles) take 107 us with three and 187 with one,
+// of 64^3 (512) 185 and 234, of 96^3 (1728) 622 and 611, of 256^3 6.21 and
+// 5.94 ms
+constexpr int kFvSplitTiles = 1024;
 
-// WENO5 smoothness indicators of a 3-cell stencil (x, y, z) by the position
-// of the midpoint it reconstructs: right end (role 0), centre (role 1), left
-// end (role 2); rec1d_p_WENO5 uses roles 0, 1, 2 on cells im-2.., im-1..,
-// im..; rec1d_m_WENO5 uses roles 0, 1, 2 on cells im-1.., im.., im+1..
-// (rec1d.c:1195-1300)
-__device__ __forceinline__ double beta_r0(double x, double y, double z) {
-  const double s1 = x - 2. * y + z, s2 = x - 4. * y + 3. * z;
-  return (13. / 12.) * s1 * s1 + 0.25 * s2 * s2;
-}
-__device__ __forceinline__ double beta_r1(double x, double y, double z) {
-  const double s1 = x - 2. * y + z, s2 = x - z;
-  return (13. / 12.) * s1 * s1 + 0.25 * s2 * s2;
-}
-__device__ __forceinline__ double beta_r2(double x, double y, double z) {
-  const double s1 = x - 2. * y + z, s2 = 3. * x - 4. * y + z;
-  return (13. / 12.) * s1 * s1 + 0.25 * s2 * s2;
-}
+// WENO5 in the differences h_k = (u[k+1] - u[k])/6 of neighbouring cells.  A
+// smoothness indicator of the stencil with differences (p, q) by the position
+// of the midpoint it reconstructs (right end: role 0, centre 1, left end 2;
+// rec1d.c:1195-1300) is 9 times
+//   13/3 (q - p)^2 + (3 q - p)^2, (p + q)^2 or (q - 3 p)^2,
+// and the weights depend only on the indicators' ratios, so the factor goes
+// into the epsilon (1e-40 over 9).  The first term is shared by the three
+// roles a stencil takes at successive midpoints; the squared indicators E of a
+// midpoint's right side are those of the next one's left side, so their
+// products are kept.  Normalised with one reciprocal: the weights g_k / E_k
+// over their sum equal g_k prod_{j != k} E_j over theirs (for the data here
+// every product stays between 1e-170 and 1e+60).
+constexpr double kWeno5Eps = 1e-40 / 9.;
 
-// Nonlinear combination with one reciprocal: the weights g_k / (beta_k +
-// eps)^2 normalised equal  g_k prod_{j != k} (beta_j + eps)^2  normalised
-// (for the data here every product stays between 1e-240 and 1e+60, so the
-// sum is a normal number for rcp_nr, fastmath.h).
-__device__ __forceinline__ double weno5_combine(double g0, double g1, double g2, double b0, double b1,
-                                                double b2, double q0, double q1, double q2) {
-  const double e0 = b0 + kWeno5Eps, e1 = b1 + kWeno5Eps, e2 = b2 + kWeno5Eps;
-  const double E0 = e0 * e0, E1 = e1 * e1, E2 = e2 * e2;
-  const double A0 = g0 * (E1 * E2), A1 = g1 * (E0 * E2), A2 = g2 * (E0 * E1);
-  return (A0 * q0 + A1 * q1 + A2 * q2) * rcp_nr(A0 + A1 + A2);
+__device__ __forceinline__ double weno_curv(double p, double q) {
+  const double s = q - p;
+  return fma(13. / 3. * s, s, kWeno5Eps);
 }
-
-// midpoint from the left over (a, b, c, d, e) = u[im-2 .. im+2], ideal
-// weights (1, 6, 3), stencils (2,-7,11)/6, (-1,5,2)/6, (2,5,-1)/6
-__device__ __forceinline__ double weno5_p(double a, double b, double c, double d, double e, double b0,
-                                          double b1, double b2) {
-  const double o6 = 1. / 6.;
-  const double q0 = (2. * o6) * a + (-7. * o6) * b + (11. * o6) * c;
-  const double q1 = (-o6) * b + (5. * o6) * c + (2. * o6) * d;
-  const double q2 = (2. * o6) * c + (5. * o6) * d + (-o6) * e;
-  return weno5_combine(1., 6., 3., b0, b1, b2, q0, q1, q2);
+// the products E1 E2, 6 E0 E2, E0 E1 of the stencils (h0, h1), (h1, h2), (h2,
+// h3) with curvature terms c0, c1, c2
+__device__ __forceinline__ void weno_products(double h0, double h1, double h2, double h3, double c0, double c1,
+                                              double c2, double (&E)[3]) {
+  const double s0 = fma(3., h1, -h0), s1 = h1 + h2, s2 = fma(-3., h2, h3);
+  double e0 = fma(s0, s0, c0), e1 = fma(s1, s1, c1), e2 = fma(s2, s2, c2);
+  e0 *= e0; e1 *= e1; e2 *= e2;
+  E[0] = e1 * e2;
+  E[1] = 6. * (e0 * e2);
+  E[2] = e0 * e1;
 }
-
-// midpoint from the right over (a, b, c, d, e) = u[im-1 .. im+3], ideal
-// weights (3, 6, 1) on the stencils starting at im-1, im, im+1
-__device__ __forceinline__ double weno5_m(double a, double b, double c, double d, double e, double b0,
-                                          double b1, double b2) {
-  const double o6 = 1. / 6.;
-  const double q2 = (11. * o6) * c + (-7. * o6) * d + (2. * o6) * e;
-  const double q1 = (2. * o6) * b + (5. * o6) * c + (-o6) * d;
-  const double q0 = (-o6) * a + (5. * o6) * b + (2. * o6) * c;
-  return weno5_combine(3., 6., 1., b0, b1, b2, q0, q1, q2);
+// midpoint right of u from its left side: ideal weights (1, 6, 3), h0 .. h3
+// the differences from two cells left of u on
+__device__ __forceinline__ double weno_left(double u, double h0, double h1, double h2, double h3,
+                                            const double (&E)[3]) {
+  const double E2 = 3. * E[2];
+  const double q = E[0] * fma(5., h1, -2. * h0) + E[1] * fma(2., h2, h1) + E2 * fma(4., h2, -h3);
+  return fma(q, rcp_nr(E[0] + E[1] + E2), u);
+}
+// midpoint left of u from its right side: ideal weights (3, 6, 1), h1 .. h4
+// the differences from two cells left of u on
+__device__ __forceinline__ double weno_right(double u, double h1, double h2, double h3, double h4,
+                                             const double (&E)[3]) {
+  const double E0 = 3. * E[0];
+  const double q = E0 * fma(-4., h2, h1) - E[1] * fma(2., h2, h3) + E[2] * fma(2., h4, -5. * h3);
+  return fma(q, rcp_nr(E0 + E[1] + E[2]), u);
 }
 
 __device__ __forceinline__ void sr_p2c(double gam, const double P[5], double U[5]) {
@@ -98,85 +91,83 @@ __device__ __forceinline__ void sr_p2c(double gam, const double P[5], double U[5
   U[4] = rhW2 - p - U[0];
 }
 
-// flux along DIR, conserved state, and max |acoustic eigenvalue|;
-// g1 = gam / (gam - 1)
-template <int DIR>
-__device__ __forceinline__ double sr_flux(double gam, double g1, const double P[5], double F[5], double U[5]) {
-  const double rho = P[0], vx = P[1], vy = P[2], vz = P[3], p = P[4];
-  const double v2 = vx * vx + vy * vy + vz * vz;
-  const double W = rsqrt_nr(1. - v2);
-  const double ph = p * rcp_nr(rho);
-  const double h = 1. + g1 * ph;
-  const double rhW2 = rho * h * W * W;
-  U[0] = rho * W;
-  U[1] = rhW2 * vx;
-  U[2] = rhW2 * vy;
-  U[3] = rhW2 * vz;
-  U[4] = rhW2 - p - U[0];
-  const double vd = P[1 + DIR];
-  F[0] = U[0] * vd;
-  F[1] = U[1] * vd;
-  F[2] = U[2] * vd;
-  F[3] = U[3] * vd;
-  F[1 + DIR] += p;
-  F[4] = (U[4] + p) * vd;
-  const double cs2 = gam * ph * rcp_nr(h);
-  const double cs = sqrt(cs2);
-  const double oden = rcp_nr(1. - v2 * cs2);
-  const double root = cs * sqrt((1. - v2) * (1. - v2 * cs2 - vd * vd * (1. - cs2)));
-  const double lm = (vd * (1. - cs2) - root) * oden;
-  const double lp = (vd * (1. - cs2) + root) * oden;
-  return fmax(fabs(lm), fabs(lp));
+// flux along the normal, conserved state and max |acoustic eigenvalue| of P =
+// (rho, v_n, v_t, v_t', p); v2 = v^2, g1 = gam / (gam - 1).  With w = rho h =
+// rho + g1 p and a = gam p (c_s^2 = a / w) the eigenvalues
+//   (v_n (1 - c_s^2) +- c_s sqrt((1 - v2) (1 - v2 c_s^2 - v_n^2 (1 - c_s^2)))) / (1 - v2 c_s^2)
+// become (v_n (w - a) +- sqrt(a (1 - v2) (w - v2 a - v_n^2 (w - a)))) / (w - v2 a).
+__device__ __forceinline__ double sr_flux(double gam, double g1, const double P[5], double v2, double F[5],
+                                          double U[5]) {
+  const double rho = P[0], vn = P[1], p = P[4];
+  const double iW2 = 1. - v2;
+  const double W = rsqrt_nr(iW2);
+  const double w = fma(g1, p, rho);
+  const double D = rho * W, q = w * (W * W), t = q - D;
+  U[0] = D;
+  U[1] = q * vn;
+  U[2] = q * P[2];
+  U[3] = q * P[3];
+  U[4] = t - p;
+  F[0] = D * vn;
+  F[1] = fma(U[1], vn, p);
+  F[2] = U[2] * vn;
+  F[3] = U[3] * vn;
+  F[4] = t * vn;
+  const double a = gam * p, wa = w - a, den = fma(-v2, a, w);
+  const double rad = a * iW2 * fma(-vn * vn, wa, den);
+  const double root = rad * rsqrt_nr(rad + 1e-300);   // 0 at 0
+  return fma(fabs(vn), wa, root) * rcp_nr(den);
 }
 
-__device__ __forceinline__ bool physical(const double P[5]) {
-  const double v2 = P[1] * P[1] + P[2] * P[2] + P[3] * P[3];
-  return P[0] > 0. && P[4] > 0. && v2 < 1.;
-}
+__device__ __forceinline__ double speed2(const double P[5]) { return P[1] * P[1] + P[2] * P[2] + P[3] * P[3]; }
 
 // ---------------------------------------------------------------------------
 // c2p
 // ---------------------------------------------------------------------------
 
+// primitives of U, p the pressure guess; false if Newton did not converge
+__device__ __forceinline__ bool sr_c2p(double gam, double tol, const double U[5], double p, double P[5]) {
+  const double D = U[0], E = U[4] + D;
+  const double S2 = U[1] * U[1] + U[2] * U[2] + U[3] * U[3];
+  const double pmin = fmax(sqrt(S2) - E, 0.0);
+  if (!(p > pmin)) p = pmin + 1e-10 * E;
+  int it;
+  // (the reciprocals and 1/sqrt by rcp_nr / rsqrt_nr: 1/W = (1 - v^2) W)
+  for (it = 1; it <= kC2pMaxIt; ++it) {
+    const double iEp = rcp_nr(E + p);
+    const double v2 = S2 * iEp * iEp;
+    const double W = rsqrt_nr(1. - v2);
+    const double iW = (1. - v2) * W;
+    const double f = (gam - 1.) * (E - S2 * iEp - D * iW) - p;
+    const double df = (gam - 1.) * v2 * (1. - D * W * iEp) - 1.;
+    double pn = p - f * rcp_nr(df);
+    if (pn <= pmin) pn = 0.5 * (p + pmin);
+    const double dp = fabs(pn - p);
+    p = pn;
+    if (dp <= tol * p) break;
+  }
+  const double iEp = rcp_nr(E + p);
+  const double v2 = S2 * iEp * iEp;
+  const double iW = (1. - v2) * rsqrt_nr(1. - v2);
+  P[0] = D * iW;
+  P[1] = U[1] * iEp;
+  P[2] = U[2] * iEp;
+  P[3] = U[3] * iEp;
+  P[4] = p;
+  return it <= kC2pMaxIt;
+}
+
 __global__ __launch_bounds__(256) void fv_c2p_kernel(FvC2pArgs a) {
   const long ncell = (long)a.g.nbx * a.g.nbx * a.g.nbx * kFvB3;
-  const double gam = a.g.gam;
   for (long c = (long)blockIdx.x * blockDim.x + threadIdx.x; c < ncell; c += (long)gridDim.x * blockDim.x) {
     const long b = c / kFvB3, q = c % kFvB3;
     const long base = b * 5 * kFvB3 + q;
-    const double D = a.U[base], Sx = a.U[base + kFvB3], Sy = a.U[base + 2 * kFvB3],
-                 Sz = a.U[base + 3 * kFvB3];
-    const double E = a.U[base + 4 * kFvB3] + D;
-    const double S2 = Sx * Sx + Sy * Sy + Sz * Sz;
-    const double pmin = fmax(sqrt(S2) - E, 0.0);
-    double p = a.P[base + 4 * kFvB3];
-    if (!(p > pmin)) p = pmin + 1e-10 * E;
-    int it;
-    // (the reciprocals and 1/sqrt by rcp_nr / rsqrt_nr: 1/W = (1 - v^2) W)
-    for (it = 1; it <= kC2pMaxIt; ++it) {
-      const double Ep = E + p;
-      const double iEp = rcp_nr(Ep);
-      const double v2 = S2 * iEp * iEp;
-      const double W = rsqrt_nr(1. - v2);
-      const double iW = (1. - v2) * W;
-      const double f = (gam - 1.) * (E - S2 * iEp - D * iW) - p;
-      const double df = (gam - 1.) * v2 * (1. - D * W * iEp) - 1.;
-      double pn = p - f * rcp_nr(df);
-      if (pn <= pmin) pn = 0.5 * (p + pmin);
-      const double dp = fabs(pn - p);
-      p = pn;
-      if (dp <= a.tol * p) break;
-    }
-    if (it > kC2pMaxIt) a.bad[b] = 1;
-    const double Ep = E + p;
-    const double iEp = rcp_nr(Ep);
-    const double v2 = S2 * iEp * iEp;
-    const double iW = (1. - v2) * rsqrt_nr(1. - v2);
-    a.P[base] = D * iW;
-    a.P[base + kFvB3] = Sx * iEp;
-    a.P[base + 2 * kFvB3] = Sy * iEp;
-    a.P[base + 3 * kFvB3] = Sz * iEp;
-    a.P[base + 4 * kFvB3] = p;
+    double U[5], P[5];
+#pragma unroll
+    for (int v = 0; v < 5; ++v) U[v] = a.U[base + v * kFvB3];
+    if (!sr_c2p(a.g.gam, a.tol, U, a.guess[base + 4 * kFvB3], P)) a.bad[b] = 1;
+#pragma unroll
+    for (int v = 0; v < 5; ++v) a.P[base + v * kFvB3] = P[v];
   }
 }
 
@@ -238,102 +229,109 @@ hipError_t launch_fv_layout(const FvGrid &g, const double *src, double *dst, int
 // fused RHS + RK stage on 8^3 tiles
 // ---------------------------------------------------------------------------
 
-// address of primitive v at global cell (x, y, z), periodic
-__device__ __forceinline__ long prim_addr(int nbx, int N, int x, int y, int z) {
-  x = x < 0 ? x + N : (x >= N ? x - N : x);
-  y = y < 0 ? y + N : (y >= N ? y - N : y);
-  z = z < 0 ? z + N : (z >= N ? z - N : z);
-  const long b = (x >> 4) + (long)nbx * ((y >> 4) + (long)nbx * (z >> 4));
-  return b * 5 * kFvB3 + ((x & 15) + kFvB * ((y & 15) + kFvB * (z & 15)));
+// Cell (cx, cy, cz) of a tile in the accumulator: rows along x, permuted so
+// that the lanes of a sweep along x, y or z (8 x 8 of the other two) spread
+// over the banks.
+__device__ __forceinline__ int acc_cell(int cx, int cy, int cz) {
+  return (cx ^ cz) + kFvT * (((cy + cz) & (kFvT - 1)) + kFvT * cz);
 }
 
-template <int DIR>
-__device__ __forceinline__ void load_cell(const FvStageArgs &a, int N, int x0, int y0, int z0, int ta, int tb,
-                                          int s, double out[5]) {
-  const int x = x0 + (DIR == 0 ? s : ta);
-  const int y = y0 + (DIR == 1 ? s : (DIR == 0 ? ta : tb));
-  const int z = z0 + (DIR == 2 ? s : tb);
-  const double *p = a.P + prim_addr(a.g.nbx, N, x, y, z);
-#pragma unroll
-  for (int v = 0; v < 5; ++v) out[v] = p[v * kFvB3];
-}
-
-// one direction: lane (ta, tb) walks the tile line along DIR; FIRST writes
-// the accumulator, later directions add to it
-template <int DIR, bool FIRST>
-__device__ __forceinline__ void fv_sweep(const FvStageArgs &a, int N, int x0, int y0, int z0,
+// One direction d of the tile at block (bx, by, bz), cells t[0..2] on of it:
+// lane (ta, tb) walks the tile line along d.  FIRST writes the accumulator
+// (twice the flux difference), later directions add to it.  The code is the
+// same for the three directions (velocities are held as normal and tangential
+// ones), so that it can be unrolled over the line's 9 faces: the windows then
+// move through registers without copies.
+// STAGED (d = 0): the tile's own cells come from the accumulator, where the
+// caller has put them; a lane reads a cell before it writes the difference there.
+template <bool FIRST, bool STAGED>
+__device__ __forceinline__ void fv_sweep(const FvStageArgs &a, int d, const int (&bl)[3], const int (&t)[3],
                                          double (*acc)[kFvT3]) {
-  const int lane = threadIdx.x;
+  const int lane = threadIdx.x & 63;
   const int ta = lane % kFvT, tb = lane / kFvT;
-  const double gam = a.g.gam;
-  double q[5][6], nx[5];
-  {
-    double t[5];
+  const double gam = a.g.gam, g1 = gam / (gam - 1.);
+  const int nbx = a.g.nbx;
+  // Along d the tile's 8 cells lie in its own block, and so do the 3 cells
+  // beyond one of its ends; the 3 beyond the other end lie in the next block
+  // (or the one before).  Cell s of the line: base(s) + off + s * st.
+  const int st = d == 0 ? 1 : d == 1 ? kFvB : kFvB * kFvB;
+  auto block = [&](int shift) {
+    int c[3] = {bl[0], bl[1], bl[2]};
+    c[d] += shift;
+    c[d] = c[d] < 0 ? nbx - 1 : c[d] >= nbx ? 0 : c[d];
+    return a.P + (c[0] + (long)nbx * (c[1] + (long)nbx * c[2])) * (5L * kFvB3);
+  };
+  const bool upper = t[d] != 0;   // the tile is the upper half of its block along d
+  const double *own = block(0);
+  const double *lo = upper ? own : block(-1) + kFvB * st;
+  const double *hi = upper ? block(1) - kFvB * st : own;
+  const int off = (t[0] + (d == 0 ? 0 : ta)) + kFvB * ((t[1] + (d == 1 ? 0 : d == 0 ? ta : tb)) +
+                                                        kFvB * (t[2] + (d == 2 ? 0 : tb)));
+  // variables held as (rho, v_n, v_t, v_t', p)
+  const int d1 = d == 2 ? 0 : d + 1, d2 = d == 0 ? 2 : d - 1;
+  const int vi[5] = {0, 1 + d, 1 + d1, 1 + d2, 4};
+  // cells f .. f + 5 (counted from 3 before the tile) surround face f
+  double u[5][kFvT + 6], h[5][kFvT + 5], c[5][kFvT + 4], E[5][3];
+  auto load = [&](int k) {
+    const int s = k - 3;
+    if (STAGED && s >= 0 && s < kFvT) {
 #pragma unroll
-    for (int s = 0; s < 6; ++s) {
-      load_cell<DIR>(a, N, x0, y0, z0, ta, tb, s - 3, t);
-#pragma unroll
-      for (int v = 0; v < 5; ++v) q[v][s] = t[v];
+      for (int v = 0; v < 5; ++v) u[v][k] = acc[v][acc_cell(s, ta, tb)];
+      return;
     }
-    load_cell<DIR>(a, N, x0, y0, z0, ta, tb, 3, nx);
-  }
-  // right-side smoothness indicators of the previous face = left-side ones
-  // of this face (same stencils, same roles)
-  double bm[5][3];
+    const double *p = (s < 0 ? lo : s < kFvT ? own : hi) + s * st;
+#pragma unroll
+    for (int v = 0; v < 5; ++v) u[v][k] = (p + vi[v] * kFvB3)[off];
+  };
+#pragma unroll
+  for (int k = 0; k < 7; ++k) load(k);
 #pragma unroll
   for (int v = 0; v < 5; ++v) {
-    bm[v][0] = beta_r0(q[v][0], q[v][1], q[v][2]);
-    bm[v][1] = beta_r1(q[v][1], q[v][2], q[v][3]);
-    bm[v][2] = beta_r2(q[v][2], q[v][3], q[v][4]);
+#pragma unroll
+    for (int k = 0; k < 4; ++k) h[v][k] = (u[v][k + 1] - u[v][k]) * (1. / 6.);
+#pragma unroll
+    for (int k = 0; k < 3; ++k) c[v][k] = weno_curv(h[v][k], h[v][k + 1]);
+    weno_products(h[v][0], h[v][1], h[v][2], h[v][3], c[v][0], c[v][1], c[v][2], E[v]);
   }
-  const double g1 = gam / (gam - 1.);
-  double Fprev[5] = {0, 0, 0, 0, 0};
-#pragma unroll 1
+  double Fprev[5];
+#pragma unroll
   for (int f = 0; f <= kFvT; ++f) {   // face between tile cells f-1 and f
-    if (f > 0) {
-#pragma unroll
-      for (int v = 0; v < 5; ++v) {
-#pragma unroll
-        for (int s = 0; s < 5; ++s) q[v][s] = q[v][s + 1];
-        q[v][5] = nx[v];
-      }
-      if (f < kFvT) load_cell<DIR>(a, N, x0, y0, z0, ta, tb, f + 3, nx);
-    }
+    if (f + 7 < kFvT + 6) load(f + 7);
     double PL[5], PR[5];
 #pragma unroll
     for (int v = 0; v < 5; ++v) {
-      const double bp0 = bm[v][0], bp1 = bm[v][1], bp2 = bm[v][2];
-      bm[v][0] = beta_r0(q[v][1], q[v][2], q[v][3]);
-      bm[v][1] = beta_r1(q[v][2], q[v][3], q[v][4]);
-      bm[v][2] = beta_r2(q[v][3], q[v][4], q[v][5]);
-      PL[v] = weno5_p(q[v][0], q[v][1], q[v][2], q[v][3], q[v][4], bp0, bp1, bp2);
-      PR[v] = weno5_m(q[v][1], q[v][2], q[v][3], q[v][4], q[v][5], bm[v][0], bm[v][1], bm[v][2]);
+      const double *q = h[v] + f;
+      PL[v] = weno_left(u[v][f + 2], q[0], q[1], q[2], q[3], E[v]);
+      h[v][f + 4] = (u[v][f + 5] - u[v][f + 4]) * (1. / 6.);
+      c[v][f + 3] = weno_curv(h[v][f + 3], h[v][f + 4]);
+      weno_products(q[1], q[2], q[3], q[4], c[v][f + 1], c[v][f + 2], c[v][f + 3], E[v]);
+      PR[v] = weno_right(u[v][f + 3], q[1], q[2], q[3], q[4], E[v]);
     }
-    if (!physical(PL)) {
+    // unphysical face states fall back to the cell's
+    double vL = speed2(PL), vR = speed2(PR);
+    if (!(PL[0] > 0. && PL[4] > 0. && vL < 1.)) {
 #pragma unroll
-      for (int v = 0; v < 5; ++v) PL[v] = q[v][2];
+      for (int v = 0; v < 5; ++v) PL[v] = u[v][f + 2];
+      vL = speed2(PL);
     }
-    if (!physical(PR)) {
+    if (!(PR[0] > 0. && PR[4] > 0. && vR < 1.)) {
 #pragma unroll
-      for (int v = 0; v < 5; ++v) PR[v] = q[v][3];
+      for (int v = 0; v < 5; ++v) PR[v] = u[v][f + 3];
+      vR = speed2(PR);
     }
-    double FL[5], FR[5], UL[5], UR[5];
-    const double aL = sr_flux<DIR>(gam, g1, PL, FL, UL);
-    const double aR = sr_flux<DIR>(gam, g1, PR, FR, UR);
+    double FL[5], FR[5], UL[5], UR[5], F[5];
+    const double aL = sr_flux(gam, g1, PL, vL, FL, UL);
+    const double aR = sr_flux(gam, g1, PR, vR, FR, UR);
     const double am = fmax(aL, aR);
-    double F[5];
 #pragma unroll
-    for (int v = 0; v < 5; ++v) F[v] = 0.5 * (FL[v] + FR[v] - am * (UR[v] - UL[v]));
+    for (int v = 0; v < 5; ++v) F[v] = fma(-am, UR[v] - UL[v], FL[v] + FR[v]);   // twice the flux
     if (f > 0) {
       const int s = f - 1;
-      const int cx = DIR == 0 ? s : ta;
-      const int cy = DIR == 1 ? s : (DIR == 0 ? ta : tb);
-      const int cz = DIR == 2 ? s : tb;
-      const int cell = cx + kFvT * (cy + kFvT * cz);
+      const int cell = d == 0 ? acc_cell(s, ta, tb) : d == 1 ? acc_cell(ta, s, tb) : acc_cell(ta, tb, s);
 #pragma unroll
       for (int v = 0; v < 5; ++v) {
-        if (FIRST) acc[v][cell] = Fprev[v] - F[v];
-        else acc[v][cell] += Fprev[v] - F[v];
+        if (FIRST) acc[vi[v]][cell] = Fprev[v] - F[v];
+        else acc[vi[v]][cell] += Fprev[v] - F[v];
       }
     }
 #pragma unroll
@@ -341,70 +339,118 @@ __device__ __forceinline__ void fv_sweep(const FvStageArgs &a, int N, int x0, in
   }
 }
 
-__global__ __launch_bounds__(64, 2) void fv_stage_kernel(FvStageArgs a) {
-  __shared__ double acc[5][kFvT3];
-  const int nbx = a.g.nbx, N = nbx * kFvB;
+// W waves per tile: 1, or 3 with one direction each, which finish a tile of a
+// small grid in about a third of the time.  The accumulators take 20 KB per
+// wave: 8 waves per CU, two per SIMD, which is also what 246 VGPRs allow.
+// 256^3 cells take 1.36 ms per stage, primitives included, at 36 TFLOP/s
+// counted by instructions (13,290 VALU instructions per tile, 86% of them FP64;
+// VALU 60% busy, the rest waits on memory and issue).  Weights and fluxes
+// as they stood, by cell values with two IEEE square roots per state, windows
+// moved by copies and the primitives in a launch of their own, took 2.09 ms.
+// The line's 9 faces are unrolled: 61 KB of code, of the 64 KB that two CUs
+// share.  One copy of the sweep for all directions, a nontemporal epilogue and
+// tiles in 2^3-block bricks measured no faster (5.5% slower, and within 0.5%).
+template <int W>
+__global__ __launch_bounds__(64 * W, 2) void fv_stage_kernel(FvStageArgs a) {
+  __shared__ double acc[W][5][kFvT3];
+  const int nbx = a.g.nbx;
   const int ntiles = nbx * nbx * nbx * 8;
-  int t_hi, t_step, t_first;
+  int tile = blockIdx.x;
   if (a.xcd_map) {
-    const int xcd = blockIdx.x & 7, g8 = gridDim.x >> 3;
-    const int chunk = (ntiles + 7) >> 3;
-    t_first = xcd * chunk + (blockIdx.x >> 3);
-    t_hi = min((xcd + 1) * chunk, ntiles);
-    t_step = g8;
-  } else {
-    t_first = blockIdx.x;
-    t_hi = ntiles;
-    t_step = gridDim.x;
+    const int chunk = (ntiles + 7) >> 3, q = blockIdx.x >> 3;
+    tile = q < chunk ? (blockIdx.x & 7) * chunk + q : ntiles;
   }
-  for (int t = t_first; t < t_hi; t += t_step) {
-    const int b = t >> 3, sub = t & 7;
-    const int bx = b % nbx, by = (b / nbx) % nbx, bz = b / (nbx * nbx);
-    const int x0 = bx * kFvB + (sub & 1) * kFvT;
-    const int y0 = by * kFvB + ((sub >> 1) & 1) * kFvT;
-    const int z0 = bz * kFvB + (sub >> 2) * kFvT;
+  if (tile >= ntiles) return;
+  const int b = tile >> 3, sub = tile & 7;
+  const int bl[3] = {b % nbx, (b / nbx) % nbx, b / (nbx * nbx)};
+  const int t[3] = {(sub & 1) * kFvT, ((sub >> 1) & 1) * kFvT, (sub >> 2) * kFvT};
+  const int tid = threadIdx.x;
+  if (W == 1) {
+    // Along x the lanes' lines lie 128 bytes apart, so that each load of the
+    // sweep would fetch 64 lines for 8 bytes of each, more than the L1 keeps:
+    // the tile's own cells go through LDS, in the accumulator.
+    const double *own = a.P + (long)b * 5 * kFvB3 + t[0] + kFvB * (t[1] + kFvB * t[2]);
+    const int cx = tid % kFvT, cy = tid / kFvT;
+#pragma unroll
+    for (int v = 0; v < 5; ++v)
+#pragma unroll
+      for (int cz = 0; cz < kFvT; ++cz)
+        acc[0][v][acc_cell(cx, cy, cz)] = own[v * kFvB3 + cx + kFvB * (cy + kFvB * cz)];
     __syncthreads();
-    fv_sweep<0, true>(a, N, x0, y0, z0, acc);
+    fv_sweep<true, true>(a, 0, bl, t, acc[0]);
     __syncthreads();
-    fv_sweep<1, false>(a, N, x0, y0, z0, acc);
-    __syncthreads();
-    fv_sweep<2, false>(a, N, x0, y0, z0, acc);
-    __syncthreads();
-    // stage combination, 8 cells per lane
-    const int lane = threadIdx.x;
-    const int cx = lane % kFvT, cy = lane / kFvT;
 #pragma unroll 1
-    for (int cz = 0; cz < kFvT; ++cz) {
-      const int cell = cx + kFvT * (cy + kFvT * cz);
-      const long gi = (long)b * 5 * kFvB3 + ((x0 & 15) + cx) + kFvB * (((y0 & 15) + cy) + kFvB * ((z0 & 15) + cz));
-      double r[5], Ubuf[5], Abuf[5];
+    for (int d = 1; d < 3; ++d) {
+      fv_sweep<false, false>(a, d, bl, t, acc[0]);
+      __syncthreads();
+    }
+  } else {
+    const int d = __builtin_amdgcn_readfirstlane(tid >> 6);
+    fv_sweep<true, false>(a, d, bl, t, acc[d]);
+    __syncthreads();
+  }
+  // stage combination and the next primitives, the next cell's registers
+  // requested while this one's primitives are solved for
+  const long g0 = (long)b * 5 * kFvB3 + t[0] + kFvB * (t[1] + kFvB * t[2]);
+  auto place = [&](int cell) {
+    return g0 + cell % kFvT + kFvB * ((cell / kFvT) % kFvT + kFvB * (cell / (kFvT * kFvT)));
+  };
+  struct Regs {
+    double U[5], w[5], Wa[5], Wb[5], p;
+  } in;
+  auto request = [&](int cell) {
+    const long gi = place(cell);
 #pragma unroll
-      for (int v = 0; v < 5; ++v) r[v] = acc[v][cell];
-      if (a.wmode) {
+    for (int v = 0; v < 5; ++v) in.U[v] = a.U[gi + v * kFvB3];
+    if (a.wmode > 1) {
 #pragma unroll
-        for (int v = 0; v < 5; ++v) Ubuf[v] = a.U[gi + v * kFvB3];
+      for (int v = 0; v < 5; ++v) in.w[v] = a.win[gi + v * kFvB3];
+    }
+    if (a.wmode == 3) {
+#pragma unroll
+      for (int v = 0; v < 5; ++v) {
+        in.Wa[v] = a.Wa[gi + v * kFvB3];
+        in.Wb[v] = a.Wb[gi + v * kFvB3];
       }
-      if (a.Aout) {
-        const double *bas = a.Ain ? a.Ain : a.win;
+    }
+    if (a.Pout) in.p = a.P[gi + 4 * kFvB3];
+  };
+  if (a.Wout) request(tid);
+#pragma unroll 1
+  for (int cell = tid; cell < kFvT3; cell += 64 * W) {
+    const int ac = acc_cell(cell % kFvT, (cell / kFvT) % kFvT, cell / (kFvT * kFvT));
+    const long gi = place(cell);
+    double r[5], out[5];
 #pragma unroll
-        for (int v = 0; v < 5; ++v) Abuf[v] = bas[gi + v * kFvB3];
-      }
-      if (a.R) {
+    for (int v = 0; v < 5; ++v) {
+      double s = acc[0][v][ac];
+      if (W == 3) s = (s + acc[1][v][ac]) + acc[2][v][ac];
+      r[v] = 0.5 * s;
+    }
+    if (a.R) {
 #pragma unroll
-        for (int v = 0; v < 5; ++v) a.R[gi + v * kFvB3] = r[v];
-      }
-      if (a.Aout) {
+      for (int v = 0; v < 5; ++v) a.R[gi + v * kFvB3] = r[v];
+    }
+    if (!a.Wout) continue;
 #pragma unroll
-        for (int v = 0; v < 5; ++v) a.Aout[gi + v * kFvB3] = Abuf[v] + a.cA * r[v];
-      }
-      if (a.wmode == 1) {
+    for (int v = 0; v < 5; ++v) {
+      const double U = in.U[v];
+      if (a.wmode == 1) out[v] = U + a.cW * r[v];
+      else if (a.wmode == 2) out[v] = 0.75 * U + 0.25 * (in.w[v] + a.cW * r[v]);
+      else if (a.wmode == 3) {
+        const double s = (in.Wa[v] - U) + 2. * (in.Wb[v] - U) + (in.w[v] - U);
+        out[v] = U + (s * (1. / 3.) + a.cW * r[v]);
+      } else out[v] = U + (2. / 3.) * ((in.w[v] - U) + a.cW * r[v]);
+    }
+    const double p = in.p;
+    if (cell + 64 * W < kFvT3) request(cell + 64 * W);
 #pragma unroll
-        for (int v = 0; v < 5; ++v) a.Wout[gi + v * kFvB3] = Ubuf[v] + a.cW * r[v];
-      } else if (a.wmode == 2) {
+    for (int v = 0; v < 5; ++v) a.Wout[gi + v * kFvB3] = out[v];
+    if (a.Pout) {
+      double P[5];
+      if (!sr_c2p(a.g.gam, a.tol, out, p, P)) a.bad[b] = 1;
 #pragma unroll
-        for (int v = 0; v < 5; ++v)
-          a.Wout[gi + v * kFvB3] = 0.75 * Ubuf[v] + 0.25 * (a.win[gi + v * kFvB3] + a.cW * r[v]);
-      }
+      for (int v = 0; v < 5; ++v) a.Pout[gi + v * kFvB3] = P[v];
     }
   }
 }
@@ -488,7 +534,8 @@ hipError_t launch_fv_max_speed(const FvGrid &g, const double *P, double *part, d
 hipError_t launch_fv_stage(const FvStageArgs &a, hipStream_t s) {
   const int ntiles = a.g.nbx * a.g.nbx * a.g.nbx * 8;
   const int grid = a.xcd_map ? 8 * ((ntiles + 7) / 8) : ntiles;
-  hipLaunchKernelGGL(fv_stage_kernel, dim3(grid), dim3(64), 0, s, a);
+  if (ntiles <= kFvSplitTiles) hipLaunchKernelGGL(fv_stage_kernel<3>, dim3(grid), dim3(192), 0, s, a);
+  else hipLaunchKernelGGL(fv_stage_kernel<1>, dim3(grid), dim3(64), 0, s, a);
   return hipGetLastError();
 }
 
