@@ -100,25 +100,25 @@ struct FilterArgs {
 };
 
 // ---------------------------------------------------------------------------
-// Discrete adjoint of the batched path.  With G = s_f A(n_f) lam at every
-// face point of every element (A the symmetric flux Jacobian, s_f the lift
-// scale), the transpose of the face gathers hands each element, at the
-// points of its face planes, the G of the points that read them:
-//   copy faces: the partner's G at the same point;
-//   interpolated faces: per (receiving face, neighbour) job the transposed
-//   tensor interpolation T = R1^T (w G) R2 on the neighbour's plane, w the
-//   averaging weight (1 / count where several neighbours hold a point),
-//   summed over the jobs that read the plane in a fixed order.
+// Discrete adjoint (adj_stage.h)
 // ---------------------------------------------------------------------------
 
-// one face of one element, as the sender of adjoint face terms
-struct AdjFace {
-  int kind;             // 0 outer boundary, 1 copy, 2 interpolated (one or several neighbours)
-  int nb, g;            // kind 1: the partner element and its face
-  int base, s1, s2;     // kind 1: partner node = base + a*s1 + b*s2 (element-local)
-  int jfirst, jcount;   // kind 2: the jobs that read this face's plane, in AdjAmrArgs::sjobs
+// One element, as the adjoint reads it.  fkind 0 outer boundary; 1 copy, with
+// the partner as in SlotRec and fg the partner's dXb/dX along the face over
+// this element's; 2 interpolated: foff the face's first entry in
+// AdjArgs::reads, fs1 their number.
+struct AdjRec {
+  SlotRec s;
+  double fg[6];
+  double pad[2];
 };
-static_assert(sizeof(AdjFace) == 32, "AdjFace is 32 bytes");
+static_assert(sizeof(AdjRec) == 320, "AdjRec is 320 bytes");
+
+// a transposed plane [4][n*n] that belongs to a face: the value of variable v
+// at face point (a, b) is T[off + v n n + a ca + b cb]
+struct AdjRead {
+  int off, ca, cb;
+};
 
 // one (receiving face, neighbour) interpolation job, transposed
 struct AdjJob {
@@ -135,41 +135,50 @@ struct AdjJob {
 };
 static_assert(sizeof(AdjJob) == 80, "AdjJob is 80 bytes");
 
-struct AdjAmrArgs {
-  const double *lam = nullptr, *phi = nullptr;   // as AdjArgs
+// One adjoint stage: y = L^T lam (L the Jacobian of the scalarwave1 DG RHS with
+// respect to u), then R = y or Wout as StageArgs' wmodes 1 and 3 to 6 with r = y
+// and win = lam.  The RHS is linear and the same at every stage, so the
+// transpose of an RK step is that RK step with L^T.  y_phi = 0 and y_pi has +
+// lam_phi, which stays what it is through a step: it is read from phi.  Wout
+// must not alias lam: neighbours read lam.
+struct AdjArgs {
+  const double *lam = nullptr, *phi = nullptr;
   const double *U = nullptr, *Wa = nullptr, *Wb = nullptr;
   double *Wout = nullptr, *R = nullptr;
   double cA = 0, cW = 0;
   int wmode = 0;
-  const int *list = nullptr;      // this launch's elements
+  int numflux = 0, xcd_map = 0;
+  const AdjRec *rec = nullptr;    // this launch's elements
   int nlist = 0;
-  const long *eoff = nullptr;     // [e]: first node
-  const int *en = nullptr;        // [e]: points per direction
-  const double *dXbdX = nullptr;  // [e][3]
-  const double *egeo = nullptr;   // [e][8]: box in patch coordinates, s0, s1
-  const int *edom = nullptr;      // [e]
+  const AdjRec *erec = nullptr;   // [e]: every element
+  const AdjRead *reads = nullptr;
   const double *dXdx = nullptr;   // element blocks of 9*np (stored geometry)
-  const double *Dall = nullptr;   // D of order n at batch_doff(n)
-  const double *xball = nullptr;  // LGL nodes of order n at batch_xoff(n)
-  const double *wend_inv = nullptr;   // [n]
-  const AdjFace *af = nullptr;    // [e][6]
-  const long *goff = nullptr;     // [e]: the element's G planes [6][4][n*n] in Gbuf
-  double *G = nullptr;
+  // D and LGL nodes of order n at batch_doff(n) and batch_xoff(n), 1 / (end
+  // weight) at [n]
+  const double *Dall = nullptr, *xball = nullptr, *wall = nullptr;
   const AdjJob *jobs = nullptr;
   int njobs = 0;
-  const int *sjobs = nullptr;     // job indices, grouped by the plane they read
   const int *mdesc = nullptr;
   const double *Btab = nullptr;
   double *T = nullptr;
-  int numflux = 0;
 };
 
-// G at every face point of the listed elements (any orders)
-hipError_t launch_adj_gflux(int geom, const AdjAmrArgs &a, hipStream_t s);
 // the transposed interpolation jobs into T
-hipError_t launch_adj_jobs(const AdjAmrArgs &a, hipStream_t s);
-// the transposed RHS and adjoint stage combination of one order bucket
-hipError_t launch_dg_adjoint_amr(int np, int geom, const AdjAmrArgs &a, int grid, hipStream_t s);
+hipError_t launch_adj_jobs_box(const AdjArgs &a, hipStream_t s);
+hipError_t launch_adj_jobs_stored(const AdjArgs &a, hipStream_t s);
+hipError_t launch_adj_jobs_shell(const AdjArgs &a, hipStream_t s);
+inline hipError_t launch_adj_jobs(int geom, const AdjArgs &a, hipStream_t s) {
+  return geom == 0 ? launch_adj_jobs_box(a, s) : geom == 1 ? launch_adj_jobs_stored(a, s) : launch_adj_jobs_shell(a, s);
+}
+// the stage over a.nlist elements of order np, or of any order up to nmax (np = 0)
+hipError_t launch_adj_box(int np, int nmax, const AdjArgs &a, hipStream_t s);
+hipError_t launch_adj_stored(int np, int nmax, const AdjArgs &a, hipStream_t s);
+hipError_t launch_adj_shell(int np, int nmax, const AdjArgs &a, hipStream_t s);
+inline hipError_t launch_adj(int np, int nmax, int geom, const AdjArgs &a, hipStream_t s) {
+  return geom == 0   ? launch_adj_box(np, nmax, a, s)
+         : geom == 1 ? launch_adj_stored(np, nmax, a, s)
+                     : launch_adj_shell(np, nmax, a, s);
+}
 
 // the DG stage kernels (dg_stage.h) over a.nlist elements of order np, or of
 // any order up to nmax (np = 0); geom 0 Cartesian, 1 stored dX/dx, 2

@@ -30,14 +30,6 @@ namespace nmx {
 // ---------------------------------------------------------------------------
 constexpr int kFaceWaves = 4;   // jobs per workgroup
 
-// LDS written by some lanes of a wave, read by others of the same wave: the
-// wave's LDS instructions are done in order, so only the compiler has to keep
-// them so
-__device__ __forceinline__ void wave_lds_fence() {
-  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-  __builtin_amdgcn_wave_barrier();
-}
-
 struct JobView {
   int n, m, ajoff, inn, in, base, t1, t2, sw, a0, a1, b0, b1, offA, offB;
   long soff;

@@ -84,7 +84,6 @@ struct nmx_ctx {
   SlotRec *dbrec = nullptr;
   double *dbD = nullptr, *dbxb = nullptr, *dbW = nullptr;
   int ndg = 0, nmaxdg = 0;   // DG elements, their largest order
-  int ncu = 0;
   bool anydg = false;     // the batched mesh has DG elements
   // troubled elements: TROUBLE values, scores, the mesh score (device),
   // the scores kept across a re-mirror, the per-element FV flags, a
@@ -133,22 +132,19 @@ struct nmx_ctx {
   // the faces with several neighbours run beside the single-neighbour ones
   double last_ms = 0;
   bool tuned = false;
-  // adjoint: lam register, neighbour face index per element face (plain
-  // path), its own graph cache, and the checkpoint pool
+  // adjoint: lam register, its own graph cache, and the checkpoint pool
   double *dL = nullptr;
-  int *dnbf = nullptr;
-  // adjoint of the batched path: the interpolation jobs as the forward
-  // tables made them (host), then the device tables, G and T buffers and
-  // one element list per order (plus one of all elements)
+  // the interpolation jobs as the forward tables made them (host), then, from
+  // the first adjoint call on, the device tables: one record per element in
+  // element order and by decreasing order, the planes that belong to each
+  // face, the jobs and their planes
   std::vector<AdjJob> hadjj;
   std::vector<int> hadjsend;   // per job: sender element, sender face
-  AdjFace *dadjf = nullptr;
+  AdjRec *dadje = nullptr, *dadjr = nullptr;
+  AdjRead *dadjp = nullptr;
   AdjJob *dadjj = nullptr;
-  int *dadjs = nullptr, *dadjl = nullptr;
-  long *dadjg = nullptr;
-  double *dadjG = nullptr, *dadjT = nullptr;
-  std::vector<std::pair<int, int>> adjlists;   // (n, first) in dadjl; all elements first
-  std::vector<int> adjcount;
+  double *dadjT = nullptr;
+  std::vector<std::pair<int, int>> adjorders;   // (order, elements) as in dadjr
   int adjnjobs = 0;
   bool adj_ready = false;
   // FV elements (fv_divf) on uniform points: every element (fvelm, plain
@@ -383,20 +379,18 @@ static void free_mesh_dev(nmx_ctx *c) {
   if (c->graph) { (void)hipGraphDestroy(c->graph); c->graph = nullptr; }
   c->graph_steps = 0;
   {
-    void **ptrs[] = {(void **)&c->dL, (void **)&c->dnbf, (void **)&c->deoff, (void **)&c->den,
+    void **ptrs[] = {(void **)&c->dL, (void **)&c->deoff, (void **)&c->den,
                      (void **)&c->dCk, (void **)&c->dwc, (void **)&c->dwcall,
                      (void **)&c->dcrctab, (void **)&c->dcrcvtab, (void **)&c->dcrcklane,
                      (void **)&c->dcrcaw, (void **)&c->dcrcypow,
                      (void **)&c->dcrcpart, (void **)&c->dcrcout, (void **)&c->dnbr,
                      (void **)&c->dlimh, (void **)&c->dwqall, (void **)&c->dldat, (void **)&c->dlimhw,
-                     (void **)&c->damat, (void **)&c->dsmat, (void **)&c->dadjf, (void **)&c->dadjj,
-                     (void **)&c->dadjs, (void **)&c->dadjl, (void **)&c->dadjg, (void **)&c->dadjG,
-                     (void **)&c->dadjT};
+                     (void **)&c->damat, (void **)&c->dsmat, (void **)&c->dadje, (void **)&c->dadjr,
+                     (void **)&c->dadjp, (void **)&c->dadjj, (void **)&c->dadjT};
     for (auto q : ptrs)
       if (*q) { (void)hipFree(*q); *q = nullptr; }
     c->adj_ready = false;
-    c->adjlists.clear();
-    c->adjcount.clear();
+    c->adjorders.clear();
   }
   if (c->agexec) { (void)hipGraphExecDestroy(c->agexec); c->agexec = nullptr; }
   if (c->agraph) { (void)hipGraphDestroy(c->agraph); c->agraph = nullptr; }
@@ -638,17 +632,8 @@ static std::vector<double> fv_cell_widths(int n) {
   return wc;
 }
 
-// The DG elements' records (in recs, element order) for launches over all
-// orders, by decreasing order, and D, nodes and end weights of every order.
-static int upload_order_tables(nmx_ctx *c, std::vector<SlotRec> &recs) {
-  c->ndg = (int)recs.size();
-  c->anydg = !recs.empty();
-  c->nmaxdg = 0;
-  if (recs.empty()) return NMX_OK;
-  std::stable_sort(recs.begin(), recs.end(), [](const SlotRec &x, const SlotRec &y) { return x.n > y.n; });
-  if (recs.back().n < 2 || recs[0].n > kBatchMaxN)
-    return fail(NMX_EUNSUP, "batched DG elements need 2 to 10 points per direction");
-  c->nmaxdg = recs[0].n;
+// D, nodes and 1 / (end weight) of every order
+static int upload_order_tables(nmx_ctx *c) {
   std::vector<double> D, xb, wi(kBatchMaxN + 1, 0.0);
   for (int n = 2; n <= kBatchMaxN; ++n) {
     const Basis &b = lgl_basis(n);
@@ -658,14 +643,24 @@ static int upload_order_tables(nmx_ctx *c, std::vector<SlotRec> &recs) {
     xb.insert(xb.end(), b.x, b.x + n);
     wi[n] = 1.0 / b.w[0];
   }
-  hipDeviceProp_t prop;
-  HIPCHK(hipGetDeviceProperties(&prop, c->device));
-  c->ncu = prop.multiProcessorCount;
   int r;
-  if ((r = dev_upload(&c->dbrec, recs)) || (r = dev_upload(&c->dbD, D)) || (r = dev_upload(&c->dbxb, xb)) ||
-      (r = dev_upload(&c->dbW, wi)))
-    return r;
+  if ((r = dev_upload(&c->dbD, D)) || (r = dev_upload(&c->dbxb, xb)) || (r = dev_upload(&c->dbW, wi))) return r;
   return NMX_OK;
+}
+
+// the DG elements' records (in recs, element order) for launches over all
+// orders, by decreasing order
+static int upload_dg_records(nmx_ctx *c, std::vector<SlotRec> &recs) {
+  c->ndg = (int)recs.size();
+  c->anydg = !recs.empty();
+  c->nmaxdg = 0;
+  if (recs.empty()) return NMX_OK;
+  std::stable_sort(recs.begin(), recs.end(), [](const SlotRec &x, const SlotRec &y) { return x.n > y.n; });
+  if (recs.back().n < 2 || recs[0].n > kBatchMaxN)
+    return fail(NMX_EUNSUP, "batched DG elements need 2 to 10 points per direction");
+  c->nmaxdg = recs[0].n;
+  if (int r = upload_order_tables(c)) return r;
+  return dev_upload(&c->dbrec, recs);
 }
 
 // Tables of the batched path: face descriptors, face interpolation jobs
@@ -868,7 +863,7 @@ static int upload_amr_tables(nmx_ctx *c) {
   c->nfacejobs = (int)(jobs1.size() / kJobInts);
   if (jobs1.empty()) jobs1.assign(kJobInts, 0);
   if ((r = dev_upload(&c->djobs1, jobs1))) return r;
-  return upload_order_tables(c, dgrecs);
+  return upload_dg_records(c, dgrecs);
 }
 
 // host -> device mirror of the mesh (element-block layout)
@@ -1010,16 +1005,6 @@ static int upload_mesh(nmx_ctx *c) {
   }
   if ((r = dev_alloc(&c->dface, hf.size()))) return r;
   HIPCHK(hipMemcpy(c->dface, hf.data(), hf.size() * sizeof(int4), hipMemcpyHostToDevice));
-  // the neighbour's face on each conforming face (adjoint gathers)
-  std::vector<int> hnbf(6 * ne, 0);
-  for (size_t i = 0; i < ne; ++i)
-    for (int f = 0; f < 6; ++f)
-      if (hf[6 * i + f].x >= 0) {
-        int nf = M.e[i].nbf[f][0];
-        if (nf < 0 || nf > 5) return fail(NMX_EINVAL, "neighbour face index out of range");
-        hnbf[6 * i + f] = nf;
-      }
-  if ((r = dev_upload(&c->dnbf, hnbf))) return r;
   const Basis &b = lgl_basis(c->np1);
   std::vector<double> hD(b.D, b.D + c->np1 * c->np1);
   // xb: the element's points per direction (uniform ones on FV elements)
@@ -2744,59 +2729,57 @@ extern "C" int nmx_state_device_ptr(nmx_ctx *c, int reg, void **p, long *len) {
 
 static AdjArgs adj_base_args(nmx_ctx *c) {
   AdjArgs a;
-  a.dXdx = c->dXdx; a.dXbdX = c->dXbdX; a.egeo = c->degeo; a.xb = c->dxb; a.D = c->dD;
-  a.edom = c->dedom; a.face = c->dface; a.nbface = c->dnbf;
-  a.wend_inv = c->np1 ? 1.0 / lgl_basis(c->np1).w[0] : 0.0;
+  a.dXdx = c->dXdx;
+  a.Dall = c->dbD; a.xball = c->dbxb; a.wall = c->dbW;
+  a.erec = c->dadje; a.reads = c->dadjp; a.jobs = c->dadjj; a.njobs = c->adjnjobs; a.T = c->dadjT;
+  a.mdesc = c->dmdesc; a.Btab = c->dBtab;
   a.numflux = (P(c, "scalarwave1_numflux") == "LLF") ? 1 : 0;
   a.xcd_map = (P(c, "nmx_xcd") == "yes") ? 1 : 0;
-  a.e0 = 0;
-  a.e1 = (int)c->mesh.e.size();
   return a;
 }
 
-// the adjoint tables of the batched path (made once per mirror, at the
-// first adjoint call): per element face its kind, copy partner or the jobs
-// that read its plane; per job its transposed plane in T; G planes per
-// element; element lists per order
-static int adj_amr_prepare(nmx_ctx *c) {
+// The adjoint's tables (made once per mirror, at the first adjoint call): per
+// element its record, with the copy partner or the planes that belong to each
+// face; per job its transposed plane in T.  Every gather is checked here.
+static int adj_prepare(nmx_ctx *c) {
   if (c->adj_ready) return NMX_OK;
   const Mesh &M = c->mesh;
   const int ne = (int)M.e.size();
-  std::vector<long> goff(ne);
-  long glen = 0;
-  for (int e = 0; e < ne; ++e) { goff[e] = glen; glen += 24L * M.e[e].n * M.e[e].n; }
-  std::vector<AdjFace> af(6L * ne);
+  int r;
+  if (!c->dbD && (r = upload_order_tables(c))) return r;
+  std::vector<AdjRec> rec(ne);
   for (int e = 0; e < ne; ++e) {
     const Elm &E = M.e[e];
+    AdjRec &A = rec[e];
+    std::memset(&A, 0, sizeof A);
+    slot_geometry(M, e, A.s);
     for (int f = 0; f < 6; ++f) {
-      AdjFace &F = af[6L * e + f];
-      std::memset(&F, 0, sizeof F);
       if (E.ajmode[f] == 0) continue;
-      if (E.ajmode[f] == 1 || E.ajmode[f] == 2) {
-        const FaceCopy &fc = M.fcopy[6L * e + f];
-        const int nb = E.fnb[f][0];
-        const Elm &N = M.e[nb];
-        F.kind = 1; F.nb = nb; F.g = E.nbf[f][0];
-        F.base = (int)(fc.nbase - N.off); F.s1 = fc.s1; F.s2 = fc.s2;
-        if (N.n != E.n || F.g < 0 || F.g > 5) return fail(NMX_EINVAL, "adjoint: copy face between different orders");
-        const int n = E.n;
-        for (int cb = 0; cb < 2; ++cb)
-          for (int ca = 0; ca < 2; ++ca) {
-            const long p = F.base + (long)ca * (n - 1) * F.s1 + (long)cb * (n - 1) * F.s2;
-            if (p < 0 || p >= (long)n * n * n) return fail(NMX_EINVAL, "adjoint: copy table out of range");
-          }
-        // the partner's point lies on its face g
-        const long p0 = F.base;
-        const int I0[3] = {(int)(p0 % n), (int)((p0 / n) % n), (int)(p0 / ((long)n * n))};
-        if (I0[F.g >> 1] != (F.g & 1) * (n - 1)) return fail(NMX_EINVAL, "adjoint: copy partner face");
-        continue;
-      }
-      F.kind = 2;
+      if (E.ajmode[f] != 1 && E.ajmode[f] != 2) { A.s.fkind[f] = 2; continue; }
+      const FaceCopy &fc = M.fcopy[6L * e + f];
+      const int nb = E.fnb[f][0], g = E.nbf[f][0], n = E.n;
+      if (nb < 0 || nb >= ne || M.e[nb].n != n || g < 0 || g > 5)
+        return fail(NMX_EINVAL, "adjoint: copy face between different orders");
+      const Elm &N = M.e[nb];
+      const long base = fc.nbase - N.off;
+      for (int cb = 0; cb < 2; ++cb)
+        for (int ca = 0; ca < 2; ++ca) {
+          const long p = base + (long)ca * (n - 1) * fc.s1 + (long)cb * (n - 1) * fc.s2;
+          if (p < 0 || p >= (long)n * n * n) return fail(NMX_EINVAL, "adjoint: copy table out of range");
+          // the partner's points lie on its face g
+          const int I[3] = {(int)(p % n), (int)((p / n) % n), (int)(p / ((long)n * n))};
+          if (I[g >> 1] != (g & 1) * (n - 1)) return fail(NMX_EINVAL, "adjoint: copy partner face");
+        }
+      A.s.fkind[f] = 1;
+      A.s.foff[f] = 5 * N.off + base;
+      A.s.fs1[f] = fc.s1;
+      A.s.fs2[f] = fc.s2;
+      A.fg[f] = (E.bbox[2 * (f >> 1) + 1] - E.bbox[2 * (f >> 1)]) / (N.bbox[2 * (g >> 1) + 1] - N.bbox[2 * (g >> 1)]);
     }
   }
   const int nj = (int)c->hadjj.size();
   std::vector<AdjJob> jobs = c->hadjj;
-  std::vector<std::vector<int>> byplane(6L * ne);
+  std::vector<std::vector<AdjRead>> byface(6L * ne);
   long tlen = 0;
   for (int j = 0; j < nj; ++j) {
     AdjJob &J = jobs[j];
@@ -2804,7 +2787,7 @@ static int adj_amr_prepare(nmx_ctx *c) {
     J.toff = (int)tlen;
     tlen += 4L * J.m * J.m;
     const int se = c->hadjsend[2 * j], sf = c->hadjsend[2 * j + 1];
-    if (se < 0 || se >= ne || M.e[se].n != J.m || af[6L * se + sf].kind != 2)
+    if (se < 0 || se >= ne || M.e[se].n != J.m || rec[se].s.fkind[sf] != 2)
       return fail(NMX_EINVAL, "adjoint: a job reads a plane that is not an interpolated face");
     if (J.e < 0 || J.e >= ne || M.e[J.e].n != J.n || J.g < 0 || J.g > 5)
       return fail(NMX_EINVAL, "adjoint: job receiver out of range");
@@ -2814,36 +2797,30 @@ static int adj_amr_prepare(nmx_ctx *c) {
         const int q1 = J.A1 * (fa - J.A0) + J.B1 * (fb - J.B0), q2 = J.A2 * (fa - J.A0) + J.B2 * (fb - J.B0);
         if (q1 < 0 || q1 >= J.m || q2 < 0 || q2 >= J.m) return fail(NMX_EINVAL, "adjoint: plane map out of range");
       }
-    byplane[6L * se + sf].push_back(j);
+    // T(q1 + m q2) with q1, q2 affine in the face point
+    const int ka = J.A1 + J.m * J.A2, kb = J.B1 + J.m * J.B2;
+    byface[6L * se + sf].push_back({J.toff - J.A0 * ka - J.B0 * kb, ka, kb});
   }
-  std::vector<int> sj;
-  for (long k = 0; k < 6L * ne; ++k) {
-    af[k].jfirst = (int)sj.size();
-    af[k].jcount = (int)byplane[k].size();
-    sj.insert(sj.end(), byplane[k].begin(), byplane[k].end());
-  }
-  // lists: all elements, then one per order
-  std::vector<int> lists;
-  c->adjlists.clear();
-  c->adjcount.clear();
-  c->adjlists.push_back({0, 0});
-  for (int e = 0; e < ne; ++e) lists.push_back(e);
-  c->adjcount.push_back(ne);
-  for (int n = 2; n <= kBatchMaxN; ++n) {
-    const int first = (int)lists.size();
-    for (int e = 0; e < ne; ++e)
-      if (M.e[e].n == n) lists.push_back(e);
-    if ((int)lists.size() > first) {
-      c->adjlists.push_back({n, first});
-      c->adjcount.push_back((int)lists.size() - first);
-    }
+  std::vector<AdjRead> reads;
+  for (int e = 0; e < ne; ++e)
+    for (int f = 0; f < 6; ++f)
+      if (rec[e].s.fkind[f] == 2) {
+        const auto &b = byface[6L * e + f];
+        rec[e].s.foff[f] = (long)reads.size();
+        rec[e].s.fs1[f] = (int)b.size();
+        reads.insert(reads.end(), b.begin(), b.end());
+      }
+  std::vector<AdjRec> sorted = rec;
+  std::stable_sort(sorted.begin(), sorted.end(), [](const AdjRec &x, const AdjRec &y) { return x.s.n > y.s.n; });
+  c->adjorders.clear();
+  for (const AdjRec &A : sorted) {
+    if (c->adjorders.empty() || c->adjorders.back().first != A.s.n) c->adjorders.push_back({A.s.n, 0});
+    c->adjorders.back().second++;
   }
   if (jobs.empty()) jobs.resize(1);
-  if (sj.empty()) sj.assign(1, 0);
-  int r;
-  if ((r = dev_upload(&c->dadjf, af)) || (r = dev_upload(&c->dadjj, jobs)) || (r = dev_upload(&c->dadjs, sj)) ||
-      (r = dev_upload(&c->dadjl, lists)) || (r = dev_upload(&c->dadjg, goff)) ||
-      (r = dev_alloc(&c->dadjG, glen)) || (r = dev_alloc(&c->dadjT, tlen > 0 ? tlen : 1)))
+  if (reads.empty()) reads.resize(1);
+  if ((r = dev_upload(&c->dadje, rec)) || (r = dev_upload(&c->dadjr, sorted)) || (r = dev_upload(&c->dadjp, reads)) ||
+      (r = dev_upload(&c->dadjj, jobs)) || (r = dev_alloc(&c->dadjT, tlen > 0 ? tlen : 1)))
     return r;
   c->adjnjobs = nj;
   c->adj_ready = true;
@@ -2855,11 +2832,7 @@ static int adj_amr_prepare(nmx_ctx *c) {
     NEED_DEV(c);                                                                         \
     if ((c)->fvelm || (c)->anyfv)                                                        \
       return fail(NMX_EUNSUP, "the adjoint of FV elements is not built");               \
-    if ((c)->amr ? !(c)->anydg : !(c)->dnbf)                                             \
-      return fail(NMX_EUNSUP, "the adjoint needs a DG mesh");                           \
-    if ((c)->amr) {                                                                      \
-      if (int r_ = adj_amr_prepare(c)) return r_;                                        \
-    }                                                                                    \
+    if (int r_ = adj_prepare(c)) return r_;                                              \
     bool filt_ = false;                                                                  \
     if (int r_ = filter_prepare((c), filt_)) return r_;                                  \
     if (filt_) return fail(NMX_EUNSUP, "the adjoint of the exponential filter is not built"); \
@@ -2867,37 +2840,37 @@ static int adj_amr_prepare(nmx_ctx *c) {
       return fail(NMX_EUNSUP, "the adjoint of the limiter is not built");                \
   } while (0)
 
-// the batched path's adjoint stage: G, the transposed jobs, then one
-// launch per order, all on the context's stream
-static int launch_adj_amr(nmx_ctx *c, const AdjArgs &s) {
-  AdjAmrArgs a;
-  a.lam = s.lam; a.phi = s.phi; a.U = s.U; a.Wa = s.Wa; a.Wb = s.Wb; a.Wout = s.Wout; a.R = s.R;
-  a.cA = s.cA; a.cW = s.cW; a.wmode = s.wmode;
-  a.eoff = c->deoff; a.en = c->den; a.dXbdX = c->dXbdX; a.egeo = c->degeo; a.edom = c->dedom;
-  a.dXdx = c->dXdx; a.Dall = c->dbD; a.xball = c->dbxb; a.wend_inv = c->dbW;
-  a.af = c->dadjf; a.goff = c->dadjg; a.G = c->dadjG; a.jobs = c->dadjj; a.njobs = c->adjnjobs;
-  a.sjobs = c->dadjs; a.mdesc = c->dmdesc; a.Btab = c->dBtab; a.T = c->dadjT;
-  a.numflux = s.numflux;
-  a.list = c->dadjl;
-  a.nlist = c->adjcount[0];
-  hipError_t err = launch_adj_gflux(c->geom, a, c->stream);
-  if (err == hipSuccess) err = launch_adj_jobs(a, c->stream);
-  for (size_t b = 1; b < c->adjlists.size() && err == hipSuccess; ++b) {
-    a.list = c->dadjl + c->adjlists[b].second;
-    a.nlist = c->adjcount[b];
-    const int grid = std::min(a.nlist, 8 * c->ncu);
-    err = launch_dg_adjoint_amr(c->adjlists[b].first, c->geom, a, grid, c->stream);
+// One adjoint stage: the transposed jobs, then the elements, in one launch up
+// to 1024 elements (4 workgroups per CU), where the launches of the orders,
+// forked and joined, take longer than the elements, else one per order side
+// by side on the stream lanes, the largest order first.
+constexpr int kAdjMixedElems = 1024;
+static int launch_adj(nmx_ctx *c, AdjArgs a) {
+  hipError_t err = launch_adj_jobs(c->geom, a, c->stream);
+  if (err != hipSuccess) return fail(NMX_EHIP, std::string("adjoint launch: ") + hipGetErrorString(err));
+  const int ne = (int)c->mesh.e.size(), no = (int)c->adjorders.size();
+  if (no > 1 && ne <= kAdjMixedElems) {
+    a.rec = c->dadjr;
+    a.nlist = ne;
+    err = launch_adj(0, c->adjorders[0].first, c->geom, a, c->stream);
+    if (err != hipSuccess) return fail(NMX_EHIP, std::string("adjoint launch: ") + hipGetErrorString(err));
+    return NMX_OK;
   }
-  if (err != hipSuccess) return fail(NMX_EHIP, std::string("adjoint launch: ") + hipGetErrorString(err));
-  return NMX_OK;
-}
-
-static int launch_adj(nmx_ctx *c, const AdjArgs &a) {
-  if (c->amr) return launch_adj_amr(c, a);
-  int nel = a.e1 - a.e0;
-  int grid = a.xcd_map ? 8 * ((nel + 7) / 8) : nel;
-  hipError_t err = launch_dg_adjoint(c->np1, c->geom, a, grid, c->stream);
-  if (err != hipSuccess) return fail(NMX_EHIP, std::string("adjoint launch: ") + hipGetErrorString(err));
+  const int lanes = P(c, "nmx_concurrent") == "yes" ? std::min(no, (int)nmx_ctx::kLanes) : 1;
+  if (lanes > 1) HIPCHK(hipEventRecord(c->evfork, c->stream));
+  for (int l = 1; l < lanes; ++l) HIPCHK(hipStreamWaitEvent(c->helper[l - 1], c->evfork, 0));
+  a.rec = c->dadjr;
+  for (int b = 0; b < no; ++b) {
+    const int l = b % lanes;
+    a.nlist = c->adjorders[b].second;
+    err = launch_adj(c->adjorders[b].first, c->adjorders[b].first, c->geom, a, l ? c->helper[l - 1] : c->stream);
+    if (err != hipSuccess) return fail(NMX_EHIP, std::string("adjoint launch: ") + hipGetErrorString(err));
+    a.rec += a.nlist;
+  }
+  for (int l = 1; l < lanes; ++l) {
+    HIPCHK(hipEventRecord(c->evjoin[l - 1], c->helper[l - 1]));
+    HIPCHK(hipStreamWaitEvent(c->stream, c->evjoin[l - 1], 0));
+  }
   return NMX_OK;
 }
 

@@ -14,6 +14,14 @@ __device__ __forceinline__ const NMX_CONST T *as_const(const T *p) {
   return (const NMX_CONST T *)p;
 }
 
+// LDS written by some lanes of a wave, read by others of the same wave: the
+// wave's LDS instructions are done in order, so only the compiler has to keep
+// them so
+__device__ __forceinline__ void wave_lds_fence() {
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+}
+
 // upwind: F = fnum - f_inner for the 4 flux-carrying fields.  With A = f.n
 // Jacobian [[0,-n^T],[-n,0]], A+/- = (A +- |A|)/2 gives
 // F_pi = (dpi + n.dc)/2 and F_c = n F_pi with d = inner - adjacent

@@ -176,14 +176,12 @@ __device__ __forceinline__ void node_rhs(const NodeGeo &m, const double x[4], co
   }
 }
 
-// lift of face 2 dir + side at a node on it: r -= scale (fnum - f)(u - ua)
-// for the unit outward normal (dg_add_surface_fluxes_sign_fvflag,
-// dg.c:90-146; normal dg.c:470-481 via node_normal_from_idXdx_at_ijk,
-// utilities.c:48-81)
+// outward unit normal of face 2 dir + side (sig -1 or 1) at a node on it and
+// the lift's scale sqrtgdiag / w_end (dg.c:90-146,470-481 via
+// node_normal_from_idXdx_at_ijk, utilities.c:48-81)
 template <int GEOM>
-__device__ __forceinline__ void node_lift(const NodeGeo &m, int dir, double sig, double wend_inv, int numflux,
-                                          const double u[4], const double ua[4], double r[4]) {
-  double nrm[3], scale;
+__device__ __forceinline__ void node_face(const NodeGeo &m, int dir, double sig, double wend_inv, double nrm[3],
+                                          double &scale) {
   if (GEOM == 2) {
     const double sg = sig * m.pm;
     if (dir == 0) {
@@ -206,6 +204,14 @@ __device__ __forceinline__ void node_lift(const NodeGeo &m, int dir, double sig,
   } else {
     face_normal<1>(m.M, m.g, 2 * dir + (sig > 0.0), wend_inv, nrm, scale);
   }
+}
+
+// lift of that face: r -= scale (fnum - f)(u - ua)
+template <int GEOM>
+__device__ __forceinline__ void node_lift(const NodeGeo &m, int dir, double sig, double wend_inv, int numflux,
+                                          const double u[4], const double ua[4], double r[4]) {
+  double nrm[3], scale;
+  node_face<GEOM>(m, dir, sig, wend_inv, nrm, scale);
   const double dc[3] = {u[1] - ua[1], u[2] - ua[2], u[3] - ua[3]};
   double F[4];
   face_flux(numflux, nrm, u[0] - ua[0], dc, F);

@@ -52,27 +52,6 @@ struct StageArgs {
   double rec_s1 = 0, rec_s2 = 1.7976931348623157e308;
 };
 
-// Arguments of one fused adjoint RHS + RK stage launch: y = L^T lam (L the
-// Jacobian of the scalarwave1 DG RHS with respect to u), then R = y or Wout
-// as StageArgs' wmodes 1 and 3 to 6 with r = y and win = lam.  The RHS is
-// linear and the same at every stage, so the transpose of an RK step is that
-// RK step with L^T.  y_phi = 0 and y_pi has + lam_phi, which stays what it is
-// through a step: it is read from phi.  Wout must not alias lam: neighbours
-// read lam.
-struct AdjArgs {
-  const double *lam = nullptr, *phi = nullptr;
-  const double *U = nullptr, *Wa = nullptr, *Wb = nullptr;
-  double *Wout = nullptr, *R = nullptr;
-  double cA = 0, cW = 0;
-  int wmode = 0;
-  const double *dXdx = nullptr, *dXbdX = nullptr, *egeo = nullptr, *xb = nullptr, *D = nullptr;
-  const int *edom = nullptr;
-  const int4 *face = nullptr;    // as StageArgs::face
-  const int *nbface = nullptr;   // [e][6]: the neighbour's face touching face f
-  double wend_inv = 0;
-  int numflux = 0, xcd_map = 0, e0 = 0, e1 = 0;
-};
-
 // the mesh's dt from the device's node coordinates (update_elm_eid_dt with
 // find_hmin): per-workgroup minima in part[grid], the mesh's in out[0]
 struct DtArgs {
@@ -87,8 +66,6 @@ struct DtArgs {
 int dt_grid(int nelem);
 hipError_t launch_dt(const DtArgs &a, int grid, hipStream_t s);
 
-// geom: 0 Cartesian, 1 stored dXdx, 2 CubedShell recomputed
-hipError_t launch_dg_adjoint(int np, int geom, const AdjArgs &a, int grid, hipStream_t s);
 // scalarwave1 on FV elements (fv_divf); rec: the interior scheme, 5 WENO5,
 // 7 WENO-Z, 9 WENOT, 3 WENOm3 (the end midpoints by StageArgs::recend);
 // wc[np]: distances between the midpoints around each uniform point
