@@ -193,10 +193,11 @@ inline hipError_t launch_dg(int np, int nmax, int geom, const AmrArgs &a, hipStr
 }
 hipError_t launch_face_interp(const FaceArgs &a, hipStream_t s);
 hipError_t launch_filter(int np, int geom, const FilterArgs &a, hipStream_t s);
-// an FV order bucket (fv_divf on uniform points): rec 5 = WENOm5_2, 7 =
-// WENOmZ_2, 3 = WENOm3_2; geom 0 Cartesian, 2 CubedShell; wc[np] the
-// distances between the midpoints around each point; a.xb uniform points
-hipError_t launch_fvelm_amr(int np, int rec, int geom, const AmrArgs &a, const double *wc, int grid,
-                            hipStream_t s);
+// the FV element kernel (fv_divf on uniform points, fvelm_stage.h) over
+// a.nlist elements of np points; rec: the interior scheme, 5 WENO5, 7 WENO-Z,
+// 9 WENOT, 3 WENOm3 (the end midpoints by AmrArgs::recend); geom 0 Cartesian,
+// 2 CubedShell; wc[np]: distances between the midpoints around each uniform
+// point; a.xb the uniform points
+hipError_t launch_fvelm(int np, int rec, int geom, const AmrArgs &a, const double *wc, hipStream_t s);
 
 }  // namespace nmx

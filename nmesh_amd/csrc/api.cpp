@@ -1656,6 +1656,15 @@ static AmrArgs amr_args(nmx_ctx *c, const StageArgs &sa) {
   return a;
 }
 
+// the FV elements of a.rec
+static hipError_t launch_fv(nmx_ctx *c, int n, AmrArgs a, const double *wc, hipStream_t st) {
+  const int rec = fv_rec_pars(c, a.recend, a.rec_s1, a.rec_s2, a.rec_opt, a.rec_on);
+  a.rec_first = P(c, "fv_rec") == "1";
+  a.fv_mid = P(c, "coordinates_midpoint_data") != "no";
+  fv_extrap_pars(c, a.ex_s1, a.ex_s2, a.ex_opt, a.ex_on);
+  return launch_fvelm(n, rec, c->geom == 0 ? 0 : 2, a, wc, st);
+}
+
 // one order bucket's stage kernel
 static int launch_bucket(nmx_ctx *c, AmrArgs a, const nmx_ctx::Bucket &b, int xcd_map, hipStream_t st) {
   a.D = c->dDall + b.doff;
@@ -1664,17 +1673,7 @@ static int launch_bucket(nmx_ctx *c, AmrArgs a, const nmx_ctx::Bucket &b, int xc
   a.rec = b.drec;
   a.nlist = b.count;
   a.xcd_map = xcd_map;
-  hipError_t err;
-  if (b.fv) {
-    const int grid = a.xcd_map ? 8 * ((b.count + 7) / 8) : b.count;
-    const int rec = fv_rec_pars(c, a.recend, a.rec_s1, a.rec_s2, a.rec_opt, a.rec_on);
-    a.rec_first = P(c, "fv_rec") == "1";
-    a.fv_mid = P(c, "coordinates_midpoint_data") != "no";
-    fv_extrap_pars(c, a.ex_s1, a.ex_s2, a.ex_opt, a.ex_on);
-    err = launch_fvelm_amr(b.n, rec, c->geom == 0 ? 0 : 2, a, c->dwcall + b.woff, grid, st);
-  } else {
-    err = launch_dg(b.n, b.n, c->geom, a, st);
-  }
+  const hipError_t err = b.fv ? launch_fv(c, b.n, a, c->dwcall + b.woff, st) : launch_dg(b.n, b.n, c->geom, a, st);
   if (err != hipSuccess) return fail(NMX_EHIP, std::string("stage launch: ") + hipGetErrorString(err));
   return NMX_OK;
 }
@@ -1749,17 +1748,6 @@ static int launch_amr(nmx_ctx *c, const StageArgs &sa) {
 
 static int launch(nmx_ctx *c, StageArgs a) {
   if (c->amr) return launch_amr(c, a);
-  if (c->fvelm) {
-    int nel = a.e1 - a.e0;
-    int grid = a.xcd_map ? 8 * ((nel + 7) / 8) : nel;
-    const int rec = fv_rec_pars(c, a.recend, a.rec_s1, a.rec_s2, a.rec_opt, a.rec_on);
-    a.rec_first = P(c, "fv_rec") == "1";
-    a.fv_mid = P(c, "coordinates_midpoint_data") != "no";
-    fv_extrap_pars(c, a.ex_s1, a.ex_s2, a.ex_opt, a.ex_on);
-    hipError_t err = launch_fvelm_stage(c->np1, rec, c->geom == 0 ? 0 : 2, a, c->dwc, grid, c->stream);
-    if (err != hipSuccess) return fail(NMX_EHIP, std::string("fv stage launch: ") + hipGetErrorString(err));
-    return NMX_OK;
-  }
   AmrArgs ca = amr_args(c, a);
   ca.D = c->dD;
   ca.xb = c->dxb;
@@ -1767,6 +1755,11 @@ static int launch(nmx_ctx *c, StageArgs a) {
   ca.rec = c->dfrec;
   ca.nlist = (int)c->mesh.e.size();
   ca.xcd_map = a.xcd_map;
+  if (c->fvelm) {
+    hipError_t err = launch_fv(c, c->np1, ca, c->dwc, c->stream);
+    if (err != hipSuccess) return fail(NMX_EHIP, std::string("fv stage launch: ") + hipGetErrorString(err));
+    return NMX_OK;
+  }
   int launches = 1;
   if (P(c, "nmx_path") == "perelement") {
     launches = ca.nlist;

@@ -1,19 +1,13 @@
-// fvelm_ex_kernels.hip -- the FV element kernels (fvelm_impl.h) with the
+// fvelm_ex_kernels.hip -- the FV element kernels (fvelm_stage.h) with the
 // fv_divf_extrap_s1 / _s2 / _opt limit of dnfn_extrap1 (rec1d.c:542-609);
-// a separate translation unit so both variants compile in parallel and the
+// a separate translation unit so the variants compile in parallel and the
 // common one keeps its registers.
-#include "fvelm_impl.h"
+#include "fvelm_stage.h"
 
 namespace nmx {
 
-hipError_t launch_fvelm_stage_ex(int np, int rec, int geom, const StageArgs &a, const double *wc, int grid,
-                                 hipStream_t s) {
-  return launch_fvelm_stage_v<true>(np, rec, geom, a, wc, grid, s);
-}
-
-hipError_t launch_fvelm_amr_ex(int np, int rec, int geom, const AmrArgs &a, const double *wc, int grid,
-                               hipStream_t s) {
-  return launch_fvelm_amr_v<true>(np, rec, geom, a, wc, grid, s);
+hipError_t launch_fvelm_ex(int np, int rec, int geom, const AmrArgs &a, const double *wc, hipStream_t s) {
+  return launch_fvelm_v<true, true>(np, rec, geom, a, wc, s);
 }
 
 }  // namespace nmx

@@ -66,14 +66,6 @@ struct DtArgs {
 int dt_grid(int nelem);
 hipError_t launch_dt(const DtArgs &a, int grid, hipStream_t s);
 
-// scalarwave1 on FV elements (fv_divf); rec: the interior scheme, 5 WENO5,
-// 7 WENO-Z, 9 WENOT, 3 WENOm3 (the end midpoints by StageArgs::recend);
-// wc[np]: distances between the midpoints around each uniform point
-// geom: 0 Cartesian, 2 CubedShell (metric recomputed at nodes and midpoints
-// from egeo, edom and the uniform points in xb)
-hipError_t launch_fvelm_stage(int np, int rec, int geom, const StageArgs &a, const double *wc, int grid,
-                              hipStream_t s);
-
 // The checkpoint's "vars" CRC-64 of a register (element blocks [e][5][np_e]).
 struct CrcArgs {
   const double *u = nullptr;
