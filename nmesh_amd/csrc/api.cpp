@@ -127,6 +127,7 @@ struct nmx_ctx {
   static constexpr int kLanes = 4;     // stream lanes of the concurrent buckets
   std::vector<int> border;             // buckets by decreasing node count
   std::vector<int> blane;              // lane of each bucket
+  bool inturn = false;                 // the launches of a stage in turn on one lane
   hipStream_t helper[kHelpers] = {};
   hipEvent_t evfork = nullptr, evjoin[kHelpers] = {};
   // the faces with several neighbours run beside the single-neighbour ones
@@ -870,6 +871,7 @@ static int upload_amr_tables(nmx_ctx *c) {
 static int upload_mesh(nmx_ctx *c) {
   free_mesh_dev(c);
   c->tuned = false;
+  c->inturn = false;
   Mesh &M = c->mesh;
   const long nn = M.nnodes;
   const size_t ne = M.e.size();
@@ -1726,7 +1728,7 @@ static int launch_amr(nmx_ctx *c, const StageArgs &sa) {
     else if (c->buckets[bi].fv)
       own.push_back({bi, c->anydg ? 1 + (int)own.size() % (nmx_ctx::kLanes - 1) : (int)own.size() % nmx_ctx::kLanes});
   }
-  if (P(c, "nmx_concurrent") != "yes")
+  if (P(c, "nmx_concurrent") != "yes" || c->inturn)
     for (auto &b : own) b.second = 0;
   unsigned used = 0;
   for (const auto &b : own) used |= 1u << b.second;
@@ -2495,16 +2497,40 @@ extern "C" int nmx_autotune(nmx_ctx *c) {
   hipEvent_t t0, t1;
   HIPCHK(hipEventCreate(&t0));
   HIPCHK(hipEventCreate(&t1));
-  // 4 steps after one to warm up
-  auto steps_ms = [&](float &ms) -> int {
-    if (int rr = issue_step(c, method, c->dt, 0, false)) return rr;
+  // what issue() launches, from a graph where steps run from one: eager
+  // launches of short kernels take the time of their host side
+  const bool use_graph = P(c, "nmx_graph") == "yes";
+  auto timed_ms = [&](auto &&issue, float &ms) -> int {
+    if (int rr = issue()) return rr;   // warm-up
+    hipGraphExec_t x = nullptr;
+    if (use_graph) {
+      HIPCHK(hipStreamBeginCapture(c->stream, hipStreamCaptureModeThreadLocal));
+      const int rr = issue();
+      hipGraph_t g = nullptr;
+      const hipError_t ec = hipStreamEndCapture(c->stream, &g);
+      const hipError_t ei = rr || ec != hipSuccess ? ec : hipGraphInstantiate(&x, g, nullptr, nullptr, 0);
+      if (g) (void)hipGraphDestroy(g);
+      if (rr) return rr;
+      if (ei != hipSuccess) return fail(NMX_EHIP, std::string("autotune graph: ") + hipGetErrorString(ei));
+      HIPCHK(hipGraphLaunch(x, c->stream));
+    }
     HIPCHK(hipEventRecord(t0, c->stream));
-    for (int s = 0; s < 4; ++s)
-      if (int rr = issue_step(c, method, c->dt, 0, (s & 1) != 0)) return rr;
+    for (int s = 0; s < 2; ++s) {
+      if (x) HIPCHK(hipGraphLaunch(x, c->stream));
+      else if (int rr = issue()) return rr;
+    }
     HIPCHK(hipEventRecord(t1, c->stream));
     HIPCHK(hipEventSynchronize(t1));
     HIPCHK(hipEventElapsedTime(&ms, t0, t1));
+    if (x) (void)hipGraphExecDestroy(x);
     return NMX_OK;
+  };
+  auto steps_ms = [&](float &ms) -> int {
+    return timed_ms([&]() -> int {
+      for (int s = 0; s < 4; ++s)
+        if (int rr = issue_step(c, method, c->dt, 0, (s & 1) != 0)) return rr;
+      return NMX_OK;
+    }, ms);
   };
   std::string best_x = P(c, "nmx_xcd");
   float best = 1e30f;
@@ -2523,29 +2549,40 @@ extern "C" int nmx_autotune(nmx_ctx *c) {
     HIPCHK(hipMemcpyAsync(c->dW0, c->dU, c->nstate * 8, hipMemcpyDeviceToDevice, c->stream));
     if ((r = launch_amr(c, sa))) return r;   // fills the face buffer
     const AmrArgs a = amr_args(c, sa);
-    for (auto &b : c->buckets) {
-      if ((r = launch_bucket(c, a, b, sa.xcd_map, c->stream))) return r;   // warm-up
-      HIPCHK(hipEventRecord(t0, c->stream));
-      for (int s = 0; s < 5; ++s)
-        if ((r = launch_bucket(c, a, b, sa.xcd_map, c->stream))) return r;
-      HIPCHK(hipEventRecord(t1, c->stream));
-      HIPCHK(hipEventSynchronize(t1));
-      HIPCHK(hipEventElapsedTime(&b.ms, t0, t1));
-    }
+    for (auto &b : c->buckets)
+      if ((r = timed_ms([&]() -> int {
+             for (int s = 0; s < 4; ++s)
+               if (int rr = launch_bucket(c, a, b, sa.xcd_map, c->stream)) return rr;
+             return NMX_OK;
+           }, b.ms)))
+        return r;
     assign_lanes(c);
-    // one launch for the DG elements of all orders, or one per order, by
-    // whole steps (unless set)
-    if (!c->batch_fixed && c->anydg) {
-      std::string best_shape;
-      float bt = 1e30f;
-      for (const char *shape : {"persistent", "buckets"}) {
+    // One launch for the DG elements of all orders, or one per order, by whole
+    // steps (unless set); and the launches of a stage side by side or in turn:
+    // a helper lane's fork and join take about 10 us of a stage in a graph (16
+    // RK4 steps of a DG and an FV bucket of 5 and 9 us: 1.40 ms side by side,
+    // 1.11 in turn; 20 of 5 buckets of about 5 us: 4.0 and 3.2, in one launch
+    // 1.1; 16 of 7 orders with 19,200 elements: 25.4 side by side).
+    std::string best_shape;
+    bool best_turn = false;
+    float bt = 1e30f;
+    const bool lanes = P(c, "nmx_concurrent") == "yes";
+    for (const char *shape : {"persistent", "buckets"}) {
+      if (c->batch_fixed || !c->anydg) {
+        if (best_shape.empty()) best_shape = P(c, "nmx_batch");
+        else break;
+      } else {
         c->par["nmx_batch"] = shape;
+      }
+      for (int turn = 0; turn < (lanes ? 2 : 1); ++turn) {
+        c->inturn = turn != 0;
         float ms = 0;
         if ((r = steps_ms(ms))) return r;
-        if (ms < bt) { bt = ms; best_shape = shape; }
+        if (ms < bt) { bt = ms; best_shape = P(c, "nmx_batch"); best_turn = c->inturn; }
       }
-      c->par["nmx_batch"] = best_shape;
     }
+    c->par["nmx_batch"] = best_shape;
+    c->inturn = best_turn;
   }
   (void)hipEventDestroy(t0);
   (void)hipEventDestroy(t1);
