@@ -15,6 +15,7 @@
 #include "../../include/nmx.h"
 #include "errors.h"
 #include "fv.h"
+#include "host_copy.h"
 
 using namespace nmx;
 
@@ -34,6 +35,7 @@ struct nmx_fv {
   hipGraphExec_t gexec = nullptr;
   int graph_steps = 0, graph_method = -1;
   double graph_dt = 0;
+  HostCopy io;
   const double *graph_prim = nullptr;   // the captured steps' first primitives
   hipEvent_t ev0 = nullptr, ev1 = nullptr;
   double last_ms = 0;
@@ -86,6 +88,7 @@ extern "C" int nmx_fv_destroy(nmx_fv *f) {
   (void)hipSetDevice(f->device);
   if (f->stream) (void)hipStreamSynchronize(f->stream);
   free_grid(f);
+  f->io.release();
   if (f->ev0) (void)hipEventDestroy(f->ev0);
   if (f->ev1) (void)hipEventDestroy(f->ev1);
   if (f->own_stream) (void)hipStreamDestroy(f->own_stream);
@@ -188,7 +191,7 @@ extern "C" int nmx_fv_set_time(nmx_fv *f, double t) {
 
 // host flat [v][cell] -> block layout register (through the R scratch register)
 static int upload_flat(nmx_fv *f, double *dst, const double *h) {
-  HIPCHK(hipMemcpyAsync(f->dT, h, f->nstate * 8, hipMemcpyHostToDevice, f->stream));
+  HIPCHK(f->io.copy(f->device, f->dT, h, f->nstate, f->stream));
   hipError_t e = launch_fv_layout(f->g, f->dT, dst, 1, f->stream);
   if (e != hipSuccess) return fail(NMX_EHIP, std::string("layout: ") + hipGetErrorString(e));
   HIPCHK(hipStreamSynchronize(f->stream));
@@ -228,8 +231,7 @@ extern "C" int nmx_fv_download(nmx_fv *f, int which, double *h) {
   if (!d || !h) return fail(NMX_EINVAL, "bad register or NULL argument");
   hipError_t e = launch_fv_layout(f->g, d, f->dT, 0, f->stream);
   if (e != hipSuccess) return fail(NMX_EHIP, std::string("layout: ") + hipGetErrorString(e));
-  HIPCHK(hipMemcpyAsync(h, f->dT, f->nstate * 8, hipMemcpyDeviceToHost, f->stream));
-  HIPCHK(hipStreamSynchronize(f->stream));
+  HIPCHK(f->io.copy_back(f->device, h, f->dT, f->nstate, f->stream));
   return NMX_OK;
 }
 
