@@ -2511,40 +2511,16 @@ extern "C" int nmx_autotune(nmx_ctx *c) {
   hipEvent_t t0, t1;
   HIPCHK(hipEventCreate(&t0));
   HIPCHK(hipEventCreate(&t1));
-  // what issue() launches, from a graph where steps run from one: eager
-  // launches of short kernels take the time of their host side
-  const bool use_graph = P(c, "nmx_graph") == "yes";
-  auto timed_ms = [&](auto &&issue, float &ms) -> int {
-    if (int rr = issue()) return rr;   // warm-up
-    hipGraphExec_t x = nullptr;
-    if (use_graph) {
-      HIPCHK(hipStreamBeginCapture(c->stream, hipStreamCaptureModeThreadLocal));
-      const int rr = issue();
-      hipGraph_t g = nullptr;
-      const hipError_t ec = hipStreamEndCapture(c->stream, &g);
-      const hipError_t ei = rr || ec != hipSuccess ? ec : hipGraphInstantiate(&x, g, nullptr, nullptr, 0);
-      if (g) (void)hipGraphDestroy(g);
-      if (rr) return rr;
-      if (ei != hipSuccess) return fail(NMX_EHIP, std::string("autotune graph: ") + hipGetErrorString(ei));
-      HIPCHK(hipGraphLaunch(x, c->stream));
-    }
+  // 4 steps after one to warm up
+  auto steps_ms = [&](float &ms) -> int {
+    if (int rr = issue_step(c, method, c->dt, 0, false)) return rr;
     HIPCHK(hipEventRecord(t0, c->stream));
-    for (int s = 0; s < 2; ++s) {
-      if (x) HIPCHK(hipGraphLaunch(x, c->stream));
-      else if (int rr = issue()) return rr;
-    }
+    for (int s = 0; s < 4; ++s)
+      if (int rr = issue_step(c, method, c->dt, 0, (s & 1) != 0)) return rr;
     HIPCHK(hipEventRecord(t1, c->stream));
     HIPCHK(hipEventSynchronize(t1));
     HIPCHK(hipEventElapsedTime(&ms, t0, t1));
-    if (x) (void)hipGraphExecDestroy(x);
     return NMX_OK;
-  };
-  auto steps_ms = [&](float &ms) -> int {
-    return timed_ms([&]() -> int {
-      for (int s = 0; s < 4; ++s)
-        if (int rr = issue_step(c, method, c->dt, 0, (s & 1) != 0)) return rr;
-      return NMX_OK;
-    }, ms);
   };
   std::string best_x = P(c, "nmx_xcd");
   float best = 1e30f;
@@ -2563,13 +2539,15 @@ extern "C" int nmx_autotune(nmx_ctx *c) {
     HIPCHK(hipMemcpyAsync(c->dW0, c->dU, c->nstate * 8, hipMemcpyDeviceToDevice, c->stream));
     if ((r = launch_amr(c, sa))) return r;   // fills the face buffer
     const AmrArgs a = amr_args(c, sa);
-    for (auto &b : c->buckets)
-      if ((r = timed_ms([&]() -> int {
-             for (int s = 0; s < 4; ++s)
-               if (int rr = launch_bucket(c, a, b, sa.xcd_map, c->stream)) return rr;
-             return NMX_OK;
-           }, b.ms)))
-        return r;
+    for (auto &b : c->buckets) {
+      if ((r = launch_bucket(c, a, b, sa.xcd_map, c->stream))) return r;   // warm-up
+      HIPCHK(hipEventRecord(t0, c->stream));
+      for (int s = 0; s < 5; ++s)
+        if ((r = launch_bucket(c, a, b, sa.xcd_map, c->stream))) return r;
+      HIPCHK(hipEventRecord(t1, c->stream));
+      HIPCHK(hipEventSynchronize(t1));
+      HIPCHK(hipEventElapsedTime(&b.ms, t0, t1));
+    }
     assign_lanes(c);
     // One launch for the DG elements of all orders, or one per order, by whole
     // steps (unless set); and the launches of a stage side by side or in turn:
