@@ -97,6 +97,7 @@ struct FilterArgs {
   const double *dXdx = nullptr;   // element blocks of 9*np (stored geometry)
   int varmask = 0;                // bit v: pi, cx, cy, cz, phi
   int jpow = 0;                   // filter u J^jpow, J = 1/det(dXb/dx)
+  int xcd_map = 0;                // as the stages', whose output is in the XCDs' L2s
 };
 
 // ---------------------------------------------------------------------------

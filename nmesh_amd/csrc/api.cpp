@@ -1856,6 +1856,7 @@ static int launch_filters(nmx_ctx *c, double *reg) {
     if (!c->filt_mask[p]) continue;
     FilterArgs fa;
     fa.u = reg; fa.dXdx = c->dXdx; fa.varmask = c->filt_mask[p]; fa.jpow = c->filt_jpow;
+    fa.xcd_map = P(c, "nmx_xcd") == "yes";
     hipError_t err = hipSuccess;
     if (c->amr) {
       for (const auto &b : c->buckets) {
