@@ -50,13 +50,12 @@ __global__ __launch_bounds__(filter_threads(NP)) void filter_kernel(FilterArgs a
 #pragma unroll
   for (int v = 0; v < 5; ++v) val[v] = ALL || (mask >> v & 1) ? u[v * NP3 + node] : 0.0;
   for (int q = tid; q < NP2; q += NT) s_F[q] = a.F[q];
-  // the weights w = J^jpow and 1 / w up to a factor constant on the element:
+  // the weight w = J^jpow up to a factor constant on the element and 1 / w:
   // none on boxes; on shells det(dX/dx) = s^3 / ((s1 - s0) R^2) up to its sign
   // (NodeGeo, dg_stage.h)
   double w = 1.0, iw = 1.0;
   const bool weighted = GEOM != 0 && (a.jpow == 1 || a.jpow == -1);
   if (weighted) {
-    double d, id;
     if (GEOM == 1) {
       double M[3][3];
       const double *g = a.dXdx + 9 * noff;
@@ -64,17 +63,19 @@ __global__ __launch_bounds__(filter_threads(NP)) void filter_kernel(FilterArgs a
       for (int m = 0; m < 3; ++m)
 #pragma unroll
         for (int q = 0; q < 3; ++q) M[m][q] = g[(3 * m + q) * NP3 + node];
-      d = det3(M);
-      id = rcp_nr(d);
+      w = det3(M);
+      iw = rcp_nr(w);
     } else {
       const double A = patch_coord(R, 1, a.xb[j]), B = patch_coord(R, 2, a.xb[k]);
       const double r = R.s0 + (R.s1 - R.s0) * patch_coord(R, 0, a.xb[i]);
       const double t = 1.0 + A * A + B * B, rs = rsqrt_nr(t), ir = rcp_nr(r);
-      d = t * t * rs * (ir * ir);
-      id = (r * r) * (rs * rs * rs);
+      w = t * t * rs * (ir * ir);
+      iw = rcp_nr(w);
     }
-    w = a.jpow == 1 ? id : d;
-    iw = a.jpow == 1 ? d : id;
+    if (a.jpow == 1) {
+      w = iw;
+      iw = rcp_nr(w);
+    }
 #pragma unroll
     for (int v = 0; v < 5; ++v) val[v] *= w;
   }
@@ -109,7 +110,12 @@ __global__ __launch_bounds__(filter_threads(NP)) void filter_kernel(FilterArgs a
   if (tid >= NP3) return;
 #pragma unroll
   for (int v = 0; v < 5; ++v) {
-    if (weighted) val[v] *= iw;
+    if (weighted) {
+      // val / w with its remainder: what the weighting rounds off, every step
+      // rounds off again
+      const double q = val[v] * iw;
+      val[v] = fma(fma(-q, w, val[v]), iw, q);
+    }
     if (ALL || (mask >> v & 1)) u[v * NP3 + node] = val[v];
   }
 }
