@@ -33,9 +33,9 @@ FP64_PEAK_TFLOPS = 78.6
 # algorithmic bytes per node-update of a fused DG RHS + RK4 stage on
 # curvilinear elements: 8 * (25 state doubles + 9 dXdx)
 BYTES_PER_NU_CURV = 272.0
-# the least the batched path moves per node-update: 20 state doubles on
-# average over the 4 stages (dXdx recomputed)
-MIN_BYTES_PER_NU = 160.0
+# the least an RK4 stage moves per node-update: 13.5 state doubles on average
+# over the 4 stages (dXdx recomputed)
+MIN_BYTES_PER_NU = 108.0
 
 
 def flops_per_nu(n):
@@ -254,17 +254,15 @@ def batched_leg(nm, steps, plain_steps):
 
 
 # FV (config 3): algorithmic figures per cell-update (one RHS evaluation at
-# one cell, all 5 fields; sspRK3 does 3 per cell per step).  Bytes: the c2p
-# pass reads the conserved state and the pressure guess and writes the
-# primitives (11 doubles); the stage pass reads the primitives once and the
-# stage registers (win, u_p, u_acc: 5, 15 and 10 doubles in stages 1, 2, 3)
-# and writes u_acc, w (10, 10, 5): (11 + 5 + (15 + 25 + 15) / 3) * 8 = 275 B.
+# one cell, all 5 fields; sspRK3 does 3 per cell per step).  Bytes: a
+# stage reads the primitives, u_p and, after the first, its input, and writes
+# its output and the next primitives: (20 + 25 + 25) / 3 doubles = 187 B.
 # FLOPs (hand count of the kernel's formulas, a division or a square root
 # counted as one): 10 WENO5 reconstructions of 68 FLOPs, 2 SR fluxes with
 # eigenvalues of 60, LLF and accumulation 32, physicality checks 10: 852
 # per face, 3 faces per cell; c2p about 115 (5 Newton iterations of 20 and
 # the primitives) and the stage combination 15: about 2690 per cell-update.
-FV_BYTES_PER_CU = 275.0
+FV_BYTES_PER_CU = 187.0
 FV_FLOPS_PER_CU = 2690.0
 
 
@@ -320,7 +318,7 @@ def fvelm_leg(nm, steps=20):
     """scalarwave1 on FV elements inside the mesh (fv_divf): a BoxMesh
     [-8,8]^3 of 16^3 elements, all FV, n = 8 uniform points per direction
     (2,097,152 cells), WENOm5_2, upwind fnum, RK4.  Bytes per cell-update as
-    the DG stage on Cartesian elements: 160 B (stage average of the 15-25
+    the DG stage on Cartesian elements: 108 B (stage average of the 8 to 22
     state doubles read and written)."""
     p = {"amr_mesh_type": "BoxMesh", "amr_BoxMesh_dout": 8.0, "amr_luni": 4,
          "amr_n0": 8, "amr_n1": 8, "amr_n2": 8, "amr_uniform_p": "0", "amr_fv_p": "0",
@@ -347,7 +345,7 @@ def fvelm_leg(nm, steps=20):
            "value": nu / wall, "unit": "cell-updates/s", "steps": steps,
            "ms_per_step": 1e3 * wall / steps, "bytes_per_cell_update": MIN_BYTES_PER_NU,
            "achieved_GBps": gbs, "hbm_frac": gbs / HBM_PEAK_GBS,
-           "kernel": "fvelm_stage_kernel<8,5,*>"}
+           "kernel": "fvelm_kernel<8,5,0,*>"}
     del m
     out["shell"] = fvelm_shell_leg(nm, steps)
     return out
@@ -379,7 +377,7 @@ def fvelm_shell_leg(nm, steps=20):
            "value": nu / wall, "unit": "cell-updates/s", "steps": steps,
            "ms_per_step": 1e3 * wall / steps, "device_us_per_stage": dev_s / (4 * steps) * 1e6,
            "bytes_per_cell_update": MIN_BYTES_PER_NU, "achieved_GBps": gbs, "hbm_frac": gbs / HBM_PEAK_GBS,
-           "kernel": "fvelm_stage_kernel<8,5,*,2,*> (shell)"}
+           "kernel": "fvelm_kernel<8,5,2,*> (shell)"}
     del m
     return out
 
@@ -526,7 +524,7 @@ def filter_leg(nm, reps=100):
                        "(1,572,864 nodes), alp 36, s 32, J-weighted",
            "value": m.nnodes / per, "unit": "node-filterings/s", "us_per_launch": per * 1e6,
            "bytes_per_node": 80.0, "achieved_GBps": gbs, "hbm_frac": gbs / HBM_PEAK_GBS,
-           "kernel": "filter_kernel<8,2,512>"}
+           "kernel": "filter_kernel<8,2,true>"}
     del m
     return out
 
@@ -895,12 +893,11 @@ def plain_leg(nm, args, have_torch):
     # u, u_p and write u, w (25 doubles) plus 9 doubles of dXdx per node on
     # curvilinear elements, face-neighbour re-reads counted 0: 272 B
     achieved = BYTES_PER_NU_CURV * nn / avg_launch_s / 1e9
-    # the least this kernel must move: stage 1 reads u and writes u_acc, w
-    # (15 doubles), stages 2-3 read w, u_acc, u_p and write u_acc, w (25),
-    # stage 4 reads w, u_acc and writes u_acc (15); dXdx recomputed (0) or
-    # streamed (9)
+    # the least this kernel must move: pi and c of its input, of u after the
+    # first stage and of its output (8, 12, 12 doubles), and in stage 4 what
+    # ends the step (22); dXdx recomputed (0) or streamed (9)
     g = 9.0 if args.geometry == "stored" else 0.0
-    min_bytes_per_nu = 8.0 * ((15 + 25 + 25 + 15) / 4.0 + g)
+    min_bytes_per_nu = 8.0 * ((8 + 12 + 12 + 22) / 4.0 + g)
     achieved_min = min_bytes_per_nu * nn / avg_launch_s / 1e9
     tflops = flops_per_nu(args.plain_n) * nn / avg_launch_s / 1e12
     traffic = load_traffic("traffic_dg_stage_shell_n8.json") if args.plain_n == 8 else None
@@ -913,10 +910,9 @@ def plain_leg(nm, args, have_torch):
            "roofline": {"bound": "hbm", "achieved": achieved, "peak": HBM_PEAK_GBS, "unit": "GB/s",
                         "frac": achieved / HBM_PEAK_GBS,
                         "traffic": traffic["bytes_per_launch"] if traffic else None,
-                        "traffic_source": "profile figure: profiles/dg_stage_kernel_shell_n8_rk4.md" if traffic else None,
-                        "kernel": "dg_stage_kernel, n=%d, %s tile, %s geometry" % (args.plain_n, m.par("nmx_block"),
-                                                                                    args.geometry),
-                        "tile": m.par("nmx_block"), "xcd_map": m.par("nmx_xcd"),
+                        "traffic_source": "profile figure: profiles/stage_kernels_by_case.md" if traffic else None,
+                        "kernel": "dg_col_kernel or dg_node_kernel, n=%d, %s geometry" % (args.plain_n, args.geometry),
+                        "xcd_map": m.par("nmx_xcd"),
                         "avg_launch_us": avg_launch_s * 1e6,
                         "bytes_per_node_update": BYTES_PER_NU_CURV,
                         "min_bytes_per_node_update": min_bytes_per_nu,

@@ -574,8 +574,8 @@ __global__ __launch_bounds__(node_threads(NMAX)) void dg_mixed_kernel(AmrArgs a)
 // workgroups per CU), the node kernel below.  Steps of a shell, column against
 // node kernel: n = 5, 24,576 elements 405 and 355 us, n = 6 688 and 630, n = 7
 // 964 and 1216, n = 8 1272 and 1403, n = 10 2963 and 3612; 3072 elements n = 8
-// 146 and 151, n = 10 765 and 875; 384 elements n = 7 (with a filter) 55 and
-// 41, n = 8 53 and 35, n = 10 175 and 138.
+// 146 and 151, n = 10 382 and 437; 384 elements n = 7 (with a filter) 55 and
+// 41, n = 8 53 and 35, n = 10 88 and 69.
 constexpr int kNodeElems = 1024;
 
 template <int NP, int GEOM, int WM>

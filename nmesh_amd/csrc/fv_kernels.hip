@@ -342,8 +342,8 @@ __device__ __forceinline__ void fv_sweep(const FvStageArgs &a, int d, const int 
 // W waves per tile: 1, or 3 with one direction each, which finish a tile of a
 // small grid in about a third of the time.  The accumulators take 20 KB per
 // wave: 8 waves per CU, two per SIMD, which is also what 246 VGPRs allow.
-// 256^3 cells take 1.36 ms per stage, primitives included, at 36 TFLOP/s
-// counted by instructions (13,290 VALU instructions per tile, 86% of them FP64;
+// 256^3 cells take 1.33 ms per stage, primitives included, at about 26
+// TFLOP/s (13,290 VALU instructions per tile, 86% of them FP64;
 // VALU 60% busy, the rest waits on memory and issue).  Weights and fluxes
 // as they stood, by cell values with two IEEE square roots per state, windows
 // moved by copies and the primitives in a launch of their own, took 2.09 ms.
