@@ -257,13 +257,10 @@ def batched_leg(nm, steps, plain_steps):
 # one cell, all 5 fields; sspRK3 does 3 per cell per step).  Bytes: a
 # stage reads the primitives, u_p and, after the first, its input, and writes
 # its output and the next primitives: (20 + 25 + 25) / 3 doubles = 187 B.
-# FLOPs (hand count of the kernel's formulas, a division or a square root
-# counted as one): 10 WENO5 reconstructions of 68 FLOPs, 2 SR fluxes with
-# eigenvalues of 60, LLF and accumulation 32, physicality checks 10: 852
-# per face, 3 faces per cell; c2p about 115 (5 Newton iterations of 20 and
-# the primitives) and the stage combination 15: about 2690 per cell-update.
+# FLOPs: the stage kernel's FP64 instructions by the SQ_INSTS_VALU_*_F64
+# counters (profiles/stage_kernels_by_case.md), an FMA counted as two.
 FV_BYTES_PER_CU = 187.0
-FV_FLOPS_PER_CU = 2690.0
+FV_FLOPS_PER_CU = 2150.0
 
 
 def fv_leg(steps=50, warmup=8, N=256, cpu=True):

@@ -26,7 +26,7 @@ namespace nmx {
 // lines of a plane normal to x (every line of the element's block) come from
 // HBM once, and four jobs, of which a CU mostly finds the plane in its L1, make
 // a workgroup (one wave per workgroup: the 100,318 jobs of 19,200 elements of 4
-// to 10 points take 118 us instead of 106, 276 MB fetched and 167 written).
+// to 10 points take 118 us instead of 106, 282 MB fetched and 171 written).
 // ---------------------------------------------------------------------------
 constexpr int kFaceWaves = 4;   // jobs per workgroup
 

@@ -342,11 +342,12 @@ __device__ __forceinline__ void fv_sweep(const FvStageArgs &a, int d, const int 
 // W waves per tile: 1, or 3 with one direction each, which finish a tile of a
 // small grid in about a third of the time.  The accumulators take 20 KB per
 // wave: 8 waves per CU, two per SIMD, which is also what 246 VGPRs allow.
-// 256^3 cells take 1.33 ms per stage, primitives included, at about 26
-// TFLOP/s (13,290 VALU instructions per tile, 86% of them FP64;
-// VALU 60% busy, the rest waits on memory and issue).  Weights and fluxes
-// as they stood, by cell values with two IEEE square roots per state, windows
-// moved by copies and the primitives in a launch of their own, took 2.09 ms.
+// 256^3 cells take 1.33 ms per stage, primitives included, at 27 TFLOP/s
+// (2,150 operations per cell by the counters; 13,140 VALU instructions per
+// tile, 85% of them FP64; VALU 60% busy, the rest waits on memory and issue).
+// Weights and fluxes as they stood, by cell values with two IEEE square roots
+// per state, windows moved by copies and the primitives in a launch of their
+// own, took 2.09 ms.
 // The line's 9 faces are unrolled: 61 KB of code, of the 64 KB that two CUs
 // share.  One copy of the sweep for all directions, a nontemporal epilogue and
 // tiles in 2^3-block bricks measured no faster (5.5% slower, and within 0.5%).
