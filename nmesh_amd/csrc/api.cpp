@@ -62,10 +62,8 @@ struct nmx_ctx {
   long iteration = 0;           // full steps taken (mesh->iteration, main.c:617)
   // device mirror
   double *dU = nullptr, *dA = nullptr, *dW0 = nullptr, *dW1 = nullptr, *dR = nullptr, *dP = nullptr;
-  double *dXdx = nullptr, *dXbdX = nullptr, *dxyz = nullptr, *dD = nullptr, *dT = nullptr;
-  double *degeo = nullptr, *dxb = nullptr;
-  int *dedom = nullptr;
-  int4 *dface = nullptr;
+  double *dXdx = nullptr, *dxyz = nullptr, *dD = nullptr, *dT = nullptr;
+  double *dxb = nullptr;
   int geom = 0;          // 0 Cartesian, 1 stored dXdx, 2 recomputed CubedShell
   // batched (order-bucketed) mirror
   bool amr = false;
@@ -356,10 +354,9 @@ static void drop_stage_graphs(nmx_ctx *c) {
 static void free_mesh_dev(nmx_ctx *c) {
   c->ldat_up = nullptr;
   double **bufs[] = {&c->dU, &c->dA, &c->dW0, &c->dW1, &c->dR, &c->dP,
-                     &c->dXdx, &c->dXbdX, &c->dxyz, &c->dD, &c->dT, &c->degeo, &c->dxb};
+                     &c->dXdx, &c->dxyz, &c->dD, &c->dT, &c->dxb};
   for (auto b : bufs)
     if (*b) { (void)hipFree(*b); *b = nullptr; }
-  if (c->dedom) { (void)hipFree(c->dedom); c->dedom = nullptr; }
   {
     void **ptrs[] = {(void **)&c->djobs1, (void **)&c->dmdesc, (void **)&c->dFilt, (void **)&c->dfrec,
                      (void **)&c->dBtab, (void **)&c->dDall, (void **)&c->dxball, (void **)&c->daj,
@@ -374,7 +371,6 @@ static void free_mesh_dev(nmx_ctx *c) {
     c->blane.clear();
     c->filt_key.clear();
   }
-  if (c->dface) { (void)hipFree(c->dface); c->dface = nullptr; }
   drop_stage_graphs(c);
   if (c->gexec) { (void)hipGraphExecDestroy(c->gexec); c->gexec = nullptr; }
   if (c->graph) { (void)hipGraphDestroy(c->graph); c->graph = nullptr; }
@@ -916,18 +912,11 @@ static int upload_mesh(nmx_ctx *c) {
   // element-block copies of the node arrays (every entry written, so no
   // fill), built over element ranges on several threads
   NodeArray h9(c->geom == 1 ? 9 * nn : 1), hx(3 * nn);
-  std::vector<double> h3(3 * ne), hg(8 * ne);
-  std::vector<int> hdom(ne);
   const int geom = c->geom;
   for_element_ranges(ne, [&](unsigned, size_t e0, size_t e1) {
     for (size_t i = e0; i < e1; ++i) {
       const Elm &E = M.e[i];
       long np = (long)E.n * E.n * E.n;
-      for (int d = 0; d < 3; ++d) h3[3 * i + d] = 2. / (E.bbox[2 * d + 1] - E.bbox[2 * d]);
-      for (int q = 0; q < 6; ++q) hg[8 * i + q] = E.bbox[q];
-      hg[8 * i + 6] = M.pat[E.p].s0;
-      hg[8 * i + 7] = M.pat[E.p].s1;
-      hdom[i] = M.pat[E.p].dom;
       for (long q = 0; q < np; ++q) {
         long g = E.off + q;
         if (geom == 1)
@@ -937,15 +926,9 @@ static int upload_mesh(nmx_ctx *c) {
     }
   });
   if (geom != 1) h9[0] = 0.0;
-  if ((r = dev_alloc(&c->dXdx, h9.size())) || (r = dev_alloc(&c->dXbdX, h3.size())) ||
-      (r = dev_alloc(&c->dxyz, hx.size())))
-    return r;
+  if ((r = dev_alloc(&c->dXdx, h9.size())) || (r = dev_alloc(&c->dxyz, hx.size()))) return r;
   HIPCHK(hipMemcpy(c->dXdx, h9.data(), h9.size() * 8, hipMemcpyHostToDevice));
-  HIPCHK(hipMemcpy(c->dXbdX, h3.data(), h3.size() * 8, hipMemcpyHostToDevice));
   HIPCHK(hipMemcpy(c->dxyz, hx.data(), hx.size() * 8, hipMemcpyHostToDevice));
-  if ((r = dev_alloc(&c->degeo, hg.size())) || (r = dev_alloc(&c->dedom, hdom.size()))) return r;
-  HIPCHK(hipMemcpy(c->degeo, hg.data(), hg.size() * 8, hipMemcpyHostToDevice));
-  HIPCHK(hipMemcpy(c->dedom, hdom.data(), hdom.size() * sizeof(int), hipMemcpyHostToDevice));
   c->tcap = 4 * 64;
   if ((r = dev_alloc(&c->dT, c->tcap))) return r;
   if (!c->hT) HIPCHK(hipHostMalloc((void **)&c->hT, c->tcap * sizeof(double), hipHostMallocDefault));
@@ -1005,8 +988,6 @@ static int upload_mesh(nmx_ctx *c) {
     }
     if ((r = dev_upload(&c->dfrec, fr))) return r;
   }
-  if ((r = dev_alloc(&c->dface, hf.size()))) return r;
-  HIPCHK(hipMemcpy(c->dface, hf.data(), hf.size() * sizeof(int4), hipMemcpyHostToDevice));
   const Basis &b = lgl_basis(c->np1);
   std::vector<double> hD(b.D, b.D + c->np1 * c->np1);
   // xb: the element's points per direction (uniform ones on FV elements)
@@ -1626,23 +1607,12 @@ extern "C" int nmx_state_set_profile(nmx_ctx *c, int reg, double t) {
 
 static StageArgs base_args(nmx_ctx *c) {
   StageArgs a;
-  a.dXdx = c->dXdx;
-  a.dXbdX = c->dXbdX;
-  a.xyz = c->dxyz;
-  a.face = c->dface;
-  a.D = c->dD;
   a.tdev = c->dT;
-  a.egeo = c->degeo;
-  a.edom = c->dedom;
-  a.xb = c->dxb;
   a.xcd_map = (P(c, "nmx_xcd") == "yes") ? 1 : 0;
-  a.wend_inv = c->np1 ? 1.0 / lgl_basis(c->np1).w[0] : 0.0;
   kvec(c, a.k);
   a.om = std::sqrt(a.k[0] * a.k[0] + a.k[1] * a.k[1] + a.k[2] * a.k[2]);
   a.profile = (a.k[0] != 0 || a.k[1] != 0 || a.k[2] != 0);
   a.numflux = (P(c, "scalarwave1_numflux") == "LLF") ? 1 : 0;
-  a.e0 = 0;
-  a.e1 = (int)c->mesh.e.size();
   return a;
 }
 
@@ -1753,7 +1723,7 @@ static int launch(nmx_ctx *c, StageArgs a) {
   AmrArgs ca = amr_args(c, a);
   ca.D = c->dD;
   ca.xb = c->dxb;
-  ca.wend_inv = a.wend_inv;
+  ca.wend_inv = 1.0 / lgl_basis(c->np1).w[0];
   ca.rec = c->dfrec;
   ca.nlist = (int)c->mesh.e.size();
   ca.xcd_map = a.xcd_map;

@@ -5,7 +5,7 @@
 
 namespace nmx {
 
-// Arguments of one fused DG RHS + RK stage launch over elements [e0, e1).
+// One fused RHS + RK stage over the mesh, as the host asks for it.
 // Output combinations (each optional):
 //   R    = r                                      (RHS only)
 //   Aout = (Ain ? Ain : win) + cA * r              (RK accumulator "u")
@@ -25,31 +25,13 @@ struct StageArgs {
   double *Aout = nullptr;
   double *Wout = nullptr;
   double *R = nullptr;
-  const double *dXdx = nullptr;  // [e][9][np]
-  const double *dXbdX = nullptr; // [e][3]
-  const double *xyz = nullptr;   // [e][3][np]
-  const int4 *face = nullptr;    // [e][6]: {nb elm (-1 none), local base, s1, s2}
-  const double *D = nullptr;     // D[i*np + l]
   const double *tdev = nullptr;  // stage times on the device; t = tdev[tidx]
-  const double *egeo = nullptr;  // [e][8]: patch bbox of the element (6), s0, s1
-  const int *edom = nullptr;     // [e]: cubed-sphere domain of the element's patch
-  const double *xb = nullptr;    // LGL nodes on [-1,1]
   int tidx = 0;
   int xcd_map = 0;               // 1: contiguous element ranges per XCD
-  double cA = 0, cW = 0, wend_inv = 0;
+  double cA = 0, cW = 0;
   double k[3] = {0, 0, 0};
   double om = 0;
-  int e0 = 0, e1 = 0;
   int wmode = 0, numflux = 0, profile = 0;
-  int fv_mid = 0;                // FV elements: metric and normal at the midpoints
-  // FV elements: fv_divf_extrap_s1, _s2, _opt (ex_on: s1 > 0 or s2 < DBL_MAX)
-  double ex_s1 = 0, ex_s2 = 1.7976931348623157e308;
-  int ex_opt = 0, ex_on = 0;
-  // fv_rec's end midpoints: recend 0 (_2 modes), 1 (_1), 2 (WENOm3/5/Z with
-  // fv_rec_WENOm_s1/_s2/_opt; rec_on: s1 > 0 or s2 < DBL_MAX)
-  int recend = 0, rec_opt = 0, rec_on = 0;
-  int rec_first = 0;               // fv_rec = 1 (first order)
-  double rec_s1 = 0, rec_s2 = 1.7976931348623157e308;
 };
 
 // the mesh's dt from the device's node coordinates (update_elm_eid_dt with
