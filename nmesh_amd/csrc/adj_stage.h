@@ -20,10 +20,11 @@
 //   y_phi = 0.
 // What the readers hand back to a face plane:
 //   copy faces (the relation is mutual): the partner's s A(n) lam at the same
-//     point.  Its normal is the opposite of this element's and |dX/dx| along
-//     the face is the same on both sides, so it is this face's scale, times
-//     the ratio of the two elements' dXb/dX, times A(-n) lam_partner: only the
-//     partner's values are gathered;
+//     point.  Its normal is the opposite of this element's, and its scale
+//     s this face's times a factor constant on the face (fg, AdjRec: the ratio
+//     of the two elements' dXb/dX, and at the interface of two shells, where
+//     |dlam/dx| jumps, of their thicknesses): only the partner's values are
+//     gathered;
 //   interpolated faces (surface.c:1081-1337, interpolate.c:296-363): T = R1^T
 //     (w G) R2 of every (receiving face, neighbour) job that reads the plane, G
 //     = s A(n) lam at the receiving points, w = 1 / count where several

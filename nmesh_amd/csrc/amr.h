@@ -105,8 +105,8 @@ struct FilterArgs {
 // ---------------------------------------------------------------------------
 
 // One element, as the adjoint reads it.  fkind 0 outer boundary; 1 copy, with
-// the partner as in SlotRec and fg the partner's dXb/dX along the face over
-// this element's; 2 interpolated: foff the face's first entry in
+// the partner as in SlotRec and fg the partner's lift scale over this
+// element's; 2 interpolated: foff the face's first entry in
 // AdjArgs::reads, fs1 their number.
 struct AdjRec {
   SlotRec s;

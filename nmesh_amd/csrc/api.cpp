@@ -2732,6 +2732,19 @@ static AdjArgs adj_base_args(nmx_ctx *c) {
   return a;
 }
 
+// The lift scale of face g of N, whose points are those of E's face f, over
+// that of f: the ratio of dXb/dX along the faces and of |dX/dx|, which is the
+// same on both sides (boxes; A and B faces of shells, for A and B run over [-1,
+// 1] in all of them) but for lam, which a shell's thickness scales.
+static double adj_scale_ratio(const Mesh &M, const Elm &E, int f, const Elm &N, int g) {
+  auto width = [&M](const Elm &Q, int d) {
+    const Patch &T = M.pat[Q.p];
+    const double w = Q.bbox[2 * d + 1] - Q.bbox[2 * d];
+    return T.type == PAT_CUBEDSHELL && d == 0 ? w * (T.s1 - T.s0) : w;
+  };
+  return width(E, f >> 1) / width(N, g >> 1);
+}
+
 // The adjoint's tables (made once per mirror, at the first adjoint call): per
 // element its record, with the copy partner or the planes that belong to each
 // face; per job its transposed plane in T.  Every gather is checked here.
@@ -2768,7 +2781,7 @@ static int adj_prepare(nmx_ctx *c) {
       A.s.foff[f] = 5 * N.off + base;
       A.s.fs1[f] = fc.s1;
       A.s.fs2[f] = fc.s2;
-      A.fg[f] = (E.bbox[2 * (f >> 1) + 1] - E.bbox[2 * (f >> 1)]) / (N.bbox[2 * (g >> 1) + 1] - N.bbox[2 * (g >> 1)]);
+      A.fg[f] = adj_scale_ratio(M, E, f, N, g);
     }
   }
   const int nj = (int)c->hadjj.size();
