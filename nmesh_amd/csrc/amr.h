@@ -62,8 +62,9 @@ struct AmrArgs {
   // launches over several orders: D and nodes of order n at batch_doff(n) and
   // batch_xoff(n), 1 / (end weight) at [n]
   const double *Dall = nullptr, *xball = nullptr, *wall = nullptr;
-  const double *tdev = nullptr;
+  const double *tdev = nullptr;   // the stage's time is tdev[tidx], t without tdev
   int tidx = 0;
+  double t = 0;
   double cA = 0, cW = 0, wend_inv = 0;
   double k[3] = {0, 0, 0};
   double om = 0;

@@ -1621,7 +1621,7 @@ static AmrArgs amr_args(nmx_ctx *c, const StageArgs &sa) {
   a.win = sa.win; a.U = sa.U; a.Wa = sa.Wa; a.Wb = sa.Wb; a.Ain = sa.Ain; a.Aout = sa.Aout; a.Wout = sa.Wout; a.R = sa.R;
   a.aj = c->daj;
   a.mdesc = c->dmdesc;
-  a.dXdx = c->dXdx; a.xyz = c->dxyz; a.tdev = sa.tdev; a.tidx = sa.tidx;
+  a.dXdx = c->dXdx; a.xyz = c->dxyz; a.tdev = sa.tdev; a.tidx = sa.tidx; a.t = sa.t;
   a.cA = sa.cA; a.cW = sa.cW;
   for (int d = 0; d < 3; ++d) a.k[d] = sa.k[d];
   a.om = sa.om; a.wmode = sa.wmode; a.numflux = sa.numflux; a.profile = sa.profile;
@@ -1746,30 +1746,36 @@ static int launch(nmx_ctx *c, StageArgs a) {
   return NMX_OK;
 }
 
-// The stage times in hT to the device, for the wave in the exterior: nothing
-// reads them without one, and the copies, with the waits until hT is free, are a
-// good part of a call on a small mesh (64 elements of 5^3 points: a right-hand
-// side 26 us, 30 with them; 100 RK4 steps 1.51 ms and 1.74).
+// The stage times of steps go to the device from hT, for the wave in the
+// exterior: nothing reads them without one, and the copies, with the waits until
+// hT is free, are a good part of a call on a small mesh (64 elements of 5^3
+// points: 100 RK4 steps 1.51 ms, 1.74 with them).
 static bool times_read(nmx_ctx *c) {
   double k[3];
   kvec(c, k);
   return k[0] != 0 || k[1] != 0 || k[2] != 0;
+}
+// before hT is written: the last copy has read it
+static int times_wait(nmx_ctx *c) {
+  if (times_read(c)) HIPCHK(hipStreamSynchronize(c->stream));
+  return NMX_OK;
 }
 static int send_times(nmx_ctx *c, int n) {
   if (times_read(c)) HIPCHK(hipMemcpyAsync(c->dT, c->hT, n * sizeof(double), hipMemcpyHostToDevice, c->stream));
   return NMX_OK;
 }
 
+// The time goes with the launch: calls follow one another without a wait, so
+// a copy from hT might be overtaken by the next call's write.
 extern "C" int nmx_setrhs(nmx_ctx *c, int reg_out, int reg_in, double t) {
   NEED_DEV(c);
   double *out = reg_ptr(c, reg_out), *in = reg_ptr(c, reg_in);
   if (!out || !in || out == in) return fail(NMX_EINVAL, "bad registers");
-  c->hT[0] = t;
-  if (int r = send_times(c, 1)) return r;
   StageArgs a = base_args(c);
   a.win = in;
   a.R = out;
-  a.tidx = 0;
+  a.tdev = nullptr;
+  a.t = t;
   return launch(c, a);
 }
 
@@ -2477,6 +2483,7 @@ extern "C" int nmx_autotune(nmx_ctx *c) {
   if ((r = dev_alloc(&backup, c->nstate))) return r;
   HIPCHK(hipMemcpyAsync(backup, c->dU, c->nstate * 8, hipMemcpyDeviceToDevice, c->stream));
   const int method = method_id(c);
+  if (int rt = times_wait(c)) return rt;
   stage_times(method, c->time, c->dt, c->hT);
   if (int rt = send_times(c, 4)) return rt;
   hipEvent_t t0, t1;
@@ -2618,7 +2625,6 @@ extern "C" int nmx_evolve(nmx_ctx *c, int nsteps) {
   G &= ~1;   // even: the U/A ping-pong returns to its start
   HIPCHK(hipEventRecord(c->ev0, c->stream));
   int done = 0;
-  const bool waves = times_read(c);
   bool parity = false;   // false: current state in dU
   if (use_graph && nsteps >= G) {
     if (!c->gexec || c->graph_steps != G || c->graph_dt != dt || c->graph_method != method) {
@@ -2640,7 +2646,7 @@ extern "C" int nmx_evolve(nmx_ctx *c, int nsteps) {
     }
     while (nsteps - done >= G) {
       // stage times of the G steps (time = Te + te, main.c:588-624)
-      if (waves) HIPCHK(hipStreamSynchronize(c->stream));   // hT is reused
+      if (int rt = times_wait(c)) return rt;
       for (int s = 0; s < G; ++s) {
         stage_times(method, c->time, dt, c->hT + 4 * s);
         advance_time(c, dt);
@@ -2651,7 +2657,7 @@ extern "C" int nmx_evolve(nmx_ctx *c, int nsteps) {
     }
   }
   for (; done < nsteps; ++done) {
-    if (waves) HIPCHK(hipStreamSynchronize(c->stream));
+    if (int rt = times_wait(c)) return rt;
     stage_times(method, c->time, dt, c->hT);
     if (int rt = send_times(c, 4)) return rt;
     int r = issue_step(c, method, dt, 0, parity);

@@ -105,7 +105,7 @@ __device__ __forceinline__ void stage_face(const AmrArgs &a, const NMX_CONST Slo
       const int kk = (dir == 2) ? pl : fb;
       const double *xp = a.xyz + 3 * R.noff + ii + NP * (jj + NP * kk);
       double w[4];
-      plane_wave(a.k, a.om, xp[0], xp[NP3], xp[2 * NP3], a.tdev[a.tidx], w);
+      plane_wave(a.k, a.om, xp[0], xp[NP3], xp[2 * NP3], a.tdev ? a.tdev[a.tidx] : a.t, w);
 #pragma unroll
       for (int v = 0; v < 4; ++v) ua[v] = cmp[v] == 0 ? w[0] : cmp[v] == 1 ? w[1] : cmp[v] == 2 ? w[2] : w[3];
     }

@@ -25,8 +25,9 @@ struct StageArgs {
   double *Aout = nullptr;
   double *Wout = nullptr;
   double *R = nullptr;
-  const double *tdev = nullptr;  // stage times on the device; t = tdev[tidx]
+  const double *tdev = nullptr;  // stage times on the device: the time is tdev[tidx], t without them
   int tidx = 0;
+  double t = 0;
   int xcd_map = 0;               // 1: contiguous element ranges per XCD
   double cA = 0, cW = 0;
   double k[3] = {0, 0, 0};
