@@ -5,7 +5,7 @@
 
 #include <algorithm>
 #include <atomic>
-#include <system_error>
+#include <exception>
 #include <thread>
 
 namespace nmx {
@@ -79,8 +79,8 @@ hipError_t HostCopy::run(int device, char *d, char *h, size_t bytes, bool up, hi
   int started = 1;
   try {
     for (; started < nt; ++started) th[started] = std::thread(work, started);
-  } catch (const std::system_error &) {
-    // fewer threads take all chunks
+  } catch (const std::exception &) {
+    // no thread, or no memory for its start: fewer threads take all chunks
   }
   work(0);
   for (int t = 1; t < started; ++t) th[t].join();
