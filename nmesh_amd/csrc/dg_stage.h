@@ -48,6 +48,8 @@
 #pragma once
 #include <hip/hip_runtime.h>
 
+#include <type_traits>
+
 #include "amr.h"
 #include "dg_common.h"
 #include "fastmath.h"
@@ -219,30 +221,56 @@ __device__ __forceinline__ void node_lift(const NodeGeo &m, int dir, double sig,
   for (int v = 0; v < 4; ++v) r[v] -= F[v] * scale;
 }
 
-// the stage's output at the node whose first state double is gi
+// What a stage with an accumulator (wmodes 0 to 2) reads at a node besides its
+// own pi and c: u_p, the accumulator and its input's phi.
+struct AccIn {
+  double U[5], A[5], phi;
+};
 template <int WM>
-__device__ __forceinline__ void node_out(const AmrArgs &a, const StageRegs &o, const StageIn &in, long gi,
-                                         const int (&vo)[4], int po, const double u[4], const double r[4]) {
-  if (WM != 0) {
-    double out[5];
-    const bool end = stage_out<true>(o, in, u, r, out);
+using NodeIn = std::conditional_t<WM == 0, AccIn, StageIn>;
+
+// the operands of node_out at the node whose first state double is gi,
+// requested together: between node_out's stores, which they may alias, they were
+// five round trips one after another (3072 shell elements of 8 points: Euler steps
+// 62 us, 41 so, RK4 steps with the MRS limiter 556 and 440; 19,200 elements of 4
+// to 10 points: Euler steps 555 and 453)
+__device__ __forceinline__ void node_in(const AmrArgs &a, const StageRegs &, long gi, const int (&vo)[4], int po,
+                                        AccIn &q) {
+  if (a.wmode) {
 #pragma unroll
-    for (int v = 0; v < 4; ++v) a.Wout[gi + vo[v]] = out[v];
-    if (end) a.Wout[gi + po] = out[4];
-    return;
+    for (int v = 0; v < 5; ++v) q.U[v] = a.U[gi + (v < 4 ? vo[v] : po)];
   }
-  const double rv[5] = {r[0], r[1], r[2], r[3], u[0]};
-  const double *bas = a.Ain ? a.Ain : a.win;
+  if (a.Ain) {
+#pragma unroll
+    for (int v = 0; v < 5; ++v) q.A[v] = a.Ain[gi + (v < 4 ? vo[v] : po)];
+  }
+  if (a.wmode == 2 || (a.Aout && !a.Ain)) q.phi = a.win[gi + po];
+}
+__device__ __forceinline__ void node_in(const AmrArgs &, const StageRegs &o, long gi, const int (&vo)[4], int po,
+                                        StageIn &q) {
+  stage_in(o, gi, vo, po, q);
+}
+
+// the stage's output there
+__device__ __forceinline__ void node_out(const AmrArgs &a, const StageRegs &, const AccIn &q, long gi,
+                                         const int (&vo)[4], int po, const double u[4], const double r[4]) {
 #pragma unroll
   for (int v = 0; v < 5; ++v) {
     const long g = gi + (v < 4 ? vo[v] : po);
-    if (a.R) a.R[g] = rv[v];
-    const double U = a.wmode ? a.U[g] : 0.0;
-    const double wv = a.wmode == 2 ? (v < 4 ? u[v] : a.win[g]) : 0.0;
-    if (a.Aout) a.Aout[g] = bas[g] + a.cA * rv[v];
-    if (a.wmode == 1) a.Wout[g] = U + a.cW * rv[v];
-    else if (a.wmode == 2) a.Wout[g] = 0.75 * U + 0.25 * (wv + a.cW * rv[v]);
+    const double rv = v < 4 ? r[v] : u[0], w = v < 4 ? u[v] : q.phi;
+    if (a.R) a.R[g] = rv;
+    if (a.Aout) a.Aout[g] = (a.Ain ? q.A[v] : w) + a.cA * rv;
+    if (a.wmode == 1) a.Wout[g] = q.U[v] + a.cW * rv;
+    else if (a.wmode == 2) a.Wout[g] = 0.75 * q.U[v] + 0.25 * (w + a.cW * rv);
   }
+}
+__device__ __forceinline__ void node_out(const AmrArgs &a, const StageRegs &o, const StageIn &q, long gi,
+                                         const int (&vo)[4], int po, const double u[4], const double r[4]) {
+  double out[5];
+  const bool end = stage_out<true>(o, q, u, r, out);
+#pragma unroll
+  for (int v = 0; v < 4; ++v) a.Wout[gi + vo[v]] = out[v];
+  if (end) a.Wout[gi + po] = out[4];
 }
 
 // components of c along the patch's axes (dir, ia, ib): cmp[v] is the
@@ -353,8 +381,8 @@ __global__ __launch_bounds__(col_threads(NP), col_waves(NP, WM)) void dg_col_ker
 #pragma unroll
         for (int c = 0; c < 3; ++c) m.M[d][c] = md[(3 * d + c) * NP3];
     }
-    StageIn in;
-    if (WM != 0) stage_in(o, gbase + q + k * NP2, vo, 4 * NP3, in);
+    NodeIn<WM> in;
+    node_in(a, o, gbase + q + k * NP2, vo, 4 * NP3, in);
     __syncthreads();
 
     // ---- derivatives along i (rows of the plane), j and k ----
@@ -412,7 +440,7 @@ __global__ __launch_bounds__(col_threads(NP), col_waves(NP, WM)) void dg_col_ker
       const double ua[4] = {sf[0][q], sf[1][q], sf[2][q], sf[3][q]};
       node_lift<GEOM>(m, 2, k ? 1.0 : -1.0, a.wend_inv, a.numflux, u, ua, r);
     }
-    if (act) node_out<WM>(a, o, in, gbase + q + k * NP2, vo, 4 * NP3, u, r);
+    if (act) node_out(a, o, in, gbase + q + k * NP2, vo, 4 * NP3, u, r);
   }
 }
 
@@ -454,8 +482,8 @@ __device__ __forceinline__ void node_elem(const AmrArgs &a, const NMX_CONST Slot
     stage_face<NP>(a, R, f, q, q % NP, q / NP, cmp, fv[c]);
   }
   const StageRegs o = node_args<WM>(a);
-  StageIn in;
-  if (WM != 0) stage_in(o, gbase + node, vo, 4 * NP3, in);
+  NodeIn<WM> in;
+  node_in(a, o, gbase + node, vo, 4 * NP3, in);
   NodeGeo m;
   node_geo_elem<GEOM>(R, m);
   if (GEOM == 1) {
@@ -522,7 +550,7 @@ __device__ __forceinline__ void node_elem(const AmrArgs &a, const NMX_CONST Slot
       node_lift<GEOM>(m, dir, side ? 1.0 : -1.0, wend_inv, a.numflux, u, ua, r);
     }
   }
-  node_out<WM>(a, o, in, gbase + node, vo, 4 * NP3, u, r);
+  node_out(a, o, in, gbase + node, vo, 4 * NP3, u, r);
 }
 
 template <int NP, int GEOM, int WM>

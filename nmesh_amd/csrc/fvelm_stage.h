@@ -440,7 +440,11 @@ __global__ __launch_bounds__(3 * fve_line_threads(NP), 2) void fvelm_kernel(AmrA
   // requested a node ahead
   const StageRegs o = {a.win, a.U, a.Wa, a.Wb, a.cA, a.cW, a.wmode};
   StageIn in;
-  if (a.wmode >= 3 && tid < NP3) stage_in(o, gbase + tid, vo, 4 * NP3, in);
+  AccIn acc_in;
+  if (tid < NP3) {
+    if (a.wmode >= 3) node_in(a, o, gbase + tid, vo, 4 * NP3, in);
+    else node_in(a, o, gbase + tid, vo, 4 * NP3, acc_in);
+  }
   __syncthreads();
 #pragma unroll 1
   for (int node = tid; node < NP3; node += NT) {
@@ -462,14 +466,12 @@ __global__ __launch_bounds__(3 * fve_line_threads(NP), 2) void fvelm_kernel(AmrA
     }
     if (a.wmode >= 3) {
       const StageIn q = in;
-      if (node + NT < NP3) stage_in(o, gi + NT, vo, 4 * NP3, in);
-      double out[5];
-      const bool end = stage_out<true>(o, q, u, r, out);
-#pragma unroll
-      for (int v = 0; v < 4; ++v) a.Wout[gi + vo[v]] = out[v];
-      if (end) a.Wout[gi + 4 * NP3] = out[4];
+      if (node + NT < NP3) node_in(a, o, gi + NT, vo, 4 * NP3, in);
+      node_out(a, o, q, gi, vo, 4 * NP3, u, r);
     } else {
-      node_out<0>(a, o, in, gi, vo, 4 * NP3, u, r);
+      const AccIn q = acc_in;
+      if (node + NT < NP3) node_in(a, o, gi + NT, vo, 4 * NP3, acc_in);
+      node_out(a, o, q, gi, vo, 4 * NP3, u, r);
     }
   }
 }
