@@ -388,6 +388,9 @@ static void free_mesh_dev(nmx_ctx *c) {
       if (*q) { (void)hipFree(*q); *q = nullptr; }
     c->adj_ready = false;
     c->adjorders.clear();
+    c->hadjj.clear();
+    c->hadjsend.clear();
+    c->adjnjobs = 0;
   }
   if (c->agexec) { (void)hipGraphExecDestroy(c->agexec); c->agexec = nullptr; }
   if (c->agraph) { (void)hipGraphDestroy(c->agraph); c->agraph = nullptr; }
