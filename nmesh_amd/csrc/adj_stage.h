@@ -21,8 +21,8 @@
 // What the readers hand back to a face plane:
 //   copy faces (the relation is mutual): the partner's s A(n) lam at the same
 //     point.  Its normal is the opposite of this element's, and its scale
-//     s this face's times a factor constant on the face (fg, AdjRec: the ratio
-//     of the two elements' dXb/dX, and at the interface of two shells, where
+//     s this face's times a factor constant on the face (fg, AdjArgs: the
+//     ratio of the two elements' dXb/dX, and at the interface of two shells, where
 //     |dlam/dx| jumps, of their thicknesses): only the partner's values are
 //     gathered;
 //   interpolated faces (surface.c:1081-1337, interpolate.c:296-363): T = R1^T
@@ -48,13 +48,13 @@ namespace nmx {
 constexpr int adj_fields(int geom) { return geom == 2 ? 7 : geom == 0 ? 4 : 12; }
 
 template <int NP, int GEOM, int WM, int NT>
-__device__ __forceinline__ void adj_elem(const AdjArgs &a, const NMX_CONST AdjRec &AR, const double *D,
+__device__ __forceinline__ void adj_elem(const AdjArgs &a, int it, const double *D,
                                          const double *xb, double wend_inv, double *l_t, double *l_f,
                                          double *s_D) {
   constexpr int NP2 = NP * NP;
   constexpr int NP3 = NP * NP * NP;
   constexpr int NQ = (6 * NP2 + NT - 1) / NT;   // face points per thread
-  const NMX_CONST SlotRec &R = AR.s;
+  const NMX_CONST SlotRec &R = as_const(a.rec)[it];
   double(*s_t)[NP3] = reinterpret_cast<double(*)[NP3]>(l_t);
   double(*s_f)[4][NP2] = reinterpret_cast<double(*)[4][NP2]>(l_f);
   const int tid = threadIdx.x;
@@ -203,7 +203,7 @@ __device__ __forceinline__ void adj_elem(const AdjArgs &a, const NMX_CONST AdjRe
       for (int v = 0; v < 4; ++v) r[v] -= scale * F[v];
       if (R.fkind[2 * dir + side] == 1) {
         const double opp[3] = {-nrm[0], -nrm[1], -nrm[2]};
-        const double sc = scale * AR.fg[2 * dir + side];
+        const double sc = scale * as_const(a.fg)[6 * it + 2 * dir + side];
         face_flux(a.numflux, opp, fa[0], fa + 1, F);
 #pragma unroll
         for (int v = 0; v < 4; ++v) r[v] += sc * F[v];
@@ -239,8 +239,7 @@ __global__ __launch_bounds__(node_threads(NP)) void adj_node_kernel(AdjArgs a) {
   __shared__ double s_D[NP * NP];
   const int it = xcd_block(a.nlist, a.xcd_map);
   if (it >= a.nlist) return;
-  adj_elem<NP, GEOM, WM, node_threads(NP)>(a, as_const(a.rec)[it], a.Dall + batch_doff(NP),
-                                           a.xball + batch_xoff(NP), as_const(a.wall)[NP], s_t, s_f, s_D);
+  adj_elem<NP, GEOM, WM, node_threads(NP)>(a, it, a.D, a.xb, a.wend_inv, s_t, s_f, s_D);
 }
 
 // elements of every order in one launch (dg_mixed_kernel, dg_stage.h)
@@ -251,13 +250,12 @@ __global__ __launch_bounds__(node_threads(NMAX)) void adj_mixed_kernel(AdjArgs a
   __shared__ double s_D[NMAX * NMAX];
   const int it = xcd_block(a.nlist, a.xcd_map);
   if (it >= a.nlist) return;
-  const NMX_CONST AdjRec &R = as_const(a.rec)[it];
-  switch (R.s.n) {
+  switch (as_const(a.rec)[it].n) {
 #define NMX_CASE(N)                                                                                       \
   case N:                                                                                                 \
     if (N <= NMAX)                                                                                        \
       adj_elem<N <= NMAX ? N : 2, GEOM, WM, node_threads(NMAX)>(                                          \
-          a, R, a.Dall + batch_doff(N), a.xball + batch_xoff(N), as_const(a.wall)[N], s_t, s_f, s_D);     \
+          a, it, a.Dall + batch_doff(N), a.xball + batch_xoff(N), as_const(a.wall)[N], s_t, s_f, s_D);     \
     break;
     NMX_CASE(2)
     NMX_CASE(3)
@@ -299,7 +297,7 @@ __device__ __forceinline__ void adj_job(const AdjArgs &a, const NMX_CONST AdjJob
   const int nx2 = (sw ? J.a1 - J.a0 : J.b1 - J.b0) + 1;
   const double *R1 = a.Btab + (sw ? J.offB : J.offA) + x1lo * m;
   const double *R2 = a.Btab + (sw ? J.offA : J.offB) + x2lo * m;
-  const NMX_CONST SlotRec &R = as_const(a.erec)[J.e].s;
+  const NMX_CONST SlotRec &R = as_const(a.erec)[J.e];
   const double *lam = a.lam + 5 * R.noff;
   const double *xb = a.xball + batch_xoff(N);
   const double wend_inv = as_const(a.wall)[N];

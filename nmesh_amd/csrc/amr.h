@@ -105,17 +105,6 @@ struct FilterArgs {
 // Discrete adjoint (adj_stage.h)
 // ---------------------------------------------------------------------------
 
-// One element, as the adjoint reads it.  fkind 0 outer boundary; 1 copy, with
-// the partner as in SlotRec and fg the partner's lift scale over this
-// element's; 2 interpolated: foff the face's first entry in
-// AdjArgs::reads, fs1 their number.
-struct AdjRec {
-  SlotRec s;
-  double fg[6];
-  double pad[2];
-};
-static_assert(sizeof(AdjRec) == 320, "AdjRec is 320 bytes");
-
 // a transposed plane [4][n*n] that belongs to a face: the value of variable v
 // at face point (a, b) is T[off + v n n + a ca + b cb]
 struct AdjRead {
@@ -124,7 +113,7 @@ struct AdjRead {
 
 // one (receiving face, neighbour) interpolation job, transposed
 struct AdjJob {
-  int e, g;             // receiving element and face
+  int e, g;             // receiving element (its record in AdjArgs::erec) and face
   int n, m;             // points per direction of the receiver and of the neighbour
   int sw, a0, a1, b0, b1;   // the forward job's axis swap and covered points
   int offA, offB;       // rows for the receiver's a and b points in Btab (m doubles each)
@@ -150,13 +139,20 @@ struct AdjArgs {
   double cA = 0, cW = 0;
   int wmode = 0;
   int numflux = 0, xcd_map = 0;
-  const AdjRec *rec = nullptr;    // this launch's elements
+  // this launch's elements: fkind 0 outer boundary; 1 copy, the partner as the
+  // forward stage gathers it; 2 interpolated: foff the face's first entry in
+  // reads, fs1 their number.  fg[6 el + f]: at a copy face the partner's lift
+  // scale over this element's
+  const SlotRec *rec = nullptr;
+  const double *fg = nullptr;
   int nlist = 0;
-  const AdjRec *erec = nullptr;   // [e]: every element
+  const SlotRec *erec = nullptr;  // every element, for the jobs
   const AdjRead *reads = nullptr;
   const double *dXdx = nullptr;   // element blocks of 9*np (stored geometry)
-  // D and LGL nodes of order n at batch_doff(n) and batch_xoff(n), 1 / (end
-  // weight) at [n]
+  // the order's D, LGL nodes and 1 / (end weight); for launches over several
+  // orders and the jobs those of order n at batch_doff(n), batch_xoff(n) and [n]
+  const double *D = nullptr, *xb = nullptr;
+  double wend_inv = 0;
   const double *Dall = nullptr, *xball = nullptr, *wall = nullptr;
   const AdjJob *jobs = nullptr;
   int njobs = 0;

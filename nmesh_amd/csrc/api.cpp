@@ -133,13 +133,14 @@ struct nmx_ctx {
   bool tuned = false;
   // adjoint: lam register, its own graph cache, and the checkpoint pool
   double *dL = nullptr;
-  // the interpolation jobs as the forward tables made them (host), then, from
-  // the first adjoint call on, the device tables: one record per element in
-  // element order and by decreasing order, the planes that belong to each
-  // face, the jobs and their planes
+  // each copy face's ratio of lift scales; on batched meshes the interpolation
+  // jobs as the forward tables made them (host) and, from the first adjoint call
+  // on, the elements' records by decreasing order, the planes that belong to
+  // each face, the jobs and their planes
   std::vector<AdjJob> hadjj;
   std::vector<int> hadjsend;   // per job: sender element, sender face
-  AdjRec *dadje = nullptr, *dadjr = nullptr;
+  SlotRec *dadjr = nullptr;
+  double *dadjfg = nullptr;
   AdjRead *dadjp = nullptr;
   AdjJob *dadjj = nullptr;
   double *dadjT = nullptr;
@@ -382,7 +383,7 @@ static void free_mesh_dev(nmx_ctx *c) {
                      (void **)&c->dcrcaw, (void **)&c->dcrcypow,
                      (void **)&c->dcrcpart, (void **)&c->dcrcout, (void **)&c->dnbr,
                      (void **)&c->dlimh, (void **)&c->dwqall, (void **)&c->dldat, (void **)&c->dlimhw,
-                     (void **)&c->damat, (void **)&c->dsmat, (void **)&c->dadje, (void **)&c->dadjr,
+                     (void **)&c->damat, (void **)&c->dsmat, (void **)&c->dadjfg, (void **)&c->dadjr,
                      (void **)&c->dadjp, (void **)&c->dadjj, (void **)&c->dadjT};
     for (auto q : ptrs)
       if (*q) { (void)hipFree(*q); *q = nullptr; }
@@ -578,6 +579,19 @@ static void slot_geometry(const Mesh &M, int e, SlotRec &R) {
   R.s1 = M.pat[E.p].s1;
   R.dom = M.pat[E.p].dom;
   R.n = E.n;
+}
+
+// The lift scale of face g of N, whose points are those of E's face f, over
+// that of f: the ratio of dXb/dX along the faces and of |dX/dx|, which is the
+// same on both sides (boxes; A and B faces of shells, for A and B run over [-1,
+// 1] in all of them) but for lam, which a shell's thickness scales.
+static double adj_scale_ratio(const Mesh &M, const Elm &E, int f, const Elm &N, int g) {
+  auto width = [&M](const Elm &Q, int d) {
+    const Patch &T = M.pat[Q.p];
+    const double w = Q.bbox[2 * d + 1] - Q.bbox[2 * d];
+    return T.type == PAT_CUBEDSHELL && d == 0 ? w * (T.s1 - T.s0) : w;
+  };
+  return width(E, f >> 1) / width(N, g >> 1);
 }
 
 // Launch order and lanes of the concurrent buckets, largest first.  Running
@@ -975,8 +989,9 @@ static int upload_mesh(nmx_ctx *c) {
       hf[6 * i + f] = d;
     }
   {
-    // every element, for the stage kernel and the filter
+    // every element, for the stage kernels and the filter
     std::vector<SlotRec> fr(ne);
+    std::vector<double> fg(6 * ne, 1.0);
     const long np3 = (long)c->np1 * c->np1 * c->np1;
     for (size_t i = 0; i < ne; ++i) {
       slot_geometry(M, (int)i, fr[i]);
@@ -987,9 +1002,10 @@ static int upload_mesh(nmx_ctx *c) {
         fr[i].foff[f] = 5 * np3 * d.x + d.y;
         fr[i].fs1[f] = d.z;
         fr[i].fs2[f] = d.w;
+        fg[6 * i + f] = adj_scale_ratio(M, M.e[i], f, M.e[d.x], M.e[i].nbf[f][0]);
       }
     }
-    if ((r = dev_upload(&c->dfrec, fr))) return r;
+    if ((r = dev_upload(&c->dfrec, fr)) || (!c->fvelm && (r = dev_upload(&c->dadjfg, fg)))) return r;
   }
   const Basis &b = lgl_basis(c->np1);
   std::vector<double> hD(b.D, b.D + c->np1 * c->np1);
@@ -2734,44 +2750,49 @@ static AdjArgs adj_base_args(nmx_ctx *c) {
   AdjArgs a;
   a.dXdx = c->dXdx;
   a.Dall = c->dbD; a.xball = c->dbxb; a.wall = c->dbW;
-  a.erec = c->dadje; a.reads = c->dadjp; a.jobs = c->dadjj; a.njobs = c->adjnjobs; a.T = c->dadjT;
+  a.fg = c->dadjfg;
+  a.erec = c->dadjr; a.reads = c->dadjp; a.jobs = c->dadjj; a.njobs = c->adjnjobs; a.T = c->dadjT;
   a.mdesc = c->dmdesc; a.Btab = c->dBtab;
   a.numflux = (P(c, "scalarwave1_numflux") == "LLF") ? 1 : 0;
   a.xcd_map = (P(c, "nmx_xcd") == "yes") ? 1 : 0;
   return a;
 }
 
-// The lift scale of face g of N, whose points are those of E's face f, over
-// that of f: the ratio of dXb/dX along the faces and of |dX/dx|, which is the
-// same on both sides (boxes; A and B faces of shells, for A and B run over [-1,
-// 1] in all of them) but for lam, which a shell's thickness scales.
-static double adj_scale_ratio(const Mesh &M, const Elm &E, int f, const Elm &N, int g) {
-  auto width = [&M](const Elm &Q, int d) {
-    const Patch &T = M.pat[Q.p];
-    const double w = Q.bbox[2 * d + 1] - Q.bbox[2 * d];
-    return T.type == PAT_CUBEDSHELL && d == 0 ? w * (T.s1 - T.s0) : w;
-  };
-  return width(E, f >> 1) / width(N, g >> 1);
-}
-
-// The adjoint's tables (made once per mirror, at the first adjoint call): per
-// element its record, with the copy partner or the planes that belong to each
-// face; per job its transposed plane in T.  Every gather is checked here.
+// The adjoint's tables of a batched mesh (made once per mirror, at the first
+// adjoint call): per element its record, with the copy partner or the planes
+// that belong to each face; per job its transposed plane in T.  Every gather is
+// checked here.  Conforming meshes have theirs from the mirror (upload_mesh):
+// their first call makes none.
 static int adj_prepare(nmx_ctx *c) {
   if (c->adj_ready) return NMX_OK;
   const Mesh &M = c->mesh;
   const int ne = (int)M.e.size();
+  if (!c->amr) {
+    c->adjorders.assign(1, {c->np1, ne});
+    c->adj_ready = true;
+    return NMX_OK;
+  }
   int r;
-  if (!c->dbD && (r = upload_order_tables(c))) return r;
-  std::vector<AdjRec> rec(ne);
+  // the elements by decreasing order
+  std::vector<int> list(ne), place(ne);
+  for (int e = 0; e < ne; ++e) list[e] = e;
+  std::stable_sort(list.begin(), list.end(), [&](int x, int y) { return M.e[x].n > M.e[y].n; });
+  c->adjorders.clear();
+  for (int q = 0; q < ne; ++q) {
+    const int n = M.e[list[q]].n;
+    place[list[q]] = q;
+    if (c->adjorders.empty() || c->adjorders.back().first != n) c->adjorders.push_back({n, 0});
+    c->adjorders.back().second++;
+  }
+  std::vector<SlotRec> rec(ne);
+  std::vector<double> fg(6L * ne, 1.0);
   for (int e = 0; e < ne; ++e) {
     const Elm &E = M.e[e];
-    AdjRec &A = rec[e];
-    std::memset(&A, 0, sizeof A);
-    slot_geometry(M, e, A.s);
+    SlotRec &A = rec[place[e]];
+    slot_geometry(M, e, A);
     for (int f = 0; f < 6; ++f) {
       if (E.ajmode[f] == 0) continue;
-      if (E.ajmode[f] != 1 && E.ajmode[f] != 2) { A.s.fkind[f] = 2; continue; }
+      if (E.ajmode[f] != 1 && E.ajmode[f] != 2) { A.fkind[f] = 2; continue; }
       const FaceCopy &fc = M.fcopy[6L * e + f];
       const int nb = E.fnb[f][0], g = E.nbf[f][0], n = E.n;
       if (nb < 0 || nb >= ne || M.e[nb].n != n || g < 0 || g > 5)
@@ -2786,16 +2807,15 @@ static int adj_prepare(nmx_ctx *c) {
           const int I[3] = {(int)(p % n), (int)((p / n) % n), (int)(p / ((long)n * n))};
           if (I[g >> 1] != (g & 1) * (n - 1)) return fail(NMX_EINVAL, "adjoint: copy partner face");
         }
-      A.s.fkind[f] = 1;
-      A.s.foff[f] = 5 * N.off + base;
-      A.s.fs1[f] = fc.s1;
-      A.s.fs2[f] = fc.s2;
-      A.fg[f] = adj_scale_ratio(M, E, f, N, g);
+      A.fkind[f] = 1;
+      A.foff[f] = 5 * N.off + base;
+      A.fs1[f] = fc.s1;
+      A.fs2[f] = fc.s2;
+      fg[6L * place[e] + f] = adj_scale_ratio(M, E, f, N, g);
     }
   }
   const int nj = (int)c->hadjj.size();
   std::vector<AdjJob> jobs = c->hadjj;
-  std::vector<std::vector<AdjRead>> byface(6L * ne);
   long tlen = 0;
   for (int j = 0; j < nj; ++j) {
     AdjJob &J = jobs[j];
@@ -2803,7 +2823,7 @@ static int adj_prepare(nmx_ctx *c) {
     J.toff = (int)tlen;
     tlen += 4L * J.m * J.m;
     const int se = c->hadjsend[2 * j], sf = c->hadjsend[2 * j + 1];
-    if (se < 0 || se >= ne || M.e[se].n != J.m || rec[se].s.fkind[sf] != 2)
+    if (se < 0 || se >= ne || M.e[se].n != J.m || rec[place[se]].fkind[sf] != 2)
       return fail(NMX_EINVAL, "adjoint: a job reads a plane that is not an interpolated face");
     if (J.e < 0 || J.e >= ne || M.e[J.e].n != J.n || J.g < 0 || J.g > 5)
       return fail(NMX_EINVAL, "adjoint: job receiver out of range");
@@ -2813,29 +2833,30 @@ static int adj_prepare(nmx_ctx *c) {
         const int q1 = J.A1 * (fa - J.A0) + J.B1 * (fb - J.B0), q2 = J.A2 * (fa - J.A0) + J.B2 * (fb - J.B0);
         if (q1 < 0 || q1 >= J.m || q2 < 0 || q2 >= J.m) return fail(NMX_EINVAL, "adjoint: plane map out of range");
       }
+    rec[place[se]].fs1[sf]++;
+  }
+  // the planes face by face
+  long nreads = 0;
+  for (int q = 0; q < ne; ++q)
+    for (int f = 0; f < 6; ++f)
+      if (rec[q].fkind[f] == 2) {
+        rec[q].foff[f] = nreads;
+        nreads += rec[q].fs1[f];
+        rec[q].fs1[f] = 0;
+      }
+  std::vector<AdjRead> reads(nreads);
+  for (int j = 0; j < nj; ++j) {
+    AdjJob &J = jobs[j];
+    SlotRec &A = rec[place[c->hadjsend[2 * j]]];
+    const int sf = c->hadjsend[2 * j + 1];
     // T(q1 + m q2) with q1, q2 affine in the face point
     const int ka = J.A1 + J.m * J.A2, kb = J.B1 + J.m * J.B2;
-    byface[6L * se + sf].push_back({J.toff - J.A0 * ka - J.B0 * kb, ka, kb});
-  }
-  std::vector<AdjRead> reads;
-  for (int e = 0; e < ne; ++e)
-    for (int f = 0; f < 6; ++f)
-      if (rec[e].s.fkind[f] == 2) {
-        const auto &b = byface[6L * e + f];
-        rec[e].s.foff[f] = (long)reads.size();
-        rec[e].s.fs1[f] = (int)b.size();
-        reads.insert(reads.end(), b.begin(), b.end());
-      }
-  std::vector<AdjRec> sorted = rec;
-  std::stable_sort(sorted.begin(), sorted.end(), [](const AdjRec &x, const AdjRec &y) { return x.s.n > y.s.n; });
-  c->adjorders.clear();
-  for (const AdjRec &A : sorted) {
-    if (c->adjorders.empty() || c->adjorders.back().first != A.s.n) c->adjorders.push_back({A.s.n, 0});
-    c->adjorders.back().second++;
+    reads[A.foff[sf] + A.fs1[sf]++] = {J.toff - J.A0 * ka - J.B0 * kb, ka, kb};
+    J.e = place[J.e];
   }
   if (jobs.empty()) jobs.resize(1);
   if (reads.empty()) reads.resize(1);
-  if ((r = dev_upload(&c->dadje, rec)) || (r = dev_upload(&c->dadjr, sorted)) || (r = dev_upload(&c->dadjp, reads)) ||
+  if ((r = dev_upload(&c->dadjfg, fg)) || (r = dev_upload(&c->dadjr, rec)) || (r = dev_upload(&c->dadjp, reads)) ||
       (r = dev_upload(&c->dadjj, jobs)) || (r = dev_alloc(&c->dadjT, tlen > 0 ? tlen : 1)))
     return r;
   c->adjnjobs = nj;
@@ -2875,13 +2896,17 @@ static int launch_adj(nmx_ctx *c, AdjArgs a) {
   const int lanes = P(c, "nmx_concurrent") == "yes" ? std::min(no, (int)nmx_ctx::kLanes) : 1;
   if (lanes > 1) HIPCHK(hipEventRecord(c->evfork, c->stream));
   for (int l = 1; l < lanes; ++l) HIPCHK(hipStreamWaitEvent(c->helper[l - 1], c->evfork, 0));
-  a.rec = c->dadjr;
+  a.rec = c->amr ? c->dadjr : c->dfrec;
   for (int b = 0; b < no; ++b) {
-    const int l = b % lanes;
+    const int l = b % lanes, n = c->adjorders[b].first;
     a.nlist = c->adjorders[b].second;
-    err = launch_adj(c->adjorders[b].first, c->adjorders[b].first, c->geom, a, l ? c->helper[l - 1] : c->stream);
+    a.D = c->amr ? c->dbD + batch_doff(n) : c->dD;
+    a.xb = c->amr ? c->dbxb + batch_xoff(n) : c->dxb;
+    a.wend_inv = 1.0 / lgl_basis(n).w[0];
+    err = launch_adj(n, n, c->geom, a, l ? c->helper[l - 1] : c->stream);
     if (err != hipSuccess) return fail(NMX_EHIP, std::string("adjoint launch: ") + hipGetErrorString(err));
     a.rec += a.nlist;
+    a.fg += 6L * a.nlist;
   }
   for (int l = 1; l < lanes; ++l) {
     HIPCHK(hipEventRecord(c->evjoin[l - 1], c->helper[l - 1]));
