@@ -102,7 +102,8 @@ int nmx_synchronize(nmx_ctx *ctx);
  * nmx_autotune: yes|no, nmx_batch: buckets|persistent (the batched path's DG
  * launches per stage: one per order, side by side, or one over all orders;
  * the autotuner times both unless it is set; legacy is another name of
- * buckets); accepted without effect: nmx_block (full|half|quarter) and
+ * buckets), nmx_inturn: no|yes (that path's launches of a stage side by side
+ * on several streams, or in turn on one; timed likewise); accepted without effect: nmx_block (full|half|quarter) and
  * nmx_stream_hints (0..7)). */
 int nmx_set_param(nmx_ctx *ctx, const char *name, const char *value);
 int nmx_get_param(nmx_ctx *ctx, const char *name, char *buf, int buflen);

@@ -91,7 +91,8 @@ struct nmx_ctx {
   nmx_trouble_fn trouble_hook = nullptr;
   void *trouble_user = nullptr;
   long trouble_redos = 0, trouble_switches = 0;
-  bool batch_fixed = false;   // nmx_batch set by the caller (the autotuner leaves it)
+  // nmx_batch, nmx_inturn set by the caller (the autotuner leaves them)
+  bool batch_fixed = false, turn_fixed = false;
   struct Bucket {
     int n; int count; SlotRec *drec; long doff; long xoff;
     float ms;   // tuned stage time alone (0: not tuned)
@@ -125,7 +126,6 @@ struct nmx_ctx {
   static constexpr int kLanes = 4;     // stream lanes of the concurrent buckets
   std::vector<int> border;             // buckets by decreasing node count
   std::vector<int> blane;              // lane of each bucket
-  bool inturn = false;                 // the launches of a stage in turn on one lane
   hipStream_t helper[kHelpers] = {};
   hipEvent_t evfork = nullptr, evjoin[kHelpers] = {};
   // the faces with several neighbours run beside the single-neighbour ones
@@ -250,6 +250,7 @@ static void set_defaults(nmx_ctx *c) {
       {"nmx_autotune", "yes"},
       {"nmx_concurrent", "yes"},
       {"nmx_batch", "legacy"},
+      {"nmx_inturn", "no"},
       {"nmx_stream_hints", "0"},
       {"nmx_trouble", "none"},
       {"nmx_trouble_delta0", "1e-4"},
@@ -469,6 +470,8 @@ extern "C" int nmx_set_param(nmx_ctx *c, const char *name, const char *value) {
     return fail(NMX_EINVAL, "evolve_redo_troubled must be step or substep");
   if (k == "nmx_batch" && v != "persistent" && v != "buckets" && v != "legacy")
     return fail(NMX_EINVAL, "nmx_batch must be persistent, buckets or legacy");
+  if (k == "nmx_inturn" && v != "yes" && v != "no")
+    return fail(NMX_EINVAL, "nmx_inturn must be yes or no");
   if (k == "nmx_path" && v != "plain" && v != "perelement" && v != "batched")
     return fail(NMX_EINVAL, "nmx_path must be plain, perelement or batched");
   if (k == "nmx_geometry" && v != "analytic" && v != "stored")
@@ -515,6 +518,7 @@ extern "C" int nmx_set_param(nmx_ctx *c, const char *name, const char *value) {
   c->par[k] = v;
   if (k == "nmx_block" || k == "nmx_xcd") c->tuned = true;   // explicit choice wins
   if (k == "nmx_batch") c->batch_fixed = true;
+  if (k == "nmx_inturn") c->turn_fixed = true;
   drop_stage_graphs(c);
   if (c->gexec) { (void)hipGraphExecDestroy(c->gexec); c->gexec = nullptr; }
   if (c->graph) { (void)hipGraphDestroy(c->graph); c->graph = nullptr; }
@@ -884,7 +888,6 @@ static int upload_amr_tables(nmx_ctx *c) {
 static int upload_mesh(nmx_ctx *c) {
   free_mesh_dev(c);
   c->tuned = false;
-  c->inturn = false;
   Mesh &M = c->mesh;
   const long nn = M.nnodes;
   const size_t ne = M.e.size();
@@ -1717,7 +1720,7 @@ static int launch_amr(nmx_ctx *c, const StageArgs &sa) {
     else if (c->buckets[bi].fv)
       own.push_back({bi, c->anydg ? 1 + (int)own.size() % (nmx_ctx::kLanes - 1) : (int)own.size() % nmx_ctx::kLanes});
   }
-  if (P(c, "nmx_concurrent") != "yes" || c->inturn)
+  if (P(c, "nmx_concurrent") != "yes" || P(c, "nmx_inturn") == "yes")
     for (auto &b : own) b.second = 0;
   unsigned used = 0;
   for (const auto &b : own) used |= 1u << b.second;
@@ -2552,26 +2555,22 @@ extern "C" int nmx_autotune(nmx_ctx *c) {
     // RK4 steps of a DG and an FV bucket of 5 and 9 us: 1.40 ms side by side,
     // 1.11 in turn; 20 of 5 buckets of about 5 us: 4.0 and 3.2, in one launch
     // 1.1; 16 of 7 orders with 19,200 elements: 25.4 side by side).
-    std::string best_shape;
-    bool best_turn = false;
+    const std::string shape0 = P(c, "nmx_batch"), turn0 = P(c, "nmx_inturn");
+    std::vector<std::string> shapes = {"persistent", "buckets"}, turns = {"no", "yes"};
+    if (c->batch_fixed || !c->anydg) shapes = {shape0};
+    if (c->turn_fixed || P(c, "nmx_concurrent") != "yes") turns = {turn0};
+    std::string best_shape = shape0, best_turn = turn0;
     float bt = 1e30f;
-    const bool lanes = P(c, "nmx_concurrent") == "yes";
-    for (const char *shape : {"persistent", "buckets"}) {
-      if (c->batch_fixed || !c->anydg) {
-        if (best_shape.empty()) best_shape = P(c, "nmx_batch");
-        else break;
-      } else {
+    for (const auto &shape : shapes)
+      for (const auto &turn : turns) {
         c->par["nmx_batch"] = shape;
-      }
-      for (int turn = 0; turn < (lanes ? 2 : 1); ++turn) {
-        c->inturn = turn != 0;
+        c->par["nmx_inturn"] = turn;
         float ms = 0;
         if ((r = steps_ms(ms))) return r;
-        if (ms < bt) { bt = ms; best_shape = P(c, "nmx_batch"); best_turn = c->inturn; }
+        if (ms < bt) { bt = ms; best_shape = shape; best_turn = turn; }
       }
-    }
     c->par["nmx_batch"] = best_shape;
-    c->inturn = best_turn;
+    c->par["nmx_inturn"] = best_turn;
   }
   (void)hipEventDestroy(t0);
   (void)hipEventDestroy(t1);
