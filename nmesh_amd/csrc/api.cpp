@@ -516,7 +516,7 @@ extern "C" int nmx_set_param(nmx_ctx *c, const char *name, const char *value) {
     return fail(NMX_EINVAL, "nmx_block must be full, half or quarter");
   const std::string prev = c->par[k];
   c->par[k] = v;
-  if (k == "nmx_block" || k == "nmx_xcd") c->tuned = true;   // explicit choice wins
+  if (k == "nmx_xcd") c->tuned = true;   // explicit choice wins
   if (k == "nmx_batch") c->batch_fixed = true;
   if (k == "nmx_inturn") c->turn_fixed = true;
   drop_stage_graphs(c);
@@ -2473,9 +2473,6 @@ static void stage_times(int method, double t, double dt, double *ts) {
   else { ts[0] = t; ts[1] = ts[2] = ts[3] = 0; }
 }
 
-// Autotuner: time the stage kernel's tile size (nodes per thread) and the
-// XCD-aware element mapping on this mesh with a few RK steps, keep the
-// fastest.  The state and time are restored afterwards.
 extern "C" int nmx_set_trouble_hook(nmx_ctx *c, nmx_trouble_fn fn, void *user) {
   if (!c) return fail(NMX_EINVAL, "ctx is NULL");
   c->trouble_hook = fn;
@@ -2495,6 +2492,9 @@ extern "C" int nmx_get_trouble_scores(nmx_ctx *c, int *score, int nelem, long *r
   return NMX_OK;
 }
 
+// Autotuner: time the XCD-aware element mapping and, on the batched path, the
+// shapes of a stage's launches on this mesh with a few RK steps, keep the
+// fastest.  The state and time are restored afterwards.
 extern "C" int nmx_autotune(nmx_ctx *c) {
   NEED_DEV(c);
   HIPCHK(hipSetDevice(c->device));

@@ -1,5 +1,6 @@
 """The launch choices of a mesh (nmx_batch, nmx_inturn) outlive the switch of an
-element to FV and back in the middle of a run, which rebuilds the device's tables."""
+element to FV and back in the middle of a run, which rebuilds the device's tables;
+nmx_block, which has no effect, leaves the autotuner on."""
 import ctypes as C
 
 import numpy as np
@@ -52,3 +53,12 @@ def test_launch_choice_survives_a_switch(batch, turn):
 def test_inturn_refuses_other_values():
     with pytest.raises(nm.NmxError, match="nmx_inturn"):
         _mesh().set_par("nmx_inturn", "maybe")
+
+
+def test_block_parameter_leaves_the_autotuner_on():
+    print("nmx_block", flush=True)
+    m = _mesh()
+    m.set_par("nmx_block", "full")
+    assert m.par("nmx_batch") == "legacy"       # no launch shape timed yet
+    nm.evolve_myln(m, 1)
+    assert m.par("nmx_batch") in ("persistent", "buckets")
