@@ -57,8 +57,9 @@
 namespace nmx {
 
 constexpr int col_threads(int np) { return (np * np + 63) / 64 * 64; }
-// waves per SIMD that the registers are kept to
-constexpr int col_waves(int np, int wm) { return np == 7 && wm >= 3 && wm <= 4 ? 3 : 2; }
+// waves per SIMD that the registers are kept to (three for 7 points and the early
+// stages measured the same: RK4 steps of 3072 elements 119 us either way)
+constexpr int kColWaves = 2;
 // row stride of an LDS plane: even, so rows of doubles load in pairs, and such
 // that the rows read together by 16 lanes lie in different banks
 constexpr int col_stride(int np) { return np == 7 || np == 8 ? 10 : (np + 1) / 2 * 2; }
@@ -303,7 +304,7 @@ __device__ __forceinline__ int xcd_block(int nblk, int xcd_map) {
 // WM: what the launch does with the RHS, wmode WM (3 to 6), or for WM = 0 any
 // of R, the accumulator and wmodes 1 and 2
 template <int NP, int GEOM, int WM>
-__global__ __launch_bounds__(col_threads(NP), col_waves(NP, WM)) void dg_col_kernel(AmrArgs a) {
+__global__ __launch_bounds__(col_threads(NP), kColWaves) void dg_col_kernel(AmrArgs a) {
   constexpr int NP2 = NP * NP;
   constexpr int NP3 = NP * NP * NP;
   constexpr int S = col_stride(NP);
@@ -598,19 +599,29 @@ __global__ __launch_bounds__(node_threads(NMAX)) void dg_mixed_kernel(AmrArgs a)
   }
 }
 
-// The column kernel from 7 points per direction on and above 1024 elements (4
-// workgroups per CU), the node kernel below.  Steps of a shell, column against
-// node kernel: n = 5, 24,576 elements 405 and 355 us, n = 6 688 and 630, n = 7
-// 964 and 1216, n = 8 1272 and 1403, n = 10 2963 and 3612; 3072 elements n = 8
-// 146 and 151, n = 10 382 and 437; 384 elements n = 7 (with a filter) 55 and
-// 41, n = 8 53 and 35, n = 10 88 and 69.
-constexpr int kNodeElems = 1024;
+// The column kernel from 7 points per direction on and above a number of
+// elements, the node kernel below.  us for RK4 steps, column against node kernel
+// (elements refined, so with the face pass, from 771 to 2052):
+//   shell, n = 5, 24,576 elements 405 and 355, n = 6 688 and 630;
+//   n = 7: box 512 38 and 27, 1023 94 and 81, 1534 114 and 106, 2052 140 and 124,
+//     shell 1504 133 and 123, 3072 119 and 130, 24,576 964 and 1216;
+//   n = 8: box 512 44 and 32, 1023 106 and 97, 1534 128 and 124, 2052 155 and 146,
+//     shell 1504 142 and 131, 3072 142 and 146, 24,576 1272 and 1403;
+//   n = 10: box 512 74 and 67, 771 126 and 148, 1023 149 and 181, 2052 291 and 322,
+//     shell 384 84 and 66, 783 143 and 161, 1084 209 and 205, 1504 255 and 258,
+//     3072 375 and 433, 24,576 2963 and 3612.
+// So for 7 and 8 points the line lies at 2048, and for 9 and 10, whose node
+// workgroups of 12 and 16 waves leave fewer in flight, at 1024: somewhat lower
+// for one order alone, but beside other orders' launches the column kernel
+// gains later (16 steps of 3744 elements of 4 to 10 points 5780, 5860 to 6220
+// with it from 256 elements on).
+constexpr int node_elems(int np) { return np <= 8 ? 2048 : 1024; }
 
 template <int NP, int GEOM, int WM>
 static hipError_t launch_dg_wm(const AmrArgs &a, hipStream_t s) {
   const dim3 grid(a.xcd_map ? 8 * ((a.nlist + 7) / 8) : a.nlist);
   if constexpr (NP >= 7) {
-    if (a.nlist > kNodeElems) {
+    if (a.nlist > node_elems(NP)) {
       hipLaunchKernelGGL((dg_col_kernel<NP, GEOM, WM>), grid, dim3(col_threads(NP)), 0, s, a);
       return hipGetLastError();
     }

@@ -1,5 +1,5 @@
 """The two shapes of the DG stage kernel against each other: one thread per
-column (7 to 10 points per direction, more than 1024 elements in a launch) and
+column (7 to 10 points per direction, thousands of elements in a launch) and
 one per node (per-element launches), and the launch over all orders against
 the per-order ones.
 
