@@ -30,21 +30,19 @@ sys.path.insert(0, ROOT)
 
 HBM_PEAK_GBS = 8000.0
 FP64_PEAK_TFLOPS = 78.6
-# algorithmic bytes per node-update of a fused DG RHS + RK4 stage on
-# curvilinear elements: 8 * (25 state doubles + 9 dXdx)
-BYTES_PER_NU_CURV = 272.0
 # the least an RK4 stage moves per node-update: 13.5 state doubles on average
 # over the 4 stages (dXdx recomputed)
 MIN_BYTES_PER_NU = 108.0
 
 
-def flops_per_nu(n):
-    """FP64 operations of one DG node-update of scalarwave1 at n points per
-    direction: 12 derivatives along the element's reference directions (of
-    pi and of the three c_i) at 2n each, and 36 for their combination with
-    the metric into grad pi and div c and the RHS.  Face terms, the metric's
-    own recomputation and the stage combination are not counted."""
-    return 24.0 * n + 36.0
+def flops_per_nu(n, stored=False):
+    """FP64 operations of one DG node-update of scalarwave1 on a shell at n
+    points per direction: 8 derivatives along the element's reference
+    directions (of pi along each, and of c along the patch's axes, node_rhs in
+    dg_stage.h) at 2n each, and 29 for their combination with the metric into
+    grad pi and div c and the RHS; with a stored metric 12 and 36.  Face terms,
+    the metric's own recomputation and the stage combination are not counted."""
+    return 24.0 * n + 36.0 if stored else 16.0 * n + 29.0
 
 
 def shell_initial_data(x, seed=2026):
@@ -150,7 +148,7 @@ def c4_headline(nm, steps, warmup, have_torch):
     m = c4_mesh(nm, "batched")
     x = m.coords()
     m.upload(shell_initial_data(x))
-    nm.evolve_myln(m, 1)                   # autotune (launch shape, tiles) and graph capture
+    nm.evolve_myln(m, 1)                   # autotune (launch shape) and graph capture
     if warmup:
         nm.evolve_myln(m, warmup)
     m.synchronize()
@@ -172,8 +170,7 @@ def c4_headline(nm, steps, warmup, have_torch):
     buckets = {int(k): int((info[:, 2] == k).sum()) for k in np.unique(info[:, 2])}
     res = {"m": m, "wall": wall, "dev_s": dev_s, "nodes": nn, "elements": m.nelem,
            "stage_us": stage_s * 1e6, "flops_per_stage": flops_stage,
-           "achieved": BYTES_PER_NU_CURV * nn / stage_s / 1e9,
-           "achieved_min": MIN_BYTES_PER_NU * nn / stage_s / 1e9,
+           "achieved": MIN_BYTES_PER_NU * nn / stage_s / 1e9,
            "tflops": flops_stage / stage_s / 1e12, "buckets": buckets,
            "shape": m.par("nmx_batch"), "dt": m.dt}
     return res
@@ -220,7 +217,7 @@ def batched_leg(nm, steps, plain_steps):
         m.synchronize()
         shapes = [m.par("nmx_batch")] if path == "batched" else [None]
         if path == "batched":
-            shapes += [q for q in ("persistent", "buckets", "legacy") if q != shapes[0]]
+            shapes += [q for q in ("persistent", "buckets") if q != shapes[0]]
         for shape in shapes:
             if shape is not None and shape != m.par("nmx_batch"):
                 m.set_par("nmx_batch", shape)
@@ -234,8 +231,7 @@ def batched_leg(nm, steps, plain_steps):
             dev_s = m.last_evolve_ms() * 1e-3
             res = {"value": rate, "steps": nsteps, "ms_per_step": 1e3 * wall / nsteps,
                    "device_ms_per_step": 1e3 * dev_s / nsteps,
-                   "achieved_GBps": BYTES_PER_NU_CURV * 4 * nsteps * m.nnodes / dev_s / 1e9,
-                   "achieved_min_GBps": MIN_BYTES_PER_NU * 4 * nsteps * m.nnodes / dev_s / 1e9}
+                   "achieved_GBps": MIN_BYTES_PER_NU * 4 * nsteps * m.nnodes / dev_s / 1e9}
             if shape is not None:
                 res["launch_shape"] = shape
                 out.setdefault("shapes", {})[shape] = res["ms_per_step"]
@@ -247,7 +243,6 @@ def batched_leg(nm, steps, plain_steps):
     if "perelement" in out:
         out["speedup_batched_vs_perelement"] = out["batched"]["value"] / out["perelement"]["value"]
     out["roofline_frac_batched"] = out["batched"]["achieved_GBps"] / HBM_PEAK_GBS
-    out["roofline_frac_min_batched"] = out["batched"]["achieved_min_GBps"] / HBM_PEAK_GBS
     out["workload"] = ("scalarwave1 DG, cubed-sphere shell r in [2,20], levels 3-5 (19,200 elements), "
                        "N uniform in {3..9} (%d nodes), upwind, outgoing, RK4" % out["nodes"])
     return out
@@ -692,7 +687,7 @@ def main():
     ap.add_argument("--geometry", default="analytic", help="dXdx recomputed (analytic) or streamed (stored)")
     ap.add_argument("--xcd", default="auto", help="contiguous element ranges per XCD (yes|no|auto)")
     ap.add_argument("--block", default="auto",
-                    help="nodes per thread: full (1), half (2), quarter (4) or auto (autotuned)")
+                    help="accepted without effect (the stage kernels have no tile size)")
     ap.add_argument("--copy-calib", type=int, default=0, metavar="MIB",
                     help="instead of the workload, run 10 device copies of MIB MiB with "
                          "torch (counter calibration for rocprofv3 --pmc) and exit")
@@ -763,7 +758,7 @@ def main():
     mh = h.pop("m")
     shapes = {h["shape"]: 1e3 * h["wall"] / args.steps}
     if args.shape_steps:
-        for shape in ("persistent", "buckets", "legacy"):
+        for shape in ("persistent", "buckets"):
             if shape in shapes:
                 continue
             mh.set_par("nmx_batch", shape)
@@ -805,10 +800,8 @@ def main():
                      "kernel": "one RK4 stage of the batched path (%s launch shape: every order "
                                "bucket's launches of the stage)" % h["shape"],
                      "avg_launch_us": h["stage_us"],
-                     "bytes_per_node_update": BYTES_PER_NU_CURV,
-                     "min_bytes_per_node_update": MIN_BYTES_PER_NU,
-                     "achieved_min": h["achieved_min"], "frac_min": h["achieved_min"] / HBM_PEAK_GBS,
-                     "fp64": {"flops_per_node_update": "24 n + 36", "flops_per_stage": h["flops_per_stage"],
+                     "bytes_per_node_update": MIN_BYTES_PER_NU,
+                     "fp64": {"flops_per_node_update": "16 n + 29", "flops_per_stage": h["flops_per_stage"],
                               "achieved_TFLOPs": h["tflops"], "peak_TFLOPs": FP64_PEAK_TFLOPS,
                               "frac": h["tflops"] / FP64_PEAK_TFLOPS}},
         "batched_shapes_ms_per_step": shapes,
@@ -864,14 +857,12 @@ def plain_leg(nm, args, have_torch):
     m.set_par("nmx_geometry", args.geometry)
     if args.xcd != "auto":
         m.set_par("nmx_xcd", args.xcd)
-    if args.block != "auto":
-        m.set_par("nmx_block", args.block)
     nm.amr_setup_mesh(m)
     x = m.coords()
     m.upload(shell_initial_data(x))
     nn = m.nnodes
-    if args.block == "auto" and args.xcd == "auto":
-        nm.autotune(m)            # times tile size / XCD mapping on this mesh
+    if args.xcd == "auto":
+        nm.autotune(m)            # times the XCD mapping on this mesh
     if args.plain_warmup:
         nm.evolve_myln(m, args.plain_warmup)
     m.synchronize()
@@ -886,17 +877,14 @@ def plain_leg(nm, args, have_torch):
     dev_ms = m.last_evolve_ms()    # HIP events on the library's stream around the steps
     launches = 4 * args.plain_steps
     avg_launch_s = dev_ms * 1e-3 / launches
-    # algorithmic bytes per node-update of a fused RHS + RK4 stage: read w,
-    # u, u_p and write u, w (25 doubles) plus 9 doubles of dXdx per node on
-    # curvilinear elements, face-neighbour re-reads counted 0: 272 B
-    achieved = BYTES_PER_NU_CURV * nn / avg_launch_s / 1e9
     # the least this kernel must move: pi and c of its input, of u after the
     # first stage and of its output (8, 12, 12 doubles), and in stage 4 what
     # ends the step (22); dXdx recomputed (0) or streamed (9)
     g = 9.0 if args.geometry == "stored" else 0.0
-    min_bytes_per_nu = 8.0 * ((8 + 12 + 12 + 22) / 4.0 + g)
-    achieved_min = min_bytes_per_nu * nn / avg_launch_s / 1e9
-    tflops = flops_per_nu(args.plain_n) * nn / avg_launch_s / 1e12
+    bytes_per_nu = MIN_BYTES_PER_NU + 8.0 * g
+    achieved = bytes_per_nu * nn / avg_launch_s / 1e9
+    flops = flops_per_nu(args.plain_n, args.geometry == "stored")
+    tflops = flops * nn / avg_launch_s / 1e12
     traffic = load_traffic("traffic_dg_stage_shell_n8.json") if args.plain_n == 8 else None
     out = {"workload": "scalarwave1 DG, cubed-sphere shell r in [2,20], 6x8^3 elements, "
                        "n=%d (%d nodes), upwind, outgoing, RK4, fused RHS+stage" % (args.plain_n, nn),
@@ -911,10 +899,8 @@ def plain_leg(nm, args, have_torch):
                         "kernel": "dg_col_kernel or dg_node_kernel, n=%d, %s geometry" % (args.plain_n, args.geometry),
                         "xcd_map": m.par("nmx_xcd"),
                         "avg_launch_us": avg_launch_s * 1e6,
-                        "bytes_per_node_update": BYTES_PER_NU_CURV,
-                        "min_bytes_per_node_update": min_bytes_per_nu,
-                        "achieved_min": achieved_min, "frac_min": achieved_min / HBM_PEAK_GBS,
-                        "fp64": {"flops_per_node_update": flops_per_nu(args.plain_n),
+                        "bytes_per_node_update": bytes_per_nu,
+                        "fp64": {"flops_per_node_update": flops,
                                  "achieved_TFLOPs": tflops, "frac": tflops / FP64_PEAK_TFLOPS}}}
     del m
     return out
