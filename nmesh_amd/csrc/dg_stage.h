@@ -227,8 +227,10 @@ __device__ __forceinline__ void node_lift(const NodeGeo &m, int dir, double sig,
 struct AccIn {
   double U[5], A[5], phi;
 };
+// ... and a right-hand side alone: nothing
+struct RhsIn {};
 template <int WM>
-using NodeIn = std::conditional_t<WM == 0, AccIn, StageIn>;
+using NodeIn = std::conditional_t<WM == 0, AccIn, std::conditional_t<WM == 1, RhsIn, StageIn>>;
 
 // the operands of node_out at the node whose first state double is gi,
 // requested together: between node_out's stores, which they may alias, they were
@@ -247,12 +249,19 @@ __device__ __forceinline__ void node_in(const AmrArgs &a, const StageRegs &, lon
   }
   if (a.wmode == 2 || (a.Aout && !a.Ain)) q.phi = a.win[gi + po];
 }
+__device__ __forceinline__ void node_in(const AmrArgs &, const StageRegs &, long, const int (&)[4], int, RhsIn &) {}
 __device__ __forceinline__ void node_in(const AmrArgs &, const StageRegs &o, long gi, const int (&vo)[4], int po,
                                         StageIn &q) {
   stage_in(o, gi, vo, po, q);
 }
 
 // the stage's output there
+__device__ __forceinline__ void node_out(const AmrArgs &a, const StageRegs &, const RhsIn &, long gi,
+                                         const int (&vo)[4], int po, const double u[4], const double r[4]) {
+#pragma unroll
+  for (int v = 0; v < 4; ++v) a.R[gi + vo[v]] = r[v];
+  a.R[gi + po] = u[0];
+}
 __device__ __forceinline__ void node_out(const AmrArgs &a, const StageRegs &, const AccIn &q, long gi,
                                          const int (&vo)[4], int po, const double u[4], const double r[4]) {
 #pragma unroll
@@ -301,8 +310,14 @@ __device__ __forceinline__ int xcd_block(int nblk, int xcd_map) {
   return q < chunk ? (blockIdx.x & 7) * chunk + q : nblk;
 }
 
-// WM: what the launch does with the RHS, wmode WM (3 to 6), or for WM = 0 any
-// of R, the accumulator and wmodes 1 and 2
+// WM: what the launch does with the RHS, wmode WM (3 to 6), 1 R alone, or for WM
+// = 0 any of R, the accumulator and wmodes 1 and 2.  R alone holds no operands and
+// so 20 to 40 registers less: right-hand sides of 4096 box elements take, with the
+// kernel for all of them and alone, 33 and 28 us (7 points), 81 and 60 (9) and
+// 107 and 92 (10), of 3072 shell elements 38 and 34 (8) and 85 and 75 (10).
+inline int stage_kind(const AmrArgs &a) {
+  return a.wmode >= 3 ? a.wmode : a.R && !a.Aout && !a.wmode ? 1 : 0;
+}
 template <int NP, int GEOM, int WM>
 __global__ __launch_bounds__(col_threads(NP), kColWaves) void dg_col_kernel(AmrArgs a) {
   constexpr int NP2 = NP * NP;
@@ -554,8 +569,14 @@ __device__ __forceinline__ void node_elem(const AmrArgs &a, const NMX_CONST Slot
   node_out(a, o, in, gbase + node, vo, 4 * NP3, u, r);
 }
 
+// waves per SIMD that the registers are kept to: with an accumulator and a stored
+// metric 8 points take 130 without a bound, two too many for two workgroups per CU
+// (Euler steps of 888 elements 31.1 us, 28.5 with it; the other modes, which
+// would spill more, measured no faster)
+constexpr int node_waves(int np, int geom, int wm) { return np == 8 && geom == 1 && wm == 0 ? 4 : 1; }
+
 template <int NP, int GEOM, int WM>
-__global__ __launch_bounds__(node_threads(NP)) void dg_node_kernel(AmrArgs a) {
+__global__ __launch_bounds__(node_threads(NP), node_waves(NP, GEOM, WM)) void dg_node_kernel(AmrArgs a) {
   __shared__ double s_u[node_fields(GEOM) * NP * NP * NP];
   __shared__ double s_f[6 * 4 * NP * NP];
   __shared__ double s_D[NP * NP];
@@ -632,7 +653,8 @@ static hipError_t launch_dg_wm(const AmrArgs &a, hipStream_t s) {
 
 template <int NP, int GEOM>
 static hipError_t launch_dg_np(const AmrArgs &a, hipStream_t s) {
-  switch (a.wmode) {
+  switch (stage_kind(a)) {
+    case 1: return launch_dg_wm<NP, GEOM, 1>(a, s);
     case 3: return launch_dg_wm<NP, GEOM, 3>(a, s);
     case 4: return launch_dg_wm<NP, GEOM, 4>(a, s);
     case 5: return launch_dg_wm<NP, GEOM, 5>(a, s);
@@ -655,7 +677,8 @@ static hipError_t launch_dg_geom(int np, int nmax, const AmrArgs &a, hipStream_t
   if (a.nlist <= 0) return hipSuccess;
   if (np == 0) {
     if (nmax < 2 || nmax > 10) return hipErrorInvalidValue;
-    switch (a.wmode) {
+    switch (stage_kind(a)) {
+      case 1: return launch_mixed_wm<GEOM, 1>(nmax, a, s);
       case 3: return launch_mixed_wm<GEOM, 3>(nmax, a, s);
       case 4: return launch_mixed_wm<GEOM, 4>(nmax, a, s);
       case 5: return launch_mixed_wm<GEOM, 5>(nmax, a, s);
