@@ -2511,26 +2511,35 @@ extern "C" int nmx_autotune(nmx_ctx *c) {
   hipEvent_t t0, t1;
   HIPCHK(hipEventCreate(&t0));
   HIPCHK(hipEventCreate(&t1));
-  // 4 steps after one to warm up
-  auto steps_ms = [&](float &ms) -> int {
-    if (int rr = issue_step(c, method, c->dt, 0, false)) return rr;
-    HIPCHK(hipEventRecord(t0, c->stream));
-    for (int s = 0; s < 4; ++s)
-      if (int rr = issue_step(c, method, c->dt, 0, (s & 1) != 0)) return rr;
-    HIPCHK(hipEventRecord(t1, c->stream));
-    HIPCHK(hipEventSynchronize(t1));
-    HIPCHK(hipEventElapsedTime(&ms, t0, t1));
+  // The fastest of n candidates, set(k) choosing one, by a few steps each: all in
+  // turn, after a step to warm up, then those within a quarter of the best once
+  // more, for a first call slows the first of them.  Times are multiplied by
+  // weight(k).
+  const int nsteps = c->mesh.nnodes > 2000000 ? 2 : 4;
+  auto fastest = [&](int n, auto &&set, auto &&weight) -> int {
+    std::vector<float> ms(n, 1e30f);
+    int best = 0;
+    for (int rep = 0; rep < 2 && n > 1; ++rep) {
+      const float limit = 1.25f * ms[best];
+      for (int k = 0; k < n; ++k) {
+        if (ms[k] > limit) continue;
+        set(k);
+        if (rep == 0)
+          if (int rr = issue_step(c, method, c->dt, 0, false)) return rr;
+        HIPCHK(hipEventRecord(t0, c->stream));
+        for (int s = 0; s < nsteps; ++s)
+          if (int rr = issue_step(c, method, c->dt, 0, (s & 1) != 0)) return rr;
+        HIPCHK(hipEventRecord(t1, c->stream));
+        HIPCHK(hipEventSynchronize(t1));
+        float t = 0;
+        HIPCHK(hipEventElapsedTime(&t, t0, t1));
+        ms[k] = std::min(ms[k], t * weight(k));
+      }
+      best = (int)(std::min_element(ms.begin(), ms.end()) - ms.begin());
+    }
+    set(best);
     return NMX_OK;
   };
-  std::string best_x = P(c, "nmx_xcd");
-  float best = 1e30f;
-  for (const char *x : {"yes", "no"}) {
-    c->par["nmx_xcd"] = x;
-    float ms = 0;
-    if ((r = steps_ms(ms))) return r;
-    if (ms < best) { best = ms; best_x = x; }
-  }
-  c->par["nmx_xcd"] = best_x;
   if (c->amr) {
     // the buckets' stages timed alone, on an RK4 second-stage launch (reads w
     // and u, writes the next w), order them for the lanes
@@ -2559,19 +2568,25 @@ extern "C" int nmx_autotune(nmx_ctx *c) {
     std::vector<std::string> shapes = {"persistent", "buckets"}, turns = {"no", "yes"};
     if (c->batch_fixed || !c->anydg) shapes = {shape0};
     if (c->turn_fixed || P(c, "nmx_concurrent") != "yes") turns = {turn0};
-    std::string best_shape = shape0, best_turn = turn0;
-    float bt = 1e30f;
-    for (const auto &shape : shapes)
-      for (const auto &turn : turns) {
-        c->par["nmx_batch"] = shape;
-        c->par["nmx_inturn"] = turn;
-        float ms = 0;
-        if ((r = steps_ms(ms))) return r;
-        if (ms < bt) { bt = ms; best_shape = shape; best_turn = turn; }
-      }
-    c->par["nmx_batch"] = best_shape;
-    c->par["nmx_inturn"] = best_turn;
+    const int nt = (int)turns.size();
+    auto set = [&](int k) { c->par["nmx_batch"] = shapes[k / nt]; c->par["nmx_inturn"] = turns[k % nt]; };
+    // Launched eagerly, forks and several launches cost more than in the steps'
+    // graphs: launches in turn have to be a fifth faster and one for all orders 3%
+    // (from graphs, side by side and in turn, us a step: 19,200 elements of 4 to 10
+    // points 1566 and 1761, 3744 of 4 to 8, DG and FV, 360 and 530, which eager
+    // steps take for equal now and then; 384 DG and FV elements of 6 points 82 and
+    // 64; 1056 elements of 9 and 10 points 200, in one launch 213).
+    auto weight = [&](int k) {
+      return (shapes[k / nt] == "persistent" ? 1.03f : 1.f) * (turns[k % nt] == "yes" ? 1.2f : 1.f);
+    };
+    if ((r = fastest((int)shapes.size() * nt, set, weight)))
+      return r;
   }
+  // the XCDs' ranges with the shape that the steps will have (under the lanes'
+  // eager forks 3744 elements of 3 to 5 points seem faster without them: 165 us a
+  // step from graphs, 147 with them), and unless 3% are gained they stay
+  if ((r = fastest(2, [c](int k) { c->par["nmx_xcd"] = k ? "no" : "yes"; }, [](int k) { return k ? 1.03f : 1.f; })))
+    return r;
   (void)hipEventDestroy(t0);
   (void)hipEventDestroy(t1);
   HIPCHK(hipMemcpyAsync(c->dU, backup, c->nstate * 8, hipMemcpyDeviceToDevice, c->stream));
