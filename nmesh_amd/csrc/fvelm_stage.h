@@ -440,11 +440,7 @@ __global__ __launch_bounds__(3 * fve_line_threads(NP), 2) void fvelm_kernel(AmrA
   // requested a node ahead
   const StageRegs o = {a.win, a.U, a.Wa, a.Wb, a.cA, a.cW, a.wmode};
   StageIn in;
-  AccIn acc_in;
-  if (tid < NP3) {
-    if (a.wmode >= 3) node_in(a, o, gbase + tid, vo, 4 * NP3, in);
-    else node_in(a, o, gbase + tid, vo, 4 * NP3, acc_in);
-  }
+  if (a.wmode >= 3 && tid < NP3) node_in(a, o, gbase + tid, vo, 4 * NP3, in);
   __syncthreads();
 #pragma unroll 1
   for (int node = tid; node < NP3; node += NT) {
@@ -469,8 +465,8 @@ __global__ __launch_bounds__(3 * fve_line_threads(NP), 2) void fvelm_kernel(AmrA
       if (node + NT < NP3) node_in(a, o, gi + NT, vo, 4 * NP3, in);
       node_out(a, o, q, gi, vo, 4 * NP3, u, r);
     } else {
-      const AccIn q = acc_in;
-      if (node + NT < NP3) node_in(a, o, gi + NT, vo, 4 * NP3, acc_in);
+      AccIn q;
+      node_in(a, o, gi, vo, 4 * NP3, q);
       node_out(a, o, q, gi, vo, 4 * NP3, u, r);
     }
   }
