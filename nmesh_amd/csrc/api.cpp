@@ -1005,7 +1005,7 @@ static int upload_mesh(nmx_ctx *c) {
         fr[i].foff[f] = 5 * np3 * d.x + d.y;
         fr[i].fs1[f] = d.z;
         fr[i].fs2[f] = d.w;
-        fg[6 * i + f] = adj_scale_ratio(M, M.e[i], f, M.e[d.x], M.e[i].nbf[f][0]);
+        if (!c->fvelm) fg[6 * i + f] = adj_scale_ratio(M, M.e[i], f, M.e[d.x], M.e[i].nbf[f][0]);
       }
     }
     if ((r = dev_upload(&c->dfrec, fr)) || (!c->fvelm && (r = dev_upload(&c->dadjfg, fg)))) return r;
@@ -2511,11 +2511,10 @@ extern "C" int nmx_autotune(nmx_ctx *c) {
   hipEvent_t t0, t1;
   HIPCHK(hipEventCreate(&t0));
   HIPCHK(hipEventCreate(&t1));
-  // The fastest of n candidates, set(k) choosing one, by a few steps each: all in
+  // The fastest of n candidates, set(k) choosing one, by 2 steps each: all in
   // turn, after a step to warm up, then those within a quarter of the best once
   // more, for a first call slows the first of them.  Times are multiplied by
   // weight(k).
-  const int nsteps = c->mesh.nnodes > 2000000 ? 2 : 4;
   auto fastest = [&](int n, auto &&set, auto &&weight) -> int {
     std::vector<float> ms(n, 1e30f);
     int best = 0;
@@ -2527,8 +2526,8 @@ extern "C" int nmx_autotune(nmx_ctx *c) {
         if (rep == 0)
           if (int rr = issue_step(c, method, c->dt, 0, false)) return rr;
         HIPCHK(hipEventRecord(t0, c->stream));
-        for (int s = 0; s < nsteps; ++s)
-          if (int rr = issue_step(c, method, c->dt, 0, (s & 1) != 0)) return rr;
+        for (int s = 0; s < 2; ++s)
+          if (int rr = issue_step(c, method, c->dt, 0, s != 0)) return rr;
         HIPCHK(hipEventRecord(t1, c->stream));
         HIPCHK(hipEventSynchronize(t1));
         float t = 0;
