@@ -437,16 +437,14 @@ __global__ __launch_bounds__(3 * fve_line_threads(NP), 2) void fvelm_kernel(AmrA
   __syncthreads();
   if (tid % NL < NP2) fve_sweep<NP, REC, GEOM, EX, LLF>(a, R, wc, ex, d, la, lb, lo, hi, s_u, acc);
   // r_{pi,c} = -divf, r_phi = pi, the RK stage; the next node's registers
-  // requested a node ahead
+  // requested a node ahead, but for the operands of stages with an accumulator,
+  // whose loop of its own leaves the other's registers as they are
   const StageRegs o = {a.win, a.U, a.Wa, a.Wb, a.cA, a.cW, a.wmode};
   StageIn in;
   if (a.wmode >= 3 && tid < NP3) node_in(a, o, gbase + tid, vo, 4 * NP3, in);
   __syncthreads();
-#pragma unroll 1
-  for (int node = tid; node < NP3; node += NT) {
+  auto rhs_at = [&](int node, double u[4], double r[4]) {
     const int p = fve_at<NP>(node % NP, (node / NP) % NP, node / NP2);
-    const long gi = gbase + node;
-    double u[4], r[4];
 #pragma unroll
     for (int v = 0; v < 4; ++v) u[v] = s_u[v][p];
 #pragma unroll
@@ -460,15 +458,25 @@ __global__ __launch_bounds__(3 * fve_line_threads(NP), 2) void fvelm_kernel(AmrA
       }
       r[v] = -div;
     }
-    if (a.wmode >= 3) {
-      const StageIn q = in;
-      if (node + NT < NP3) node_in(a, o, gi + NT, vo, 4 * NP3, in);
-      node_out(a, o, q, gi, vo, 4 * NP3, u, r);
-    } else {
+  };
+  if (a.wmode < 3) {
+#pragma unroll 1
+    for (int node = tid; node < NP3; node += NT) {
       AccIn q;
-      node_in(a, o, gi, vo, 4 * NP3, q);
-      node_out(a, o, q, gi, vo, 4 * NP3, u, r);
+      double u[4], r[4];
+      node_in(a, o, gbase + node, vo, 4 * NP3, q);
+      rhs_at(node, u, r);
+      node_out(a, o, q, gbase + node, vo, 4 * NP3, u, r);
     }
+    return;
+  }
+#pragma unroll 1
+  for (int node = tid; node < NP3; node += NT) {
+    double u[4], r[4];
+    rhs_at(node, u, r);
+    const StageIn q = in;
+    if (node + NT < NP3) node_in(a, o, gbase + node + NT, vo, 4 * NP3, in);
+    node_out(a, o, q, gbase + node, vo, 4 * NP3, u, r);
   }
 }
 
