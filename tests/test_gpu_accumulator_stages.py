@@ -46,3 +46,23 @@ def test_euler_step_is_u_plus_dt_r(luni, n):
     nm.evolve_Euler_mesh(m)
     e = u + m.dt * r.ravel()
     assert np.abs(m.download().ravel() - e).max() <= 4 * np.finfo(float).eps * np.abs(e).max()
+
+
+@pytest.mark.parametrize("hi", [4, 8, 10])
+@pytest.mark.parametrize("geometry", ["analytic", "stored"])
+def test_rhs_alone_in_one_launch_per_order_and_with_an_accumulator(hi, geometry):
+    """the right-hand side alone, in one launch over all orders and per order, bit
+    for bit; and the one that an Euler step adds, up to the step's rounding"""
+    print("rhs alone", hi, geometry, flush=True)
+    out = []
+    for batch in ("persistent", "buckets"):
+        m = _mesh(1, 4, nmx_path="batched", nmx_batch=batch, nmx_geometry=geometry, evolve_method="Euler",
+                  amr_hrefine_sphere_radius=7, amr_hrefine_sphere_levels=1)
+        m.set_elm_n(np.random.default_rng(5).integers(2, hi + 1, m.nelem).astype(np.int32))
+        u = np.random.default_rng(6).standard_normal(5 * m.nnodes)
+        m.upload(u)
+        out.append(nm.evolve_setrhs_mesh(m, t=0.0).ravel().copy())
+        nm.evolve_Euler_mesh(m)
+        e = u + m.dt * out[-1]
+        assert np.abs(m.download().ravel() - e).max() <= 4 * np.finfo(float).eps * np.abs(e).max()
+    assert np.array_equal(*out)

@@ -1,5 +1,5 @@
 """GPU parity of scalarwave1 on FV elements (fv_divf with the reference's
-default FV parameters; libnmx fvelm_stage_kernel) against the oracle.
+default FV parameters; libnmx fvelm_kernel) against the oracle.
 
 The kernel and the oracle evaluate the same reconstructions and metric
 factors; the numerical flux is the closed form on the device and the
